@@ -12,49 +12,106 @@
 // takes e^{i k im a}, its mirror np + 1 - j the conjugate (for even np
 // index np/2 is left at 0, as in the reference).
 //
-// Sums are deterministic: every wavefront reduces each coefficient with
-// shuffles and its lane 0 adds the result to the wave's own LDS row in
-// particle order; the rows are added in wave order into one partial per
-// block, and a second kernel adds the block partials in block order.
+// The sums take 8 FP64 operations per coefficient pair and particle and read
+// 9 bytes (FP32) per particle: FP64 issue bounds them.  A wavefront owns one
+// harmonic and a run of pitches for the whole pass, so its sums stay in
+// registers (four products per pitch and its mirror) and are reduced over
+// the lanes once at the end; the particles' e^{i nsect theta} and e^{i a}
+// are formed once per block, a tile at a time, and handed to the wavefronts
+// through LDS.  25 pitches x 6 harmonics of 1e7 particles: 0.64 ms against
+// 6.36 ms with each coefficient reduced over the wavefront per particle.
+//
+// Sums are deterministic: the order depends only on n, np and nm.
 #include "galhip_ctx.h"
 
 #include <algorithm>
 
 namespace gh {
 
-constexpr int LG_BLOCK = 256;
-constexpr int LG_WAVES = LG_BLOCK / 64;
-constexpr int LG_MAXQ = 512;    // np * nm coefficients at most (LDS: 4 x 2 x 512 doubles)
+constexpr int LG_MAXQ = 512;     // np * nm coefficients at most
+constexpr int LG_MAXW = 8;       // wavefronts per block at most
+constexpr int LG_SUM_BLOCK = 256;
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// How the coefficients are dealt out: a unit is harmonic im with len pitch
+// offsets (unit u: im = u / nch + 1, offsets (u % nch) len + 1 ..); a block
+// has one wavefront per unit of its group.
+struct LgPlan {
+    int kmax;      // largest pitch offset
+    int nch, len;  // runs per harmonic and their length
+    int units;     // nm * nch
+    int groups;    // gridDim.y
+    int waves;     // wavefronts per block
+    int nb;        // gridDim.x
+};
+
+// Runs of at most 12 offsets: 48 FP64 sums (96 VGPRs) per lane, three
+// wavefronts per SIMD.
+static LgPlan lg_plan(long long n, int np, int nm) {
+    LgPlan p;
+    p.kmax = np - (np / 2 + 1);
+    p.nch = p.kmax > 12 ? (p.kmax + 11) / 12 : 1;
+    p.len = (p.kmax + p.nch - 1) / p.nch;
+    p.units = nm * p.nch;
+    p.groups = (p.units + LG_MAXW - 1) / LG_MAXW;
+    p.waves = (p.units + p.groups - 1) / p.groups;
+    // twelve wavefronts per CU (three per SIMD) over 256 CUs
+    const long long tiles = (n + 64 * p.waves - 1) / (64 * p.waves);
+    const long long most = std::max(1, 256 * 12 / (p.waves * p.groups));
+    p.nb = (int)std::max<long long>(1, std::min(tiles, most));
+    return p;
 }
 
-template <typename R>
-__global__ __launch_bounds__(LG_BLOCK) void lgsp_part_kernel(
+// z^e for e >= 1 by squaring
+__device__ __forceinline__ void cpow(double zr, double zi, int e, double &pr, double &pi) {
+    while (!(e & 1)) {
+        const double t = fma(zr, zr, -(zi * zi));
+        zi = 2.0 * (zr * zi);
+        zr = t;
+        e >>= 1;
+    }
+    pr = zr;
+    pi = zi;
+    while (e >>= 1) {
+        double t = fma(zr, zr, -(zi * zi));
+        zi = 2.0 * (zr * zi);
+        zr = t;
+        if (e & 1) {
+            t = fma(pr, zr, -(pi * zi));
+            pi = fma(pi, zr, pr * zi);
+            pr = t;
+        }
+    }
+}
+
+// part[q][block]: q = [cos parts][sin parts][count].  KC: pitch offsets of
+// a run at most.
+template <typename R, int KC>
+__global__ __launch_bounds__(64 * LG_MAXW, 3) void lgsp_part_kernel(
     const typename Vec4<R>::T *__restrict__ xv, int ps, const uint8_t *__restrict__ zone,
-    long long n, int nz, int offanal, int nsect, int np, int nm, double inv_lscale,
+    long long n, int nz, int offanal, int nsect, int np, int nm, double inv_lscale, LgPlan pl,
     double *__restrict__ part) {
-    __shared__ double acc[LG_WAVES][2 * LG_MAXQ];
-    __shared__ double cnt_w[LG_WAVES];
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int nq = np * nm;
-    for (int i = tid; i < LG_WAVES * 2 * LG_MAXQ; i += LG_BLOCK) (&acc[0][0])[i] = 0.0;
-    if (tid < LG_WAVES) cnt_w[tid] = 0.0;
-    __syncthreads();
-    const int jc = np / 2 + 1;           // 1-based centre (k = 0)
-    const int kmax = np - jc;
-    const long long stride = (long long)gridDim.x * LG_BLOCK;
-    double cnt = 0.0;
-    for (long long base = (long long)blockIdx.x * LG_BLOCK; base < n; base += stride) {
+    __shared__ double2 s_z[64 * LG_MAXW], s_w[64 * LG_MAXW];
+    __shared__ double s_cnt[LG_MAXW];
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, T = blockDim.x;
+    const int nq = np * nm, jc = np / 2 + 1;   // 1-based centre (offset 0)
+    const int unit = blockIdx.y * pl.waves + w;
+    const bool work = unit < pl.units;         // uniform over the wavefront
+    const int im = work ? unit / pl.nch + 1 : 1;
+    const int k0 = work ? (unit - (im - 1) * pl.nch) * pl.len + 1 : 1;
+    // gr zr, gi zi, gi zr, gr zi summed for offsets k0 ..; z itself
+    double p1[KC], p2[KC], p3[KC], p4[KC], zsr = 0.0, zsi = 0.0, cnt = 0.0;
+#pragma unroll
+    for (int k = 0; k < KC; k++) p1[k] = p2[k] = p3[k] = p4[k] = 0.0;
+    const long long stride = (long long)gridDim.x * T;
+    for (long long base = (long long)blockIdx.x * T; base < n; base += stride) {
         const long long i = base + tid;
         double c1 = 0.0, s1 = 0.0, ca = 1.0, sa = 0.0;
         if (i < n) {
             const int z = zone[i];
             const bool inc = z >= 1 && (z <= nz || (offanal && z == nz + 1));
-            const typename Vec4<R>::T p = xv[i * ps];   // x, y lead the particle's data
+            // x, y lead the particle's data
+            const typename Vec2<R>::T p =
+                *reinterpret_cast<const typename Vec2<R>::T *>(xv + i * ps);
             const double x = (double)p.x, y = (double)p.y;
             const double rc = sqrt(x * x + y * y);
             if (inc && rc > 0.0) {
@@ -66,103 +123,130 @@ __global__ __launch_bounds__(LG_BLOCK) void lgsp_part_kernel(
                     s1 = s1 * cx + c1 * sy;
                     c1 = t;
                 }
-                const double a = 0.25 * (double)nsect * log(rc * inv_lscale);
-                sincos(a, &sa, &ca);
+                sincos(0.25 * (double)nsect * log(rc * inv_lscale), &sa, &ca);
                 cnt += 1.0;
             }
         }
-        // powers: z^im (harmonic), w^im (pitch step of this harmonic)
-        double zr = 1.0, zi = 0.0, wr = 1.0, wi = 0.0;
-        for (int im = 1; im <= nm; im++) {
-            double t = zr * c1 - zi * s1;
-            zi = zi * c1 + zr * s1;
-            zr = t;
-            t = wr * ca - wi * sa;
-            wi = wi * ca + wr * sa;
-            wr = t;
-            const int q0 = (jc - 1) * nm + im - 1;
-            double vr = wave_sum(zr), vi = wave_sum(zi);
-            if (lane == 0) {
-                acc[w][2 * q0] += vr;
-                acc[w][2 * q0 + 1] += vi;
-            }
-            double gr = 1.0, gi = 0.0;
-            for (int k = 1; k <= kmax; k++) {
-                t = gr * wr - gi * wi;
-                gi = gi * wr + gr * wi;
-                gr = t;
-                // pitch jc + k: g z; its mirror np + 1 - (jc + k): conj(g) z
-                const int qp = (jc + k - 1) * nm + im - 1;
-                const int qm = (np - jc - k) * nm + im - 1;
-                const double pr = wave_sum(gr * zr - gi * zi);
-                const double pi = wave_sum(gi * zr + gr * zi);
-                const double mr = wave_sum(gr * zr + gi * zi);
-                const double mi = wave_sum(gr * zi - gi * zr);
-                if (lane == 0) {
-                    acc[w][2 * qp] += pr;
-                    acc[w][2 * qp + 1] += pi;
-                    acc[w][2 * qm] += mr;
-                    acc[w][2 * qm + 1] += mi;
+        __syncthreads();   // the last tile has been read
+        s_z[tid] = make_double2(c1, s1);
+        s_w[tid] = make_double2(ca, sa);
+        __syncthreads();
+        if (work)
+            for (int e = lane; e < T; e += 64) {
+                double zr, zi, wr, wi, gr = 1.0, gi = 0.0;
+                cpow(s_z[e].x, s_z[e].y, im, zr, zi);
+                cpow(s_w[e].x, s_w[e].y, im, wr, wi);
+                if (k0 > 1) cpow(wr, wi, k0 - 1, gr, gi);
+                zsr += zr;
+                zsi += zi;
+#pragma unroll
+                for (int k = 0; k < KC; k++) {
+                    const double t = fma(gr, wr, -(gi * wi));
+                    gi = fma(gi, wr, gr * wi);
+                    gr = t;
+                    p1[k] = fma(gr, zr, p1[k]);
+                    p2[k] = fma(gi, zi, p2[k]);
+                    p3[k] = fma(gi, zr, p3[k]);
+                    p4[k] = fma(gr, zi, p4[k]);
                 }
+            }
+    }
+    const size_t nb = gridDim.x, b = blockIdx.x;
+    if (work) {
+        // q = (j - 1) nm + im - 1 for pitch index j
+        const double r0 = wave_sum_dpp(zsr), i0 = wave_sum_dpp(zsi);
+        if (lane == 0 && k0 == 1) {
+            const int q = (jc - 1) * nm + im - 1;
+            part[(size_t)q * nb + b] = r0;
+            part[(size_t)(nq + q) * nb + b] = i0;
+        }
+        if (lane == 0 && k0 == 1 && np % 2 == 0) {   // index np / 2 holds no pitch
+            const int q = (np / 2 - 1) * nm + im - 1;
+            part[(size_t)q * nb + b] = 0.0;
+            part[(size_t)(nq + q) * nb + b] = 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            if (k >= pl.len || k0 + k > pl.kmax) break;
+            const double a1 = wave_sum_dpp(p1[k]), a2 = wave_sum_dpp(p2[k]);
+            const double a3 = wave_sum_dpp(p3[k]), a4 = wave_sum_dpp(p4[k]);
+            if (lane == 0) {
+                // offset k0 + k: g z; its mirror: conj(g) z
+                const int qp = (jc + k0 + k - 1) * nm + im - 1;
+                const int qm = (np - jc - k0 - k) * nm + im - 1;
+                part[(size_t)qp * nb + b] = a1 - a2;
+                part[(size_t)(nq + qp) * nb + b] = a3 + a4;
+                part[(size_t)qm * nb + b] = a1 + a2;
+                part[(size_t)(nq + qm) * nb + b] = a4 - a3;
             }
         }
     }
-    cnt = wave_sum(cnt);
-    if (lane == 0) cnt_w[w] = cnt;
-    __syncthreads();
-    double *out = part + (size_t)blockIdx.x * (2 * nq + 1);
-    for (int q = tid; q < 2 * nq; q += LG_BLOCK) {
-        double v = 0.0;
-        for (int ww = 0; ww < LG_WAVES; ww++) v += acc[ww][q];
-        // [cos parts][sin parts]
-        out[(q & 1) * nq + (q >> 1)] = v;
-    }
-    if (tid == 0) {
-        double v = 0.0;
-        for (int ww = 0; ww < LG_WAVES; ww++) v += cnt_w[ww];
-        out[2 * nq] = v;
+    if (blockIdx.y == 0) {
+        cnt = wave_sum_dpp(cnt);
+        if (lane == 0) s_cnt[w] = cnt;
+        __syncthreads();
+        if (tid == 0) {
+            double v = 0.0;
+            for (int k = 0; k < T / 64; k++) v += s_cnt[k];
+            part[2 * (size_t)nq * nb + b] = v;
+        }
     }
 }
 
-// out[2 * nq] = (sum over blocks in order) / count
-__global__ __launch_bounds__(LG_BLOCK) void lgsp_sum_kernel(const double *__restrict__ part,
-                                                             int nb, int nq,
-                                                             double *__restrict__ out) {
-    const int stride = 2 * nq + 1;
-    double cnt = 0.0;
-    for (int b = 0; b < nb; b++) cnt += part[(size_t)b * stride + 2 * nq];
-    const double inv = cnt > 0.0 ? 1.0 / cnt : 0.0;
-    for (int q = threadIdx.x; q < 2 * nq; q += LG_BLOCK) {
-        double v = 0.0;
-        for (int b = 0; b < nb; b++) v += part[(size_t)b * stride + q];
-        out[q] = v * inv;
-    }
+// Fixed-order sum of row[0 .. nb) over the block.
+__device__ __forceinline__ double lg_row_sum(const double *__restrict__ row, int nb,
+                                             double *red) {
+    const int tid = threadIdx.x;
+    double v = 0.0;
+    for (int b = tid; b < nb; b += LG_SUM_BLOCK) v += row[b];
+    v = wave_sum_dpp(v);
+    __syncthreads();
+    if ((tid & 63) == 0) red[tid >> 6] = v;
+    __syncthreads();
+    v = red[0];
+    for (int k = 1; k < LG_SUM_BLOCK / 64; k++) v += red[k];
+    return v;
+}
+
+// block q: out[q] = (sum of the blocks' partials of q) / count
+__global__ __launch_bounds__(LG_SUM_BLOCK) void lgsp_sum_kernel(const double *__restrict__ part,
+                                                                 int nb, int nq,
+                                                                 double *__restrict__ out) {
+    __shared__ double red[LG_SUM_BLOCK / 64];
+    const double v = lg_row_sum(part + (size_t)blockIdx.x * nb, nb, red);
+    const double cnt = lg_row_sum(part + 2 * (size_t)nq * nb, nb, red);
+    if (threadIdx.x == 0) out[blockIdx.x] = cnt > 0.0 ? v * (1.0 / cnt) : 0.0;
+}
+
+template <typename R, int KC>
+static void launch_lgsp_part(const void *xv, int ps, const uint8_t *zone, long long n, int nz,
+                             int offanal, int nsect, int np, int nm, double lscale,
+                             const LgPlan &pl, double *part, hipStream_t s) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(lgsp_part_kernel<R, KC>), dim3(pl.nb, pl.groups),
+                       dim3(64 * pl.waves), 0, s, (const typename Vec4<R>::T *)xv, ps, zone, n,
+                       nz, offanal, nsect, np, nm, 1.0 / lscale, pl, part);
 }
 
 template <typename R>
 hipError_t launch_lgspia(const void *xv, int ps, const uint8_t *zone, long long n, int nz,
                          int offanal, int nsect, int np, int nm, double lscale, double *part,
-                         int nb, double *out, hipStream_t s) {
+                         double *out, hipStream_t s) {
     if (np * nm > LG_MAXQ) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(lgsp_part_kernel<R>, dim3(nb), dim3(LG_BLOCK), 0, s,
-                       (const typename Vec4<R>::T *)xv, ps, zone, n, nz, offanal, nsect, np, nm,
-                       1.0 / lscale, part);
-    hipLaunchKernelGGL(lgsp_sum_kernel, dim3(1), dim3(LG_BLOCK), 0, s, (const double *)part, nb,
-                       np * nm, out);
+    const LgPlan pl = lg_plan(n, np, nm);
+    if (pl.len <= 4)
+        launch_lgsp_part<R, 4>(xv, ps, zone, n, nz, offanal, nsect, np, nm, lscale, pl, part, s);
+    else if (pl.len <= 8)
+        launch_lgsp_part<R, 8>(xv, ps, zone, n, nz, offanal, nsect, np, nm, lscale, pl, part, s);
+    else
+        launch_lgsp_part<R, 12>(xv, ps, zone, n, nz, offanal, nsect, np, nm, lscale, pl, part, s);
+    hipLaunchKernelGGL(lgsp_sum_kernel, dim3(2 * np * nm), dim3(LG_SUM_BLOCK), 0, s,
+                       (const double *)part, pl.nb, np * nm, out);
     return hipGetLastError();
 }
 
 }  // namespace gh
 
 using namespace gh;
-
-// Blocks of the partial-sum pass: enough to fill the device, each striding
-// over the particles (the sums' order depends only on n and this count).
-static int lgsp_blocks(long long n) {
-    long long nb = (n + LG_BLOCK - 1) / LG_BLOCK;
-    if (nb > 2048) nb = 2048;
-    return nb < 1 ? 1 : (int)nb;
-}
 
 extern "C" int galhip_lgspia(galhip_ctx *c, int32_t np, int32_t nm, double lscale,
                              double *out) {
@@ -176,7 +260,7 @@ extern "C" int galhip_lgspia(galhip_ctx *c, int32_t np, int32_t nm, double lscal
     int nbmax = 1;
     for (int m = 0; m < c->nmem; m++) {
         const long long nm_ = c->ens ? c->m_off[m + 1] - c->m_off[m] : c->n;
-        nbmax = std::max(nbmax, lgsp_blocks(nm_));
+        nbmax = std::max(nbmax, lg_plan(nm_, np, nm).nb);
     }
     int rc = dalloc(&part, sizeof(double) * (size_t)nbmax * (2 * nq + 1)) |
              dalloc(&dout, sizeof(double) * (size_t)c->nmem * 2 * nq);
@@ -192,10 +276,10 @@ extern "C" int galhip_lgspia(galhip_ctx *c, int32_t np, int32_t nm, double lscal
             const uint8_t *zn = c->zone + off;
             e = c->prec == GALHIP_FP32
                     ? launch_lgspia<float>(xv, ps, zn, cnt, c->nz, c->offanal, c->nsect, np,
-                                           nm, lscale, part, lgsp_blocks(cnt),
+                                           nm, lscale, part,
                                            dout + 2 * nq * m, c->s)
                     : launch_lgspia<double>(xv, ps, zn, cnt, c->nz, c->offanal, c->nsect, np,
-                                            nm, lscale, part, lgsp_blocks(cnt),
+                                            nm, lscale, part,
                                             dout + 2 * nq * m, c->s);
         }
         if (e == hipSuccess)
