@@ -667,18 +667,14 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_gather_kernel(P3GatherArgs<R> b)
 }
 
 // icheck's global integrals for the 3-D grid (SRC/lib15/icheck.f:24-70):
-// per-block FP64 sums of 11 quantities in a fixed order, then one block adds
-// the block sums in order.  [0] count, [1..3] position, [4..6] velocity per
+// per-block FP64 sums of 11 quantities in a fixed order (P3_INT_PT particles
+// per thread, as on the p2d grid), then a block per quantity adds the block
+// sums in a fixed order.  [0] count, [1..3] position, [4..6] velocity per
 // zone-1 step ((v + a/2)/tfac when centred), [7] v^2, [8] Lz, [9] the grid
 // potential interpolated with the particle's own weights (grid particles),
 // [10] the fixed potential of the spherical radius.
 constexpr int NINT3 = 11;
-
-__device__ __forceinline__ double p3_wave_sumd(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
+constexpr int P3_INT_PT = 8;
 
 template <typename R, int J>
 __global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_kernel(P3Args<R> a, int with_pot,
@@ -688,11 +684,12 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_kernel(P3Args<R> a, in
     typedef typename Vec4<R>::T R4;
     __shared__ double red[P3_PBLOCK / 64][NINT3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const long long i = (long long)blockIdx.x * P3_PBLOCK + tid;
     double v[NINT3];
 #pragma unroll
     for (int q = 0; q < NINT3; q++) v[q] = 0.0;
-    if (i < a.n) {
+    for (int k = 0; k < P3_INT_PT; k++) {
+        const long long i = ((long long)blockIdx.x * P3_INT_PT + k) * P3_PBLOCK + tid;
+        if (i >= a.n) break;
         const int z = a.zone[i];
         if (z >= 1) {
             const R4 p = a.rec[2 * i];
@@ -711,15 +708,15 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_kernel(P3Args<R> a, in
             const double sf = 1.0 / (double)a.nstep[zs - 1];
             const double x = p.x, y = p.y, zz = p.z;
             const double ux = vx * sf, uy = vy * sf, uz = vz * sf;
-            v[0] = 1.0;
-            v[1] = x;
-            v[2] = y;
-            v[3] = zz;
-            v[4] = ux;
-            v[5] = uy;
-            v[6] = uz;
-            v[7] = ux * ux + uy * uy + uz * uz;
-            v[8] = x * uy - y * ux;
+            v[0] += 1.0;
+            v[1] += x;
+            v[2] += y;
+            v[3] += zz;
+            v[4] += ux;
+            v[5] += uy;
+            v[6] += uz;
+            v[7] += ux * ux + uy * uy + uz * uz;
+            v[8] += x * uy - y * ux;
             if (with_pot && z <= a.nz) {
                 constexpr int NW = P3NW<J>::v;
                 R w[NW];
@@ -730,41 +727,38 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_kernel(P3Args<R> a, in
                 double ph = 0.0;
                 for (int k = 0; k < NW; k++)
                     if (ic[k] >= 0 && ic[k] < a.mesh) ph += (double)w[k] * (double)a.fld[ic[k]].w;
-                v[9] = ph;
+                v[9] += ph;
             }
             if (nfp > 0)
-                v[10] = fixforce(sqrt(x * x + y * y + zz * zz), nfp, 1.0 / fp_dr, fp_c);
+                v[10] += fixforce(sqrt(x * x + y * y + zz * zz), nfp, 1.0 / fp_dr, fp_c);
         }
     }
 #pragma unroll
     for (int q = 0; q < NINT3; q++) {
-        const double t = p3_wave_sumd(v[q]);
+        const double t = wave_sum_dpp(v[q]);
         if (lane == 0) red[wave][q] = t;
     }
     __syncthreads();
     if (tid < NINT3) {
         double t = 0.0;
         for (int w = 0; w < P3_PBLOCK / 64; w++) t += red[w][tid];
-        part[(long long)blockIdx.x * NINT3 + tid] = t;
+        part[(long long)tid * gridDim.x + blockIdx.x] = t;
     }
 }
 
-__global__ __launch_bounds__(P3_BLOCK) void p3_integrals_sum_kernel(const double *part, int nb,
-                                                                    double *out) {
-    __shared__ double red[P3_BLOCK / 64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int q = 0; q < NINT3; q++) {
-        double t = 0.0;
-        for (int b = tid; b < nb; b += P3_BLOCK) t += part[(long long)b * NINT3 + q];
-        t = p3_wave_sumd(t);
-        if (lane == 0) red[wave] = t;
-        __syncthreads();
-        if (tid == 0) {
-            double s = 0.0;
-            for (int w = 0; w < P3_BLOCK / 64; w++) s += red[w];
-            out[q] = s;
-        }
-        __syncthreads();
+__global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_sum_kernel(const double *part, int nb,
+                                                                     double *out) {
+    __shared__ double red[P3_PBLOCK / 64];
+    const int tid = threadIdx.x, q = blockIdx.x;
+    double t = 0.0;
+    for (int b = tid; b < nb; b += P3_PBLOCK) t += part[(long long)q * nb + b];
+    t = wave_sum_dpp(t);
+    if ((tid & 63) == 0) red[tid >> 6] = t;
+    __syncthreads();
+    if (tid == 0) {
+        double s = 0.0;
+        for (int w = 0; w < P3_PBLOCK / 64; w++) s += red[w];
+        out[q] = s;
     }
 }
 
@@ -1323,7 +1317,7 @@ template <typename R>
 hipError_t launch_p3_integrals(const P3Args<R> &a, int with_pot, const double4 *fp_c,
                                int nfp, double fp_dr, int centred,
                                double *part, double *out, hipStream_t s) {
-    const unsigned nb = a.n > 0 ? p3_blocks(a.n) : 0;
+    const unsigned nb = a.n > 0 ? p3_blocks((a.n + P3_INT_PT - 1) / P3_INT_PT) : 0;
     if (nb && a.jmass == 3)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_integrals_kernel<R, 3>), dim3(nb), dim3(P3_PBLOCK), 0, s, a,
                            with_pot, fp_c, nfp, fp_dr, centred, part);
@@ -1332,7 +1326,7 @@ hipError_t launch_p3_integrals(const P3Args<R> &a, int with_pot, const double4 *
                            with_pot, fp_c, nfp, fp_dr, centred, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(p3_integrals_sum_kernel, dim3(1), dim3(P3_BLOCK), 0, s, part, (int)nb,
+    hipLaunchKernelGGL(p3_integrals_sum_kernel, dim3(NINT3), dim3(P3_PBLOCK), 0, s, part, (int)nb,
                        out);
     return hipGetLastError();
 }
