@@ -831,15 +831,15 @@ extern "C" int galhip_adj_record(galhip_ctx *c, int32_t slot) {
              dalloc(&s.zone, n ? n : 1) | dalloc(&s.id, sizeof(unsigned) * (n ? n : 1)) |
              dalloc(&s.counters, sizeof(long long) * 4) |
              dalloc(&s.mass, sizeof(long long) * cells * c->nz) |
-             dalloc(&s.rng, sizeof(int) * 2 * GH_MAXZ);
+             dalloc(&s.rng, sizeof(int) * 2 * range_ints(c));
         if (rc) return rc;
         s.n = c->n;
     }
     for (int z = 0; z < c->nz; z++)
         HIPCHK(hipMemcpyAsync(s.mass + z * cells, c->mfx[z], sizeof(long long) * cells,
                               hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(hipMemcpyAsync(s.rng, c->jrad, sizeof(int) * GH_MAXZ, hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(hipMemcpyAsync(s.rng + GH_MAXZ, c->krad, sizeof(int) * GH_MAXZ,
+    HIPCHK(hipMemcpyAsync(s.rng, c->jrad, sizeof(int) * range_ints(c), hipMemcpyDeviceToDevice, c->s));
+    HIPCHK(hipMemcpyAsync(s.rng + range_ints(c), c->krad, sizeof(int) * range_ints(c),
                           hipMemcpyDeviceToDevice, c->s));
     if (n) {
         HIPCHK(hipMemcpyAsync(s.xv, c->xv, 4 * es * n, hipMemcpyDeviceToDevice, c->s));
@@ -875,8 +875,8 @@ extern "C" int galhip_adj_restore(galhip_ctx *c, int32_t slot) {
     for (int z = 0; z < c->nz; z++)
         HIPCHK(hipMemcpyAsync(c->mfx[z], s.mass + z * cells, sizeof(long long) * cells,
                               hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(hipMemcpyAsync(c->jrad, s.rng, sizeof(int) * GH_MAXZ, hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(hipMemcpyAsync(c->krad, s.rng + GH_MAXZ, sizeof(int) * GH_MAXZ,
+    HIPCHK(hipMemcpyAsync(c->jrad, s.rng, sizeof(int) * range_ints(c), hipMemcpyDeviceToDevice, c->s));
+    HIPCHK(hipMemcpyAsync(c->krad, s.rng + range_ints(c), sizeof(int) * range_ints(c),
                           hipMemcpyDeviceToDevice, c->s));
     c->istep = s.istep;
     c->order_ver = s.order_ver;

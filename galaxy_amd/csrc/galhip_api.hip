@@ -71,7 +71,7 @@ hipError_t launch_ens_gemm(const EnsGemmArgs &, int, hipStream_t);
 hipError_t launch_d2f(const double *, float *, long long, hipStream_t);
 hipError_t launch_fill_i64(long long *, long long, long long, hipStream_t);
 hipError_t launch_fill_i32(int *, int, long long, hipStream_t);
-hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, int,
+hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, int, int,
                          hipStream_t);
 }  // namespace gh
 
@@ -200,11 +200,13 @@ static int p2d_create(const galhip_p2d_params *p, int nmem, const double *pmass,
         rc |= dalloc(&c->mfx[z], sizeof(long long) * cells);
         rc |= dalloc(&c->moz[z], sizeof(long long) * cells);
     }
-    rc |= dalloc(&c->jrad, sizeof(int) * GH_MAXZ * nm);
-    rc |= dalloc(&c->krad, sizeof(int) * GH_MAXZ * nm);
+    c->rstride = range_stride(nmem);
+    rc |= dalloc(&c->jrad, sizeof(int) * range_ints(c));
+    rc |= dalloc(&c->krad, sizeof(int) * range_ints(c));
     rc |= dalloc(&c->ranges, sizeof(int) * 4 * nm);
     rc |= dalloc(&c->lg_d, sizeof(int) * c->mmax);
     rc |= dalloc(&c->counters, sizeof(long long) * 4 * nm);
+    rc |= dalloc(&c->push_cnt, sizeof(long long) * 8 * GH_PUSH_STRIPES);
     rc |= dalloc(&c->rho, es * cells);
     rc |= dalloc(&c->coef, es * c->ncoef * c->nr * nm);
     rc |= dalloc(&c->fld2, 2 * es * cells);
@@ -234,10 +236,11 @@ static int p2d_create(const galhip_p2d_params *p, int nmem, const double *pmass,
         HIPCHK(hipMemcpy(c->tw, twd.data(), sizeof(double) * 2 * na, hipMemcpyHostToDevice));
     }
     HIPCHK(hipMemcpy(c->lg_d, c->lg.data(), sizeof(int) * c->mmax, hipMemcpyHostToDevice));
-    std::vector<int> jr(GH_MAXZ * nm, c->nr), kr(GH_MAXZ * nm, 0);
-    HIPCHK(hipMemcpy(c->jrad, jr.data(), sizeof(int) * GH_MAXZ * nm, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->krad, kr.data(), sizeof(int) * GH_MAXZ * nm, hipMemcpyHostToDevice));
+    std::vector<int> jr(range_ints(c), c->nr), kr(range_ints(c), 0);
+    HIPCHK(hipMemcpy(c->jrad, jr.data(), sizeof(int) * jr.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->krad, kr.data(), sizeof(int) * kr.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->counters, 0, sizeof(long long) * 4 * nm));
+    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     HIPCHK(hipMemset(c->fld2, 0, 2 * es * cells));
     HIPCHK(hipMemset(c->pot, 0, es * cells));
     HIPCHK(hipMemset(c->rho, 0, es * cells));
@@ -283,6 +286,7 @@ extern "C" int galhip_free(galhip_ctx *c) {
     free_particles(c);
     for (int z = 0; z < GH_MAXZ; z++) { dfree(c->mfx[z]); dfree(c->moz[z]); }
     dfree(c->jrad); dfree(c->krad); dfree(c->ranges); dfree(c->lg_d); dfree(c->counters);
+    dfree(c->push_cnt);
     dfree(c->fp_c);
     dfree(c->rho); dfree(c->coef); dfree(c->fld2); dfree(c->pot); dfree(c->tw); dfree(c->twd);
     if (c->G != (void *)c->Gd) dfree(c->G);
@@ -547,7 +551,7 @@ extern "C" int galhip_restrt(galhip_ctx *c, int64_t n, const void *x,
     if (rc) return rc;
     size_t es = esize(c);
     std::vector<uint8_t> z(n);
-    long long cnt[4] = {0, 0, 0, 0};   // counters: [0] noff, [1] pushes
+    long long cnt[4] = {0, 0, 0, 0};   // counters: [0] noff
     for (long long i = 0; i < n; i++) {
         int v = iz[i];
         if (v < 1 || v > c->nz + 1)
@@ -556,6 +560,7 @@ extern "C" int galhip_restrt(galhip_ctx *c, int64_t n, const void *x,
         if (v == c->nz + 1) cnt[0]++;    // /admin/ noff: the off-grid list
     }
     HIPCHK(hipMemcpy(c->counters, cnt, sizeof cnt, hipMemcpyHostToDevice));
+    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     c->qbits = qbits_for(n);
     c->order_ver++;
     if (n == 0) return 0;
@@ -695,6 +700,12 @@ static UtConst ut_const(const galhip_ctx *c) {
     return k;
 }
 
+// Particles per thread of the push and the mass assignment (the table at
+// PushShape): FP64 one; FP32 one up to 1.5e6 particles, four above.
+static int push_ppt(int prec, long long n) {
+    return prec == GALHIP_FP64 || n <= 1500000 ? 1 : 4;
+}
+
 template <typename R> static PushArgs<R> push_args(galhip_ctx *c) {
     PushArgs<R> a;
     memset(&a, 0, sizeof a);
@@ -706,7 +717,9 @@ template <typename R> static PushArgs<R> push_args(galhip_ctx *c) {
     for (int z = 0; z < c->nz; z++) a.mfx[z] = c->mfx[z];
     a.jrad = c->jrad;
     a.krad = c->krad;
+    a.rstride = c->rstride;
     a.counters = c->counters;
+    a.pushes = c->push_cnt;
     a.fr_c = c->fr_c;
     a.fr_inv_dr = c->nfr > 0 ? 1.0 / c->fr_dr : 0.0;
     a.nfr = c->nfr;
@@ -724,6 +737,7 @@ template <typename R> static PushArgs<R> push_args(galhip_ctx *c) {
         a.qbits_m = c->m_qbits_d;
         a.nblocks = c->nblk;
     }
+    a.ppt = push_ppt(c->prec, c->n);
     a.xlo = (typename Vec2<R>::T *)c->xlo;
     return a;
 }
@@ -771,7 +785,7 @@ static AnaArgs<R> ana_args(galhip_ctx *c, int lpot, int explicit_zones,
         a.use_new[z] = c->use_new[z];
         a.use_old[z] = c->use_old[z];
     }
-    a.jrad = c->jrad; a.krad = c->krad; a.ranges = c->ranges;
+    a.jrad = c->jrad; a.krad = c->krad; a.rstride = c->rstride; a.ranges = c->ranges;
     a.rho = (R *)c->rho; a.coef = (R *)c->coef; a.tw = (const R *)c->tw; a.lg = c->lg_d;
     a.q = ldexp(1.0, -c->qbits);
     a.pmass = c->pmass;
@@ -796,6 +810,7 @@ template <typename R> static SynArgs<R> syn_args(galhip_ctx *c, int lpot,
     }
     a.jrad = c->jrad;
     a.krad = c->krad;
+    a.rstride = c->rstride;
     a.masscl_z = masscl_z;
     a.coef = (const R *)c->coef;
     a.G = (const R *)c->G;
@@ -818,8 +833,8 @@ template <typename R> static int masset_impl(galhip_ctx *c) {
     ZonePtrs zp;
     memset(&zp, 0, sizeof zp);
     for (int z = 0; z < c->nz; z++) { zp.mfx[z] = c->mfx[z]; zp.moz[z] = c->moz[z]; }
-    HIPCHK(launch_masscl(zp, c->nz, c->mesh, c->jrad, c->krad, c->nr, c->nmem, c->s));
-    for (int m = 0; m < c->nmem; m++) HIPCHK(launch_massgn<R>(member_args<R>(c, m), c->s));
+    HIPCHK(launch_masscl(zp, c->nz, c->mesh, c->jrad, c->krad, c->rstride, c->nr, c->nmem, c->s));
+    HIPCHK(launch_massgn<R>(push_args<R>(c), c->s));
     int rc = zoncmb_host(c);
     if (rc) return rc;
     c->masscl_done = 0;
@@ -979,7 +994,7 @@ template <typename R> static int step_impl(galhip_ctx *c) {
         ZonePtrs zp;
         memset(&zp, 0, sizeof zp);
         for (int z = 0; z < c->nz; z++) { zp.mfx[z] = c->mfx[z]; zp.moz[z] = c->moz[z]; }
-        HIPCHK(launch_masscl(zp, c->mzone, c->mesh, c->jrad, c->krad, c->nr, c->nmem, c->s));
+        HIPCHK(launch_masscl(zp, c->mzone, c->mesh, c->jrad, c->krad, c->rstride, c->nr, c->nmem, c->s));
     }
     c->masscl_done = 0;
     PushArgs<R> a = push_args<R>(c);
@@ -1347,6 +1362,7 @@ static int group_impl(galhip_ctx *c, int kind, int64_t n, void *x, void *y, void
         a.ut = dut;
         a.zone = dz;
         a.n = n;
+        a.ppt = push_ppt(c->prec, n);
         a.xlo = nullptr;
         if (e == hipSuccess) {
             if (kind == GRP_GETACC) e = launch_getacc_group<R>(a, dacc, c->s);
@@ -1440,8 +1456,21 @@ static int get_mass_m(const galhip_ctx *c, int m, int64_t *mfx, int64_t *mozfx, 
         if (mfx) HIPCHK(hipMemcpy(mfx + (size_t)z * c->mesh, c->mfx[z] + mo, 8 * c->mesh, hipMemcpyDeviceToHost));
         if (mozfx) HIPCHK(hipMemcpy(mozfx + (size_t)z * c->mesh, c->moz[z] + mo, 8 * c->mesh, hipMemcpyDeviceToHost));
     }
-    if (jrad) HIPCHK(hipMemcpy(jrad, c->jrad + m * GH_MAXZ, sizeof(int) * c->nz, hipMemcpyDeviceToHost));
-    if (krad) HIPCHK(hipMemcpy(krad, c->krad + m * GH_MAXZ, sizeof(int) * c->nz, hipMemcpyDeviceToHost));
+    const size_t w = sizeof(int) * c->nz, pitch = sizeof(int) * c->rstride;
+    std::vector<int> v((size_t)GH_RANGE_STRIPES * c->nz);
+    for (int hi = 0; hi < 2; hi++) {
+        int32_t *out = hi ? krad : jrad;
+        if (!out) continue;
+        HIPCHK(hipMemcpy2D(v.data(), w, (hi ? c->krad : c->jrad) + m * GH_MAXZ, pitch, w,
+                           GH_RANGE_STRIPES, hipMemcpyDeviceToHost));
+        for (int z = 0; z < c->nz; z++) {
+            out[z] = v[z];
+            for (int s = 1; s < GH_RANGE_STRIPES; s++) {
+                const int x = v[(size_t)s * c->nz + z];
+                out[z] = hi ? std::max(out[z], x) : std::min(out[z], x);
+            }
+        }
+    }
     if (qbits) *qbits = c->ens ? c->m_qbits[m] : c->qbits;
     return 0;
 }
@@ -1463,8 +1492,16 @@ extern "C" int galhip_set_mass(galhip_ctx *c, const int64_t *mfx,
         if (mfx) HIPCHK(hipMemcpy(c->mfx[z], mfx + (size_t)z * c->mesh, 8 * c->mesh, hipMemcpyHostToDevice));
         if (mozfx) HIPCHK(hipMemcpy(c->moz[z], mozfx + (size_t)z * c->mesh, 8 * c->mesh, hipMemcpyHostToDevice));
     }
-    if (jrad) HIPCHK(hipMemcpy(c->jrad, jrad, sizeof(int) * c->nz, hipMemcpyHostToDevice));
-    if (krad) HIPCHK(hipMemcpy(c->krad, krad, sizeof(int) * c->nz, hipMemcpyHostToDevice));
+    // every stripe holds the given range
+    const size_t w = sizeof(int) * c->nz, pitch = sizeof(int) * c->rstride;
+    std::vector<int> v((size_t)GH_RANGE_STRIPES * c->nz);
+    for (int hi = 0; hi < 2; hi++) {
+        const int32_t *in = hi ? krad : jrad;
+        if (!in) continue;
+        for (size_t e = 0; e < v.size(); e++) v[e] = in[e % c->nz];
+        HIPCHK(hipMemcpy2D(hi ? c->krad : c->jrad, pitch, v.data(), w, w, GH_RANGE_STRIPES,
+                           hipMemcpyHostToDevice));
+    }
     return 0;
 }
 
@@ -1548,11 +1585,10 @@ extern "C" int galhip_get_noff(const galhip_ctx *c, int64_t *noff) {
 
 // pushes counted so far over every grid of the context
 static int pushes_total(const galhip_ctx *c, long long *out) {
-    const int nm = c->nmem > 0 ? c->nmem : 1;
-    std::vector<long long> v(4 * (size_t)nm);
-    HIPCHK(hipMemcpy(v.data(), c->counters, sizeof(long long) * v.size(), hipMemcpyDeviceToHost));
+    std::vector<long long> v(8 * GH_PUSH_STRIPES);
+    HIPCHK(hipMemcpy(v.data(), c->push_cnt, sizeof(long long) * v.size(), hipMemcpyDeviceToHost));
     long long t = 0;
-    for (int m = 0; m < nm; m++) t += v[4 * m + 1];
+    for (int k = 0; k < GH_PUSH_STRIPES; k++) t += v[8 * k];
     *out = t;
     return 0;
 }
@@ -1612,10 +1648,10 @@ extern "C" int galhip_ens_restrt(galhip_ctx *c, const int64_t *count, const void
     c->tcent = 0;
     int rc = ensure_particles(c, n);
     if (rc) return rc;
-    // member ranges, push blocks of at most GH_PUSH_PER particles that never
+    // member ranges, push blocks of at most `per` particles that never
     // straddle two members, fixed-point scales as a lone disc of that size
     // would have them
-    const int per = GH_PUSH_PER;
+    const int per = GH_PUSH_BLOCK * push_ppt(c->prec, n);
     std::vector<int4> blk;
     c->m_off.assign(c->nmem + 1, 0);
     for (int m = 0; m < c->nmem; m++) {
@@ -1643,6 +1679,7 @@ extern "C" int galhip_ens_restrt(galhip_ctx *c, const int64_t *count, const void
             if (v == c->nz + 1) cnt[4 * m]++;
         }
     HIPCHK(hipMemcpy(c->counters, cnt.data(), sizeof(long long) * cnt.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     drop_graphs(c);
     if (n == 0) return 0;
     rc = load_xv(c, n, x, y, vx, vy);

@@ -48,8 +48,10 @@ struct galhip_ctx {
     void *sort_tmp;
     size_t sort_tmp_bytes;
     long long *mfx[GH_MAXZ], *moz[GH_MAXZ];
-    int *jrad, *krad, *ranges, *lg_d;
-    long long *counters;
+    int *jrad, *krad, *ranges, *lg_d;   // ring ranges in stripes (widen_range)
+    int rstride;
+    long long *counters;              // [0] off-grid count (per grid)
+    long long *push_cnt;              // pushes, striped (count_pushes)
     void *rho, *coef, *fld2, *pot, *G, *tw;
     double *Gd, *twd;
     // fixed radial tables as cubic coefficients per interval (radtab_coeffs):
@@ -117,7 +119,7 @@ struct galhip_ctx {
         unsigned *id;
         long long *counters;
         long long *mass;              // zone sums [nz][mesh]
-        int *rng;                     // jrad, krad [2][GH_MAXZ]
+        int *rng;                     // jrad, krad
         long long n, order_ver;
         int istep;
     };
@@ -134,6 +136,10 @@ struct galhip_ctx {
     float *wpre;
     double gemm_us[3];
 };
+
+// Row length of the striped ring ranges and their size in ints.
+static int range_stride(int nmem) { return (nmem * GH_MAXZ + 31) / 32 * 32; }
+static size_t range_ints(const galhip_ctx *c) { return (size_t)GH_RANGE_STRIPES * c->rstride; }
 
 static size_t esize(const galhip_ctx *c) { return c->prec == GALHIP_FP64 ? 8 : 4; }
 
@@ -180,7 +186,7 @@ namespace gh {
 hipError_t launch_d2f(const double *, float *, long long, hipStream_t);
 hipError_t launch_fill_i64(long long *, long long, long long, hipStream_t);
 hipError_t launch_fill_i32(int *, int, long long, hipStream_t);
-hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, int,
+hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, int, int,
                          hipStream_t);
 }  // namespace gh
 

@@ -13,15 +13,8 @@
 
 #define GH_MAXZ 10
 #define GH_BLOCK 256
-// the p2d push kernel's launch shape: threads per block and particles per
-// thread (a block takes GH_PUSH_PER consecutive particles)
-#ifndef GH_PUSH_BLOCK
+// threads per block of the p2d push and mass assignment
 #define GH_PUSH_BLOCK 256
-#endif
-#ifndef GH_PPT
-#define GH_PPT 4
-#endif
-#define GH_PUSH_PER (GH_PUSH_BLOCK * GH_PPT)
 // 2.d0 * pi of SRC/lib15/inc/pi.f
 #define GH_TWO_PI (2.0 * 3.141592653589793238462643)
 
@@ -156,6 +149,136 @@ __device__ __forceinline__ void ut_of(double x, double y, double rr,
     u = l / k.alpha_d;
     t = gh_atan2(y, x, tab) * (double)k.na / GH_TWO_PI;
     if (t < 0.0) t = t + (double)k.na;
+}
+
+// ---- the same values with fewer instructions (FP32) -------------------------
+//
+// The push kernels are bound by VALU issue, and the general forms of the
+// FP32 square root and quotient (operand scaling, special cases) and of the
+// logarithm and angle to double precision were a third of a particle's
+// instructions.  The forms below return the same bits: each takes a short
+// evaluation whose error is bounded, tests whether that could have changed
+// the rounded result (or whether an operand is outside the range the short
+// form is for), and only a wavefront with such a lane takes the general form
+// for it, behind a wave-uniform branch (the empty asm in it keeps the
+// compiler from evaluating both forms and selecting).
+__device__ __forceinline__ bool any_lane(bool c) { return __ballot(c) != 0; }
+
+// sqrt(x), correctly rounded: the hardware estimate is within one unit, and
+// the two neighbours' residuals decide (no scaling for x >= 2^-96).
+__device__ __forceinline__ double sqrt_rn(double x) { return sqrt(x); }
+__device__ __forceinline__ float sqrt_rn(float x) {
+    float s = __builtin_amdgcn_sqrtf(x);
+    const float lo = __uint_as_float(__float_as_uint(s) - 1u);
+    const float hi = __uint_as_float(__float_as_uint(s) + 1u);
+    const float rlo = fmaf(-lo, s, x), rhi = fmaf(-hi, s, x);
+    s = rlo <= 0.0f ? lo : s;
+    s = rhi > 0.0f ? hi : s;
+    const bool out = !(x >= 0x1p-96f && x < 0x1p126f);
+    if (any_lane(out)) {
+        asm volatile("");
+        if (out) s = sqrt(x);
+    }
+    return s;
+}
+
+// a / b, correctly rounded: reciprocal with one Newton step, the quotient
+// corrected twice by its residual (|a| and b within 2^-60 .. 2^60, where no
+// step can underflow or overflow).
+__device__ __forceinline__ double div_rn(double a, double b) { return a / b; }
+__device__ __forceinline__ float div_rn(float a, float b) {
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    float q = a * r;
+    q = fmaf(fmaf(-b, q, a), r, q);
+    q = fmaf(fmaf(-b, q, a), r, q);
+    const float m = fabsf(a);
+    const bool out = !(m >= 0x1p-60f && m < 0x1p60f && b >= 0x1p-60f && b < 0x1p60f);
+    if (any_lane(out)) {
+        asm volatile("");
+        if (out) q = a / b;
+    }
+    return q;
+}
+
+// Tables of ut_push, staged in LDS: FP64 those of galhip_math.h; FP32
+// [0, 32) ln(1 + j/32), [32, 49) atan(j/16).
+template <typename R> struct UtTab { static constexpr int n = sizeof(R) == 4 ? 49 : GH_MATH_TAB_N; };
+template <typename R> __device__ __forceinline__ double ut_tab_entry(int j) {
+    if (sizeof(R) == 8) return GH_MATH_TAB[j];
+    return j < 32 ? GH_MATH_TAB[GH_LOGC_HI + j] + GH_MATH_TAB[GH_LOGC_LO + j]
+                  : GH_MATH_TAB[GH_ATANC_HI + j - 32];
+}
+
+// Could an error of GH_UT_SLACK units in the last place of the double d, or
+// a magnitude outside 2^-119 .. 2^127, change its rounding to float?  (The
+// low 29 bits of the significand against the midpoint.)
+#define GH_UT_SLACK 8192u
+__device__ __forceinline__ bool float_rounding_open(double d) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(d);
+    const unsigned low = (unsigned)b & 0x1fffffffu, hi = (unsigned)(b >> 32) & 0x7fffffffu;
+    return low - (0x10000000u - GH_UT_SLACK) < 2u * GH_UT_SLACK ||
+           hi - 0x38800000u >= 0x47e00000u - 0x38800000u;
+}
+
+// 1 / d from the hardware estimate (2^-23) and one Newton step (2^-46)
+__device__ __forceinline__ double rcp_46(double d) {
+    const double r = __builtin_amdgcn_rcp(d);
+    return fma(fma(-d, r, 1.0), r, r);
+}
+
+// ut_of for a position on the grid (rr = its radius).  FP32: ln v with
+// v = 1 + r = m 2^e and the angle by the table reductions of galhip_math.h,
+// the quotients by rcp_46 and the series cut at 2^-48: together within
+// 2^-43 of the value (2^-48.6 at most in 2.4e9 samples), 512 units in the
+// last place; l and t keep the bits ut_of gives them through the test above.
+// Push of 1e7 particles in three zones: 110 us with ut_of, 102 with this.
+__device__ __forceinline__ void ut_push(double x, double y, double rr, const UtConst &k,
+                                        double &u, double &t, const double *tab) {
+    ut_of(x, y, rr, k, u, t, tab);
+}
+__device__ __forceinline__ void ut_push(float x, float y, float rr, const UtConst &k, float &u,
+                                        float &t, const double *tab) {
+    const float v = 1.0f + rr;
+    const unsigned b = __float_as_uint(v);
+    // m in [1, 2), c = 1 + j/32 at or below it: m - c is exact in FP32
+    const float m = __uint_as_float((b & 0x7fffffu) | 0x3f800000u);
+    const float c = __uint_as_float((b & 0x7c0000u) | 0x3f800000u);
+    const int j = (int)((b >> 18) & 31u), e = (int)(b >> 23) - 127;
+    const double s = (double)(m - c) * rcp_46((double)m + (double)c);
+    const double z = s * s;
+    const double p = z * fma(z, fma(z, 1.0 / 7.0, 1.0 / 5.0), 1.0 / 3.0);
+    const double s2 = s + s;
+    const double l = fma((double)e, 0x1.62e42fefa39efp-1, tab[j]) + fma(s2, p, s2);
+    // the angle of the first octant, z = tan(atan(num/den) - atan(c))
+    const float ax = fabsf(x), ay = fabsf(y);
+    const bool swap = ay > ax;
+    const float num = swap ? ax : ay, den = swap ? ay : ax;
+    int i = (int)fmaf(num * __builtin_amdgcn_rcpf(den), 16.0f, 0.5f);
+    i = min(max(i, 0), 16);
+    const double ca = (double)((float)i * 0.0625f);
+    const double dn = (double)num, dd = (double)den;
+    const double w = fma(-ca, dd, dn) * rcp_46(fma(ca, dn, dd));
+    const double w2 = w * w;
+    const double q = w2 * fma(w2, fma(w2, fma(w2, 1.0 / 9.0, -1.0 / 7.0), 1.0 / 5.0), -1.0 / 3.0);
+    double a = tab[32 + i] + fma(w, q, w);
+    const bool nx = __float_as_int(x) < 0, ny = __float_as_int(y) < 0;
+    const double base = swap ? 0x1.921fb54442d18p+0 : nx ? 0x1.921fb54442d18p+1 : 0.0;
+    a = base + (swap != nx ? -a : a);
+    a = ny ? -a : a;
+    const double tt = a * k.tscale;
+    float lf = (float)l, tf = (float)tt;
+    const bool open = float_rounding_open(tt) || float_rounding_open(l) ||
+                      !(den >= 0x1p-100f && den < 0x1p100f);
+    if (any_lane(open)) {
+        asm volatile("");
+        if (open) {
+            lf = (float)gh_log_ge1((double)v);
+            tf = (float)(gh_atan2((double)y, (double)x) * k.tscale);
+        }
+    }
+    u = (float)((double)lf * k.inv_alpha);
+    t = tf < 0.0f ? tf + (float)k.na : tf;
 }
 
 // Cell and CIC weights from (u, t) (weight.f:84-95).  The reference's cell
@@ -380,6 +503,48 @@ __device__ __forceinline__ void deposit_global(long long *const *mfx, int nz,
     }
 }
 
+// ---- block-level results kept off shared addresses -----------------------------
+//
+// Every block of a particle kernel ends with a few one-word results: the ring
+// range of its deposits and its number of pushes.  Atomics of all blocks to
+// one address run one after another, about 5 ns each, which three of them per
+// block made the longest chain of a push (6e6 particles in 5860 blocks: 98 us with them, 82 us
+// without).
+// They go to stripes a cache line or more apart, by block, and are combined
+// where they are read.  (Reading the range first and skipping the atomic was
+// no faster: reads of one address past the caches queue just the same.)
+
+// The zones' ring ranges: jrad / krad of stripe s, member m and zone z at
+// s * rstride + m * GH_MAXZ + z - 1 (rstride a multiple of 32 ints).
+#define GH_RANGE_STRIPES 16
+__device__ __forceinline__ void widen_range(int *jrad, int *krad, int rstride, unsigned b, int z,
+                                            int j, int k) {
+    const int s = (int)(b & (GH_RANGE_STRIPES - 1)) * rstride + z - 1;
+    atomicMin(&jrad[s], j);
+    atomicMax(&krad[s], k);
+}
+// The combined ranges of nz zones into j[], k[] (LDS), by one wavefront, all
+// lanes active.
+__device__ __forceinline__ void combine_ranges(const int *jrad, const int *krad, int rstride,
+                                               int nz, int *j, int *k) {
+    const int lane = threadIdx.x & 63, s = (lane & (GH_RANGE_STRIPES - 1)) * rstride;
+    for (int z = 0; z < nz; z++) {
+        const int lo = wave_min_i32(jrad[s + z]), hi = wave_max_i32(krad[s + z]);
+        if (lane == 0) {
+            j[z] = lo;
+            k[z] = hi;
+        }
+    }
+}
+
+// Pushes are counted in GH_PUSH_STRIPES counters a cache line apart, by
+// block, and added when they are read.
+#define GH_PUSH_STRIPES 256
+__device__ __forceinline__ void count_pushes(long long *stripes, unsigned b, int n) {
+    if (n) atomicAdd((unsigned long long *)&stripes[8 * (b & (GH_PUSH_STRIPES - 1))],
+                     (unsigned long long)n);
+}
+
 // ---- kernel argument blocks -------------------------------------------------
 
 struct ZonePtrs {
@@ -398,8 +563,10 @@ template <typename R> struct PushArgs {
     long long n;
     const typename Vec2<R>::T *fld;   // [mesh] (F_x, F_y) after polcat
     long long *mfx[GH_MAXZ];          // zone mass sums, fixed point
-    int *jrad, *krad;                 // [nz] 1-based ring ranges
-    long long *counters;              // [0] off-grid delta, [1] pushes
+    int *jrad, *krad;                 // 1-based ring ranges (widen_range)
+    int rstride;
+    long long *counters;              // [0] off-grid count
+    long long *pushes;                // push counters (count_pushes)
     const double4 *fr_c;              // fixed force table (coefficients)
     double fr_inv_dr;
     int nfr, fixforce;
@@ -416,6 +583,7 @@ template <typename R> struct PushArgs {
     const int4 *blk;
     const int *qbits_m;
     int nblocks;
+    int ppt;                          // particles per thread (push_ppt)
     // compensated positions (FP32, opt-in): the low words of (x, y), or NULL
     typename Vec2<R>::T *xlo;
 };
@@ -438,7 +606,7 @@ template <typename R> struct AnaArgs {
     const long long *moz[GH_MAXZ];
     double fnew[GH_MAXZ], fold[GH_MAXZ];
     int use_new[GH_MAXZ], use_old[GH_MAXZ];
-    int *jrad, *krad;
+    int *jrad, *krad, rstride;
     int *ranges;                      // out: jrs, krs, jrf, krf
     R *rho;                           // [mesh]
     R *coef;                          // [ncoef][nr]
@@ -467,7 +635,7 @@ template <typename R> struct SynArgs {
     // zones 2..masscl_z saved, their jrad/krad reset (0 = none)
     long long *mfx[GH_MAXZ];
     long long *moz[GH_MAXZ];
-    int *jrad, *krad;
+    int *jrad, *krad, rstride;
     int masscl_z;
     int nmem;                         // grids (blockIdx.z); 1 for one grid
     const float *wpre;                // contraction done beforehand, or NULL

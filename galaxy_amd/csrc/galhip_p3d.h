@@ -14,8 +14,9 @@ template <typename R> struct P3Args {
     long long n;
     const typename Vec4<R>::T *fld;   // (F_x, F_y, F_z, potential) per cell
     long long *mfx[GH_MAXZ];
-    int *jrad, *krad;
-    long long *counters;              // [0] off-grid count, [1] pushes
+    int *jrad, *krad, rstride;
+    long long *counters;              // [0] off-grid count
+    long long *pushes;                // push counters (count_pushes)
     const double4 *fr_c;              // fixed force table (coefficients)
     double fr_inv_dr;
     int nfr, fixforce;
@@ -43,7 +44,7 @@ template <typename R> struct P3SolveArgs {
     const long long *moz[GH_MAXZ];
     double fnew[GH_MAXZ], fold[GH_MAXZ];
     int use_new[GH_MAXZ], use_old[GH_MAXZ];
-    int *jrad, *krad, *ranges;
+    int *jrad, *krad, rstride, *ranges;
     R *rho;          // [mesh] combined, scaled mass
     R *A;            // [nr][nm][ngz] azimuthal components per plane
     R *M;            // [nr][nm][2 ngz] after the vertical transform

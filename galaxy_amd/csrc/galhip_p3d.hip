@@ -58,6 +58,14 @@ __device__ __forceinline__ void ut3(R x, R y, const P3Args<R> &a, R &u, R &t) {
     if (!(rr > (R)0)) t = (R)0;
 }
 
+// ut3 in the push (ut_push); rr the position's cylindrical radius
+template <typename R>
+__device__ __forceinline__ void ut3_push(R x, R y, R rr, const P3Args<R> &a, R &u, R &t,
+                                         const double *tab) {
+    ut_push(x, y, rr, a.k, u, t, tab);
+    if (!(rr > (R)0)) t = (R)0;
+}
+
 // weight() for one position given its (u, t), p3d jmass = 2
 // (weight.f:219-248): returns the 0-based cell (ju ngz + jz) na + jt and the
 // 8 weights in the reference's order (bit 0 = dt, bit 1 = dz, bit 2 = du).
@@ -69,7 +77,7 @@ __device__ __forceinline__ int cell3(R u, R t, R z, const P3Args<R> &a, bool fol
     int ju = (int)u;
     if (ju > a.nr - 2) ju = a.nr - 2;
     int jt = (int)t;
-    zz = zz / a.dzg;
+    zz = div_rn(zz, a.dzg);
     int jz = (int)zz;
     if (jz < 0) jz = 0;
     if (jz > a.ngz - 2) jz = a.ngz - 2;
@@ -110,7 +118,7 @@ __device__ __forceinline__ int cell3q(R u, R t, R z, const P3Args<R> &a, bool fo
     if (ju > a.nr - 2) ju = a.nr - 2;
     if (ju < 1) ju = 1;
     const int jt = (int)(t + h);
-    zz = zz / a.dzg;
+    zz = div_rn(zz, a.dzg);
     int jz = (int)(zz + h);
     if (jz < 0) jz = 0;
     if (jz > a.ngz - 2) jz = a.ngz - 2;
@@ -250,10 +258,10 @@ __device__ __forceinline__ void getacc3(const P3Args<R> &a, R ox, R oy, R oz, R 
             r2 = r2 + ox * ox;
             r2 = r2 + oy * oy;
             r2 = r2 + oz * oz;
-            const R rr = sqrt(r2);
+            const R rr = sqrt_rn(r2);
             R fr = (R)fixforce((double)rr, a.nfr, a.fr_inv_dr, a.fr_c);
             if (fr != (R)0) {
-                fr = fr / rr;
+                fr = div_rn(fr, rr);
                 sx = sx + fr * ox;
                 sy = sy + fr * oy;
                 sz = sz + fr * oz;
@@ -469,12 +477,12 @@ __device__ __forceinline__ void deposit3_block(const P3Args<R> &a, bool on, int 
 // jrad/krad from the block's central rings: 1-based rings j+1..j+2 about a
 // central ring j (massgn.f:146-149), j..j+2 for jmass 3 (massgn.f:176-179)
 __device__ __forceinline__ void flush_ranges(int nz, int nr, int lo, const int *s_jr,
-                                             const int *s_kr, int *jrad, int *krad) {
+                                             const int *s_kr, int *jrad, int *krad,
+                                             int rstride) {
     const int tid = threadIdx.x;
     if (tid < nz && s_kr[tid] >= 0) {
-        atomicMin(&jrad[tid], s_jr[tid] + 1 - lo);
         const int k = s_kr[tid] + 2;
-        atomicMax(&krad[tid], k < nr ? k : nr);
+        widen_range(jrad, krad, rstride, blockIdx.x, tid + 1, s_jr[tid] + 1 - lo, k < nr ? k : nr);
     }
 }
 
@@ -507,7 +515,7 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_massgn_kernel(P3Args<R> a) {
     }
     deposit3_block<R, J>(a, on, z, c, rg, pl, sp, w, tile, s_b, s_ref, s_jr, s_kr);
     __syncthreads();
-    flush_ranges(a.nz, a.nr, J == 3 ? 1 : 0, s_jr, s_kr, a.jrad, a.krad);
+    flush_ranges(a.nz, a.nr, J == 3 ? 1 : 0, s_jr, s_kr, a.jrad, a.krad, a.rstride);
 }
 
 template <typename R, int J>
@@ -518,6 +526,7 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
     __shared__ unsigned long long s_ref[2];
     __shared__ int s_dn, s_np;
     __shared__ long long tile[P3_TILE];
+    __shared__ double s_tab[UtTab<R>::n];
     const int tid = threadIdx.x;
     if (tid < GH_MAXZ) {
         s_jr[tid] = INT_MAX;
@@ -527,6 +536,7 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
         s_dn = s_np = 0;
         s_b[0] = INT_MAX;
     }
+    if (tid < UtTab<R>::n) s_tab[tid] = ut_tab_entry<R>(tid);
     __syncthreads();
     const long long i = (long long)blockIdx.x * P3_PBLOCK + tid;
     int dn = 0, np = 0;
@@ -555,7 +565,8 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
                 nx[d] = o[d] + nv[d];
             }
             int znew = z0;
-            const R rnew = sqrt(nx[0] * nx[0] + nx[1] * nx[1]);
+            const R nx0 = nx[0], nx1 = nx[1];
+            R rnew = sqrt_rn(nx0 * nx0 + nx1 * nx1);
             const R az = nx[2] < (R)0 ? -nx[2] : nx[2];
             const bool off = (az > a.zm) || (rnew > a.rgrid);
             if (!offlist) {
@@ -585,7 +596,8 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
                 }
             }
             R un, tn;
-            ut3(nx[0], nx[1], a, un, tn);
+            if (nx0 != nx[0] || nx1 != nx[1]) rnew = sqrt_rn(nx[0] * nx[0] + nx[1] * nx[1]);
+            ut3_push(nx[0], nx[1], rnew, a, un, tn, s_tab);
             a.rec[2 * i] = mk4(nx[0], nx[1], nx[2], nv[0]);
             a.rec[2 * i + 1] = mk4(nv[1], nv[2], un, tn);
             a.zone[i] = (uint8_t)znew;
@@ -605,10 +617,10 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
         if (np) atomicAdd(&s_np, np);
     }
     __syncthreads();
-    flush_ranges(a.nz, a.nr, J == 3 ? 1 : 0, s_jr, s_kr, a.jrad, a.krad);
+    flush_ranges(a.nz, a.nr, J == 3 ? 1 : 0, s_jr, s_kr, a.jrad, a.krad, a.rstride);
     if (tid == 0) {
         if (s_dn) atomicAdd((unsigned long long *)&a.counters[0], (unsigned long long)(long long)s_dn);
-        if (s_np) atomicAdd((unsigned long long *)&a.counters[1], (unsigned long long)(long long)s_np);
+        count_pushes(a.pushes, blockIdx.x, s_np);
     }
 }
 
@@ -842,12 +854,13 @@ template <typename R>
 __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) {
     __shared__ R rho_s[P3_MAX_NA];
     __shared__ R tws[2 * P3_MAX_NA];
-    __shared__ int s_rng[4], s_ok;
+    __shared__ int s_rng[4], s_ok, s_jr[GH_MAXZ], s_kr[GH_MAXZ];
     const int tid = threadIdx.x, na = a.na;
     const int plane = blockIdx.x, ir = blockIdx.y + 1;
+    if (tid < 64) combine_ranges(a.jrad, a.krad, a.rstride, a.nz, s_jr, s_kr);
     if (tid == 0) {
         int kr[GH_MAXZ], rg[4] = {0, 0, 0, 0};
-        const bool ok = solve_ranges(a.jrad, a.krad, a.nz, a.nr, a.mzone, a.lpot,
+        const bool ok = solve_ranges(s_jr, s_kr, a.nz, a.nr, a.mzone, a.lpot,
                                      a.explicit_zones, a.jzone, a.kzone, kr, rg);
         s_ok = ok;
         for (int q = 0; q < 4; q++) s_rng[q] = rg[q];

@@ -137,14 +137,16 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
         rc |= dalloc(&c->mfx[z], sizeof(long long) * c->mesh);
         rc |= dalloc(&c->moz[z], sizeof(long long) * c->mesh);
     }
-    rc |= dalloc(&c->jrad, sizeof(int) * GH_MAXZ);
-    rc |= dalloc(&c->krad, sizeof(int) * GH_MAXZ);
+    c->rstride = range_stride(1);
+    rc |= dalloc(&c->jrad, sizeof(int) * range_ints(c));
+    rc |= dalloc(&c->krad, sizeof(int) * range_ints(c));
     rc |= dalloc(&c->ranges, sizeof(int) * 4);
     rc |= dalloc(&c->lg_d, sizeof(int) * c->mmax);
     rc |= dalloc(&c->slot_m_d, sizeof(int) * (nm > 0 ? nm : 1));
     rc |= dalloc(&c->slot_p_d, sizeof(int) * (nm > 0 ? nm : 1));
     rc |= dalloc(&c->slot_of_d, sizeof(int) * c->mmax);
     rc |= dalloc(&c->counters, sizeof(long long) * 4);
+    rc |= dalloc(&c->push_cnt, sizeof(long long) * 8 * GH_PUSH_STRIPES);
     rc |= dalloc(&c->rho, es * c->mesh);
     rc |= dalloc(&c->A3, es * c->nr * nm * c->ngz);
     rc |= dalloc(&c->M3, es * c->nr * nm * P);
@@ -187,10 +189,11 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
         HIPCHK(hipMemcpy(c->slot_p_d, slot_p.data(), sizeof(int) * nm, hipMemcpyHostToDevice));
     }
     HIPCHK(hipMemcpy(c->slot_of_d, slot_of.data(), sizeof(int) * c->mmax, hipMemcpyHostToDevice));
-    std::vector<int> jr(GH_MAXZ, c->nr), kr(GH_MAXZ, 0);
-    HIPCHK(hipMemcpy(c->jrad, jr.data(), sizeof(int) * GH_MAXZ, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->krad, kr.data(), sizeof(int) * GH_MAXZ, hipMemcpyHostToDevice));
+    std::vector<int> jr(range_ints(c), c->nr), kr(range_ints(c), 0);
+    HIPCHK(hipMemcpy(c->jrad, jr.data(), sizeof(int) * jr.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->krad, kr.data(), sizeof(int) * kr.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->counters, 0, sizeof(long long) * 4));
+    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     HIPCHK(hipMemset(c->fld4, 0, 4 * es * c->mesh));
     HIPCHK(hipMemset(c->rho, 0, es * c->mesh));
     // entries of W no contraction writes (e.g. F_z at k_z = 0) stay zero
@@ -307,6 +310,7 @@ extern "C" int galhip_restrt3(galhip_ctx *c, int64_t n, const void *x, const voi
         if (v == c->nz + 1) cnt[0]++;
     }
     HIPCHK(hipMemcpy(c->counters, cnt, sizeof cnt, hipMemcpyHostToDevice));
+    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     if (n > 0) {
         // the planar arrays through the second record buffer (free outside a
         // sort, 8 n values), interleaved on the device
@@ -415,7 +419,9 @@ template <typename R> static P3Args<R> p3_args(galhip_ctx *c) {
     for (int z = 0; z < c->nz; z++) a.mfx[z] = c->mfx[z];
     a.jrad = c->jrad;
     a.krad = c->krad;
+    a.rstride = c->rstride;
     a.counters = c->counters;
+    a.pushes = c->push_cnt;
     a.fr_c = c->fr_c;
     a.fr_inv_dr = c->nfr > 0 ? 1.0 / c->fr_dr : 0.0;
     a.nfr = c->nfr;
@@ -448,7 +454,7 @@ static P3SolveArgs<R> p3_solve_args(galhip_ctx *c, int lpot, int explicit_zones,
         a.use_new[z] = c->use_new[z];
         a.use_old[z] = c->use_old[z];
     }
-    a.jrad = c->jrad; a.krad = c->krad; a.ranges = c->ranges;
+    a.jrad = c->jrad; a.krad = c->krad; a.rstride = c->rstride; a.ranges = c->ranges;
     a.rho = (R *)c->rho; a.A = (R *)c->A3; a.M = (R *)c->M3; a.W = (R *)c->W3; a.Z = (R *)c->Z3;
     a.G = (const R *)c->G; a.tw = (const R *)c->tw; a.twz = (const R *)c->twz;
     a.lg = c->lg_d; a.slot_m = c->slot_m_d; a.slot_p = c->slot_p_d; a.slot_of = c->slot_of_d;
@@ -470,7 +476,7 @@ template <typename R> static int p3_masset_impl(galhip_ctx *c) {
     ZonePtrs zp;
     memset(&zp, 0, sizeof zp);
     for (int z = 0; z < c->nz; z++) { zp.mfx[z] = c->mfx[z]; zp.moz[z] = c->moz[z]; }
-    HIPCHK(launch_masscl(zp, c->nz, c->mesh, c->jrad, c->krad, c->nr, 1, c->s));
+    HIPCHK(launch_masscl(zp, c->nz, c->mesh, c->jrad, c->krad, c->rstride, c->nr, 1, c->s));
     HIPCHK(launch_p3_massgn<R>(p3_args<R>(c), c->s));
     int rc = zoncmb_host(c);
     if (rc) return rc;
@@ -503,7 +509,7 @@ template <typename R> static int p3_step_impl(galhip_ctx *c) {
     ZonePtrs zp;
     memset(&zp, 0, sizeof zp);
     for (int z = 0; z < c->nz; z++) { zp.mfx[z] = c->mfx[z]; zp.moz[z] = c->moz[z]; }
-    HIPCHK(launch_masscl(zp, c->mzone, c->mesh, c->jrad, c->krad, c->nr, 1, c->s));
+    HIPCHK(launch_masscl(zp, c->mzone, c->mesh, c->jrad, c->krad, c->rstride, c->nr, 1, c->s));
     c->masscl_done = 0;
     const P3Args<R> a = p3_args<R>(c);
     if (c->prof) HIPCHK(hipEventRecord(take_event(c), c->s));

@@ -23,51 +23,51 @@
 // commute, so the sums are bit-identical for any processing order and need
 // no float atomics.  Each block deposits into an LDS tile that covers the
 // rings x spokes window of its particles (particles are kept ordered by
-// cell, so the window is small), with TILE_REP copies chosen by lane so
-// that lanes hitting the same cell are spread over copies; the block then
-// flushes every non-zero tile cell with one 64-bit global atomic.  Blocks
-// whose window exceeds the tile, and deposits into another zone than the
-// tile's, go straight to global atomics.  Global 64-bit atomics are the
-// scarce resource on MI355X (about 24 G/s device-wide), LDS atomics far
-// less so.
+// cell, so the window is small) and flushes every non-zero tile cell with
+// one 64-bit global atomic.  Global 64-bit atomics are the scarce resource
+// on MI355X (about 24 G/s device-wide), LDS atomics far less so.
 #include "galhip_kern.h"
 #include <climits>
 
 namespace gh {
 
-// Launch shape (tuned on MI355X; see the DESIGN notes of the deposit):
-#ifndef GH_TILE_CAP
-#define GH_TILE_CAP 1024
-#endif
-#ifndef GH_TILE_REP
-#define GH_TILE_REP 2
-#endif
-
-constexpr int PPT = GH_PPT;            // particles per thread
 constexpr int PB = GH_PUSH_BLOCK;      // threads per block
-// minimum wavefronts per SIMD of push_kernel (launch bounds), FP32 and FP64
-#ifndef GH_PUSH_WAVES32
-#define GH_PUSH_WAVES32 6
-#endif
-#ifndef GH_PUSH_WAVES64
-#define GH_PUSH_WAVES64 4
-#endif
-constexpr int TILE_CAP = GH_TILE_CAP;  // LDS tile, cells of a ring x spoke window
-constexpr int TILE_REP = GH_TILE_REP;  // replicas (lane & (REP-1)) against conflicts
-constexpr int FF_CAP = 256;            // staged fixed-force table entries
-#ifndef GH_PUSH_PASSES
-#define GH_PUSH_PASSES 3               // deposit window passes before global atomics
-#endif
 
-// fields of a packed deposit cell (zone << 28 | ring << 16 | spoke)
-__device__ __forceinline__ int dc_zone(int c) { return (int)((unsigned)c >> 28); }
-__device__ __forceinline__ int dc_ring(int c) { return (c >> 16) & 0xFFF; }
-__device__ __forceinline__ int dc_spoke(int c) { return c & 0xFFFF; }
+// Launch shapes by particles per thread, measured (push time, us; FP32, 128
+// spokes | 512 spokes where two figures are given):
+//   particles       1 per thread     2            4
+//   5e4             13.1 | 26.4      16.0 | 34.1  22.0 | 45.4
+//   8e5             24.3 | 27.9      24.3 | 31.9  26.3 | 42.7
+//   2e6             45.6 | 47.9      43.7 | 44.7  44.3 | 45.7
+//   1e7, 3 zones    124              104          102
+// FP64, 3e6 in 3 zones: 55.8, 56.2, 60.6; 1e7: 169, -, 170.  A block's own latency is what a
+// small count waits for, and it grows with the particles per thread; a large
+// one pays for the window work of every block.  The tile: 3072 cells in one
+// copy against 1024 in two copies (lanes of one cell spread over them) takes
+// the ensemble's push from 171 to 143 us, 1e7 particles in 3 zones from 101.8
+// to 101.1 us (fewer second passes, the same LDS).  Wavefronts per SIMD: as
+// many as the registers allow without spills.
+template <typename R, bool COMP, int PPT> struct PushShape {
+    static constexpr int tile = PPT == 1 ? 2048 : 3072;
+    static constexpr int waves = sizeof(R) == 8 ? 8
+                                 : PPT == 1     ? 8
+                                                : (COMP ? 5 : 6);
+};
+constexpr int PUSH_PASSES = 8;         // deposit window passes before global atomics
+constexpr int CLIP_RINGS = 16;          // rings of a window that had to be clipped
 
+// step ratio of list iz: the first three by selection between uniform values
+// (an indexed read of the argument block is a load, and a load after the
+// particle stores waits for them)
 template <typename R>
 __device__ __forceinline__ R tsfac(const PushArgs<R> &a, int iz) {
-    int i = iz < a.nz ? iz : a.nz;
-    return (R)a.nstep[i - 1];
+    const int i = iz < a.nz ? iz : a.nz;
+    int n = i == 1 ? a.nstep[0] : i == 2 ? a.nstep[1] : a.nstep[2];
+    if (a.nz > 3) {
+        for (int q = 4; q <= a.nz; q++)
+            if (i == q) n = a.nstep[q - 1];
+    }
+    return (R)n;
 }
 
 // zoneno for a position of known radius (zoneno.f:40-55)
@@ -123,408 +123,103 @@ __device__ __forceinline__ int wave_min(int v) { return wave_min_i32(v); }
 __device__ __forceinline__ int wave_max(int v) { return wave_max_i32(v); }
 
 
-// ENS: an ensemble launch, the block's particles and member from a.blk.
-// COMP: compensated positions (a.xlo holds the low words).
-template <typename R, bool ENS, bool COMP>
-// Wavefronts per SIMD, measured: FP32 at least 6 (80 VGPRs at most; faster
-// than 5 waves at 86 VGPRs; the LDS of six blocks per CU just fits); FP64
-// at least 4 (128 VGPRs, a few spills, 4 % faster than 3 waves without).
-__global__ __launch_bounds__(PB, sizeof(R) == 4 ? GH_PUSH_WAVES32 : GH_PUSH_WAVES64) void push_kernel(PushArgs<R> a) {
-    typedef typename Vec2<R>::T R2;
-    typedef typename Vec4<R>::T R4;
-    __shared__ long long tile[TILE_REP][TILE_CAP];
-    __shared__ int s_jr[GH_MAXZ], s_kr[GH_MAXZ];
-    __shared__ int s_dnoff, s_pushes;
-    __shared__ int s_box[8];                 // two (ring min, max, offset min, max) boxes
-    __shared__ unsigned long long s_ref[2];  // two deposit-pass reference keys
-    __shared__ int s_fref, s_frmin, s_frmax, s_fdmin, s_fdmax, s_kmin, s_kmax;
-    // slice of the fixed-force table that the block's radii use
-    __shared__ double4 s_ffc[FF_CAP];
-    // the logarithm and arc-tangent tables, read per particle by ut_of
-    __shared__ double s_tab[GH_MATH_TAB_N];
+// Hides a value's origin from the optimiser (no instruction is issued).
+__device__ __forceinline__ void opaque(float2 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
+__device__ __forceinline__ void opaque(double2 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    // the block's particles and its grid (ensembles: member eb.x)
-    const int4 eb = ENS ? a.blk[blockIdx.x] : make_int4(0, 0, 0, 0);
-    const long long base = ENS ? (long long)eb.y : (long long)blockIdx.x * (PB * PPT);
-    const long long mo = ENS ? (long long)eb.x * a.mesh : 0;
-    const R2 *const fld = a.fld + mo;
-    int *const jrad = a.jrad + (ENS ? eb.x * GH_MAXZ : 0);
-    int *const krad = a.krad + (ENS ? eb.x * GH_MAXZ : 0);
-    long long *const counters = a.counters + (ENS ? eb.x * 4 : 0);
-    const int qbits = ENS ? a.qbits_m[eb.x] : a.qbits;
-    const int nz = a.nz, nlists = a.nz + 1, na = a.na, nr = a.nr;
-    for (int j = tid; j < GH_MATH_TAB_N; j += PB) s_tab[j] = GH_MATH_TAB[j];
-    const double *const mtab = s_tab;
+// LDS of a block's deposit.
+template <int TILE> struct DepositLds {
+    long long tile[TILE];
+    int jr[GH_MAXZ], kr[GH_MAXZ];    // ring ranges by zone
+    int box[8];                      // two (ring min, max, offset min, max) boxes
+    unsigned long long ref[2];       // two reference keys
+};
+
+// Set up before the block's first barrier.
+template <int TILE> __device__ __forceinline__ void deposit_init(DepositLds<TILE> &s) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < TILE; j += PB) s.tile[j + tid] = 0;
     if (tid < GH_MAXZ) {
-        s_jr[tid] = INT_MAX;
-        s_kr[tid] = -1;
+        s.jr[tid] = INT_MAX;
+        s.kr[tid] = -1;
     }
     if (tid == 0) {
-        s_dnoff = 0;
-        s_pushes = 0;
-        s_box[0] = s_box[4] = INT_MAX;
-        s_box[1] = s_box[5] = -1;
-        s_box[2] = s_box[6] = INT_MAX;
-        s_box[3] = s_box[7] = INT_MIN;
-        s_ref[0] = s_ref[1] = ~0ull;
-        s_frmin = INT_MAX;
-        s_frmax = -1;
-        s_fdmin = INT_MAX;
-        s_fdmax = INT_MIN;
-        s_kmin = INT_MAX;
-        s_kmax = -1;
+        s.box[0] = s.box[4] = INT_MAX;
+        s.box[1] = s.box[5] = -1;
+        s.box[2] = s.box[6] = INT_MAX;
+        s.box[3] = s.box[7] = INT_MIN;
+        s.ref[0] = s.ref[1] = ~0ull;
     }
+}
 
-    // the block's particles through block-based pointers and 32-bit
-    // offsets (uniform base, per-lane offset: no 64-bit address arithmetic)
-    R4 *const xvb = a.xv + base;
-    R2 *const utb = a.ut + base;
-    R2 *const lob = COMP ? a.xlo + base : nullptr;
-    uint8_t *const zb = a.zone + base;
-    const int nblk = ENS ? eb.z : (int)min((long long)(PB * PPT), a.n - base);
-    int zin[PPT];
-    bool mv[PPT];
-    int any = 0;
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        const int j = k * PB + tid;
-        zin[k] = j < nblk ? (int)zb[j] : 0;
-        bool off = zin[k] == nlists;
-        mv[k] = zin[k] > 0 &&
-                (off ? (a.offanal && a.mzone == nz) : (zin[k] <= a.mzone));
-        any |= mv[k];
-    }
-    // every thread reaches this barrier; a block with nothing to move exits
-    if (!__syncthreads_or(any)) return;
+// The reference of the first deposit window: the block's middle particle.
+struct PushRef {
+    int zone, ring, spoke;
+};
+template <typename R2> __device__ __forceinline__ PushRef push_ref(R2 ut, int zone, int nz, int nr, int na) {
+    PushRef r;
+    r.zone = min(max(zone, 1), nz);
+    r.ring = min(max((int)ut.x, 0), nr - 2);
+    r.spoke = min(max((int)ut.y, 0), na - 1);
+    return r;
+}
 
-    // The loads of all PPT particles are issued before any is consumed:
-    // state and (u, t) first, then the 4 x PPT field gathers, then the
-    // fixed-force table reads.  These phases are straight-line code (indices
-    // clamped, results selected), so each phase's reads are in flight
-    // together instead of one particle's latency chain after another's.
-    R4 st[PPT];
-    R2 cu[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        const int j = min(k * PB + tid, nblk - 1);
-        st[k] = xvb[j];
-        cu[k] = utb[j];
-    }
-    // grdacc: weights of the old position from its (u, t) (off-grid and
-    // idle particles weigh nothing), the field read from an LDS copy of the
-    // window of rings x spokes that the block's old cells span -- the same
-    // windowing as the deposit tile below, whose LDS it borrows.  A window
-    // larger than that space falls back to reads from global memory.
-    const int half = na >> 1;
-    int gring[PPT], gspoke[PPT], gd[PPT];
-    R gw[PPT][4];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        const bool grid = mv[k] && zin[k] != nlists;
-        cic(grid ? cu[k].x : (R)0, grid ? cu[k].y : (R)0, nr, na, gring[k],
-            gspoke[k], gw[k]);
-        if (!grid) gring[k] = -1;
-    }
-    R rr[PPT], fr[PPT];
-    int kf[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        rr[k] = sqrt(st[k].x * st[k].x + st[k].y * st[k].y);
-        fr[k] = 0;
-        kf[k] = a.fixforce ? fixforce_index((double)rr[k], a.nfr, a.fr_inv_dr) : 0;
-    }
-    if (tid == 0) {
-        int r = 0;
-#pragma unroll
-        for (int k = PPT - 1; k >= 0; k--)
-            if (gring[k] >= 0) r = gspoke[k];
-        s_fref = r;
-    }
-    __syncthreads();
-    const int fref = s_fref;
-    {
-        int rmin = INT_MAX, rmax = -1, dmin = INT_MAX, dmax = INT_MIN;
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            int d = gspoke[k] - fref;
-            if (d < -half) d += na;
-            else if (d >= half) d -= na;
-            gd[k] = d;
-            if (gring[k] >= 0) {
-                rmin = min(rmin, gring[k]);
-                rmax = max(rmax, gring[k]);
-                dmin = min(dmin, d);
-                dmax = max(dmax, d);
-            }
-        }
-        int kmin = INT_MAX, kmax = -1;
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-            if (gring[k] >= 0) {
-                kmin = min(kmin, kf[k]);
-                kmax = max(kmax, kf[k]);
-            }
-        rmin = wave_min(rmin);
-        rmax = wave_max(rmax);
-        dmin = wave_min(dmin);
-        dmax = wave_max(dmax);
-        kmin = wave_min(kmin);
-        kmax = wave_max(kmax);
-        if (lane == 0 && rmax >= 0) {
-            atomicMin(&s_frmin, rmin);
-            atomicMax(&s_frmax, rmax);
-            atomicMin(&s_fdmin, dmin);
-            atomicMax(&s_fdmax, dmax);
-            atomicMin(&s_kmin, kmin);
-            atomicMax(&s_kmax, kmax);
-        }
-    }
-    __syncthreads();
-    R2 *ftile = reinterpret_cast<R2 *>(&tile[0][0]);
-    constexpr int FT_CAP = (int)(sizeof(tile) / sizeof(R2));
-    const int fr0 = s_frmin, fr1 = s_frmax, fd0 = s_fdmin, fd1 = s_fdmax;
-    const int ftw = fd1 - fd0 + 2, fth = fr1 - fr0 + 2;
-    const bool use_ft = fr1 >= 0 && fth * ftw <= FT_CAP;
-    if (use_ft) {
-        // rows past the last ring read as zero, as the global path does
-        // (row, col) of element j advanced incrementally: one division per
-        // thread instead of one per element
-        const int drow = PB / ftw, dcol = PB - drow * ftw;
-        int row = tid / ftw, col = tid - row * ftw;
-        for (int j = tid; j < fth * ftw; j += PB) {
-            const int ring = fr0 + row;
-            int spoke = fref + fd0 + col;
-            row += drow;
-            col += dcol;
-            if (col >= ftw) {
-                col -= ftw;
-                row++;
-            }
-            if (spoke < 0) spoke += na;
-            else if (spoke >= na) spoke -= na;
-            if (spoke >= na) spoke -= na;
-            ftile[j] = ring < nr ? fld[ring * na + spoke] : zero2<R>();
-        }
-    }
-    // the table intervals k0 .. k1 that the block's grid particles read
-    const int k0 = s_kmin, nk = s_kmax + 1 - s_kmin;
-    const bool use_ff = a.fixforce && s_kmax >= 0 && nk <= FF_CAP;
-    if (use_ff)
-        for (int j = tid; j < nk; j += PB) s_ffc[j] = a.fr_c[k0 + j];
-    __syncthreads();
-    R ax[PPT], ay[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        const bool grid = gring[k] >= 0;
-        R sx = 0, sy = 0;
-        if (use_ft) {
-            const int b = grid ? (gring[k] - fr0) * ftw + (gd[k] - fd0) : 0;
-            const int ti[4] = {b, b + 1, b + ftw, b + ftw + 1};
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const R2 f = ftile[ti[q]];
-                const R wq = grid ? gw[k][q] : (R)0;
-                sx = sx + f.x * wq;
-                sy = sy + f.y * wq;
-            }
-        } else {
-            int ic[4];
-            corners_rs(grid ? gring[k] : 0, gspoke[k], na, ic);
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                // the last ring with t == na points past the field: 0
-                const bool in = ic[q] < a.mesh;
-                R2 f = fld[in ? ic[q] : 0];
-                R wq = (grid && in) ? gw[k][q] : (R)0;
-                sx = sx + f.x * wq;
-                sy = sy + f.y * wq;
-            }
-        }
-        ax[k] = sx;
-        ay[k] = sy;
-    }
-    if (use_ff) {
-        // the staged slice; particles off the grid or idle (their force is
-        // not used) read its first interval
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            const bool grid = gring[k] >= 0;
-            fr[k] = (R)fixforce_at((double)rr[k], grid ? kf[k] : k0, a.nfr, a.fr_inv_dr,
-                                   s_ffc, k0);
-        }
-    } else if (a.fixforce) {
-#pragma unroll
-        for (int k = 0; k < PPT; k++)
-            fr[k] = (R)fixforce_at((double)rr[k], kf[k], a.nfr, a.fr_inv_dr, a.fr_c, 0);
-    }
-
-    // FP32: the states of particles 1 .. PPT-1 read once more (L2 hits):
-    // held in registers across the gathers above, one of them would be
-    // spilled to scratch at 6 wavefronts per SIMD, a store and a reload
-    // through memory (FP64 keeps them: the re-read spills more there)
-    if constexpr (sizeof(R) == 4) {
-#pragma unroll
-        for (int k = 1; k < PPT; k++) st[k] = xvb[min(k * PB + tid, nblk - 1)];
-    }
-
-    // deposit state kept per particle: ring, spoke, zone (0 = none), weights
-    // dcell: zone << 28 | ring << 16 | spoke (zone 0: no deposit)
-    int dcell[PPT];
-    R dw[PPT][4];
-    // off-grid list changes: +1 leaving the grid, -1 returning
-    bool dn_plus[PPT], dn_minus[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) {
-        dcell[k] = 0;
-        dn_plus[k] = false;
-        dn_minus[k] = false;
-        if (mv[k]) {
-            const int j = k * PB + tid;
-            const int z0 = zin[k];
-            const bool offlist = z0 == nlists;
-            R ox = st[k].x, oy = st[k].y, ovx = st[k].z, ovy = st[k].w;
-            R ax_ = ax[k], ay_ = ay[k];
-            if (!offlist && fr[k] != (R)0) {
-                R f = fr[k] / rr[k];
-                ax_ = ax_ + f * ox;
-                ay_ = ay_ + f * oy;
-            }
-            if (nz > 1 && z0 > 1) {
-                R t = tsfac(a, z0);
-                t = t * t;
-                ax_ = t * ax_;
-                ay_ = t * ay_;
-            }
-            R nvx = ovx + ax_, nvy = ovy + ay_;
-            R nx = ox + nvx, ny = oy + nvy;
-            R2 lo = zero2<R>(), elo = zero2<R>();
-            if (COMP) {
-                lo = lob[j];
-                nx = comp_add(ox, nvx, lo.x, elo.x);
-                ny = comp_add(oy, nvy, lo.y, elo.y);
-            }
-            int znew = z0;
-            R rnew = sqrt(nx * nx + ny * ny);
-            bool off = rnew > a.rgrid;
-            if (!offlist) {
-                if (off) {
-                    znew = nlists;
-                    dn_plus[k] = true;
-                    if (a.offanal && z0 < nz) {
-                        R tfac = tsfac(a, nz) / tsfac(a, z0);
-                        chstep(tfac, ox, oy, ovx, ovy, ax_, ay_, nx, ny, nvx, nvy);
-                        if (COMP) {
-                            nx = comp_add(ox, nvx, lo.x, elo.x);
-                            ny = comp_add(oy, nvy, lo.y, elo.y);
-                        }
-                        rnew = sqrt(nx * nx + ny * ny);
-                    }
-                }
-            } else if (!off) {
-                dn_minus[k] = true;
-                znew = nz;
-            }
-            if (a.mzone > 1 && !offlist && znew <= a.mzone) {
-                int kz = zone_of(a, rnew);
-                if (kz > a.mzone) kz = a.mzone;
-                if (kz > znew) kz = zone_of(a, rr[k]);
-                if (kz != znew) {
-                    R tfac = tsfac(a, kz) / tsfac(a, znew);
-                    chstep(tfac, ox, oy, ovx, ovy, ax_, ay_, nx, ny, nvx, nvy);
-                    if (COMP) {
-                        nx = comp_add(ox, nvx, lo.x, elo.x);
-                        ny = comp_add(oy, nvy, lo.y, elo.y);
-                    }
-                    rnew = sqrt(nx * nx + ny * ny);
-                    znew = kz;
-                }
-            }
-            xvb[j] = mk4(nx, ny, nvx, nvy);
-            if (COMP) lob[j] = elo;
-            if (znew != z0) zb[j] = (uint8_t)znew;
-            if (znew >= 1 && znew <= nz) {
-                R u, t;
-                ut_of(nx, ny, rnew, a.k, u, t, mtab);
-                utb[j] = mk2(u, t);
-                R tf = a.nsect > 1 ? (R)fmod(t, a.thmax) : t;
-                int ring, spoke;
-                cic(u, tf, nr, na, ring, spoke, dw[k]);
-                dcell[k] = (int)(((unsigned)znew << 28) | ((unsigned)ring << 16) | (unsigned)spoke);
-            }
-        }
-    }
-    // the wave's pushes and off-grid change by ballots (scalar counts),
-    // added to the block's counters by one lane
-    {
-        int wp = 0, wd = 0;
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            wp += __popcll(__ballot(mv[k]));
-            wd += __popcll(__ballot(dn_plus[k])) - __popcll(__ballot(dn_minus[k]));
-        }
-        if (lane == 0) {
-            if (wp) atomicAdd(&s_pushes, wp);
-            if (wd) atomicAdd(&s_dnoff, wd);
-        }
-    }
-    // Deposit passes.  A pass takes a reference deposit -- the pending one
-    // first in particle order from the block's middle particle -- and the
-    // box of the pending deposits of the reference's zone (rings x spoke
-    // offsets from the reference spoke, which wrap around the ring); a box
-    // over TILE_CAP cells is clipped about the reference, which therefore
-    // always fits.  The deposits inside go to the LDS tile, which is then
-    // flushed with one global atomic per touched cell.  What the clip or a
-    // second zone leaves pending gets the next pass; after PUSH_PASSES
-    // passes (and for a cell on the last ring) the corners go to global
-    // atomics directly.
-    bool pend[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; k++) pend[k] = dcell[k] != 0 && dc_ring(dcell[k]) + 1 < nr;
-    // this thread's reference candidate: the lowest rotated particle index
-    // among its pending deposits; the wave's lowest goes to s_ref[slot]
-    auto offer_ref = [&](int slot) {
-        int myrot = INT_MAX, mypack = 0;
-#pragma unroll
-        for (int k = 0; k < PPT; k++) {
-            const int rot = (k * PB + tid - PB * PPT / 2) & (PB * PPT - 1);
-            if (pend[k] && rot < myrot) {
-                myrot = rot;
-                mypack = dcell[k];
-            }
-        }
-        const int wmin = wave_min(myrot);
-        if (wmin != INT_MAX) {
-            const unsigned long long bal = __ballot(myrot == wmin);
-            const int fl = __ffsll((long long)bal) - 1;
-            const int pk = __builtin_amdgcn_readlane(mypack, fl);
-            if (lane == 0)
-                atomicMin(&s_ref[slot], ((unsigned long long)(unsigned)wmin << 32) | (unsigned)pk);
+// The block's deposits (massgn.f:68-89).  A pass takes a zone, a reference cell and the box of
+// the zone's pending deposits (rings x spoke offsets from the reference
+// spoke, which wrap around the ring); a box over TILE cells is
+// clipped about the reference.  The deposits inside go to the LDS tile,
+// which is then flushed with one global atomic per touched cell and
+// cleared.  What the clip or a second zone leaves pending gets the next
+// pass.  The first pass's reference is the block's middle particle, a
+// later one's the pending deposit first in particle order from there
+// (always inside its own window); after PUSH_PASSES passes (and for a
+// cell on the last ring) the corners go to global atomics directly.
+// cu: (u, t) of the thread's particles, t folded into the sector; dzone: their
+// zones, four bits each (0: no deposit).  Every thread of the block calls it.
+template <typename R, int PPT, int TILE>
+__device__ __forceinline__ void deposit_block(const PushArgs<R> &a, DepositLds<TILE> &s,
+                                              typename Vec2<R>::T (&cu)[PPT], unsigned dzone,
+                                              PushRef ref, int qbits, long long mo) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int na = a.na, nr = a.nr, nz = a.nz, half = na >> 1;
+    auto cell_of = [&](int k, int &ring, int &spoke) {
+        ring = min((int)cu[k].x, nr - 2);
+        spoke = (int)cu[k].y;
+        if (spoke >= na) {
+            ring++;
+            spoke -= na;
         }
     };
-    offer_ref(0);
-    __syncthreads();
+    unsigned pend = 0;
 #pragma unroll
-    for (int pass = 0; pass < GH_PUSH_PASSES; pass++) {
-        const unsigned long long kref = s_ref[pass & 1];
-        if (kref == ~0ull) break;                  // nothing pending (uniform)
-        const int zt = (int)((kref >> 28) & 0xF), rref = (int)((kref >> 16) & 0xFFF);
-        const int sref = (int)(kref & 0xFFFF);
-        int *const bx = s_box + 4 * (pass & 1);
-        if (tid == 0) s_ref[(pass + 1) & 1] = ~0ull;   // last read in the previous pass
-        // ring and spoke-offset box of the zone's pending deposits; dd: the
-        // deposits' spoke offsets from the reference spoke
-        int dd[PPT];
+    for (int k = 0; k < PPT; k++) {
+        int ring, spoke;
+        cell_of(k, ring, spoke);
+        if ((dzone >> (4 * k) & 15u) && ring + 1 < nr) pend |= 1u << k;
+    }
+    // pending deposits of zone z
+    auto in_zone = [&](int k, int z) {
+        return (pend >> k & 1u) && (int)(dzone >> (4 * k) & 15u) == z;
+    };
+#pragma unroll 1
+    for (int pass = 0;; pass++) {
+        int *const bx = s.box + 4 * (pass & 1);
+        // cells and weights are formed again from (u, t) in every pass: kept
+        // across the passes they would not fit the registers
+#pragma unroll
+        for (int k = 0; k < PPT; k++) opaque(cu[k]);
+        // ring and spoke-offset box of the zone's pending deposits
         {
             int rmin = INT_MAX, rmax = -1, dmin = INT_MAX, dmax = INT_MIN;
 #pragma unroll
             for (int k = 0; k < PPT; k++) {
-                int d = dc_spoke(dcell[k]) - sref;
+                int ring, d;
+                cell_of(k, ring, d);
+                d -= ref.spoke;
                 if (d < -half) d += na;
                 else if (d >= half) d -= na;
-                dd[k] = d;
-                if (pend[k] && dc_zone(dcell[k]) == zt) {
-                    const int ring = dc_ring(dcell[k]);
+                if (in_zone(k, ref.zone)) {
                     rmin = min(rmin, ring);
                     rmax = max(rmax, ring);
                     dmin = min(dmin, d);
@@ -543,156 +238,409 @@ __global__ __launch_bounds__(PB, sizeof(R) == 4 ? GH_PUSH_WAVES32 : GH_PUSH_WAVE
             }
         }
         __syncthreads();
-        // tile: rings [r0, r0 + th) x spoke offsets [d0, d0 + tw) of zone zt
+        // tile: rings [r0, r0 + th) x spoke offsets [d0, d0 + tw)
         int r0 = bx[0], th = bx[1] - bx[0] + 2, d0 = bx[2], tw = bx[3] - bx[2] + 2;
+        const bool some = bx[1] >= 0;
         if (tid == 0) {
-            atomicMin(&s_jr[zt - 1], bx[0]);
-            atomicMax(&s_kr[zt - 1], bx[1]);
-            int *const nb = s_box + 4 * ((pass + 1) & 1);   // last read in the previous pass
+            if (some) {
+                atomicMin(&s.jr[ref.zone - 1], bx[0]);
+                atomicMax(&s.kr[ref.zone - 1], bx[1]);
+            }
+            // the other box and key were last read before this barrier
+            int *const nb = s.box + 4 * ((pass + 1) & 1);
             nb[0] = INT_MAX;
             nb[1] = -1;
             nb[2] = INT_MAX;
             nb[3] = INT_MIN;
+            s.ref[(pass + 1) & 1] = ~0ull;
         }
-        if (th * tw > TILE_CAP) {
-            if (th > 8) {
-                r0 = min(max(rref - 3, r0), r0 + th - 8);
-                th = 8;
+        if (some && th * tw > TILE) {
+            if (th > CLIP_RINGS) {
+                r0 = min(max(ref.ring - (CLIP_RINGS / 2 - 1), r0), r0 + th - CLIP_RINGS);
+                th = CLIP_RINGS;
             }
-            const int mw = TILE_CAP / th;
+            const int mw = TILE / th;
             if (tw > mw) {
                 d0 = min(max(-((mw - 2) >> 1), d0), d0 + tw - mw);
                 tw = mw;
             }
         }
-        const int tlen = th * tw;
-        for (int j = tid; j < tlen; j += PB) {
-#pragma unroll
-            for (int rep = 0; rep < TILE_REP; rep++) tile[rep][j] = 0;
-        }
-        __syncthreads();
-        long long *trep = tile[lane & (TILE_REP - 1)];
+        const int tlen = some ? th * tw : 0;
 #pragma unroll
         for (int k = 0; k < PPT; k++) {
-            const int ring = dc_ring(dcell[k]), d = dd[k];
-            if (!pend[k] || dc_zone(dcell[k]) != zt || ring < r0 || ring - r0 + 1 >= th ||
-                d < d0 || d - d0 + 1 >= tw)
+            R w[4];
+            int ring, d;
+            cic(cu[k].x, cu[k].y, nr, na, ring, d, w);
+            d -= ref.spoke;
+            if (d < -half) d += na;
+            else if (d >= half) d -= na;
+            if (!in_zone(k, ref.zone) || ring < r0 || ring - r0 + 1 >= th || d < d0 ||
+                d - d0 + 1 >= tw)
                 continue;
             long long qv[4];
-            quant_n<R, 4>(dw[k], qbits, true, qv);
+            quant_n<R, 4>(w, qbits, true, qv);
             const int b = (ring - r0) * tw + (d - d0);
             const int ti[4] = {b, b + 1, b + tw, b + tw + 1};
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                if (qv[q] != 0)
-                    atomicAdd((unsigned long long *)&trep[ti[q]], (unsigned long long)qv[q]);
-            pend[k] = false;
+                atomicAdd((unsigned long long *)&s.tile[ti[q]], (unsigned long long)qv[q]);
+            pend &= ~(1u << k);
         }
-        const bool last = pass + 1 >= GH_PUSH_PASSES;
-        if (!last) offer_ref((pass + 1) & 1);
+        // the next pass's reference: the lowest particle index, counted from
+        // the block's middle, among the pending deposits
+        if (any_lane(pend != 0)) {
+            int myrot = INT_MAX, mypack = 0;
+#pragma unroll
+            for (int k = 0; k < PPT; k++) {
+                const int rot = (k * PB + tid - PB * PPT / 2) & (PB * PPT - 1);
+                int ring, spoke;
+                cell_of(k, ring, spoke);
+                if ((pend >> k & 1u) && rot < myrot) {
+                    myrot = rot;
+                    mypack = (int)((dzone >> (4 * k) << 28) | ((unsigned)ring << 16) |
+                                   (unsigned)spoke);
+                }
+            }
+            const int wmin = wave_min(myrot);
+            const int fl = __ffsll((long long)__ballot(myrot == wmin)) - 1;
+            const int pk = __builtin_amdgcn_readlane(mypack, fl);
+            if (lane == 0)
+                atomicMin(&s.ref[pass & 1], ((unsigned long long)(unsigned)wmin << 32) | (unsigned)pk);
+        }
         __syncthreads();
         // flush: one global atomic per touched cell, the tile's cells over
         // all threads in storage order (a row's cells are consecutive
-        // spokes, so a wave's atomics coalesce)
-        for (int j = tid; j < tlen; j += PB) {
-            long long v = 0;
-#pragma unroll
-            for (int rep = 0; rep < TILE_REP; rep++) v += tile[rep][j];
-            if (v != 0) {
-                const int row = div_small(j, tw), col = j - row * tw;
-                int spoke = sref + d0 + col;
-                if (spoke < 0) spoke += na;
-                else if (spoke >= na) spoke -= na;
-                if (spoke >= na) spoke -= na;
-                atomicAdd((unsigned long long *)&a.mfx[zt - 1][mo + (r0 + row) * na + spoke],
-                          (unsigned long long)v);
+        // spokes, so a wave's atomics coalesce); (row, col) advanced by the
+        // block size with a carry
+        if (tid < tlen) {
+            const int drow = div_small(PB, tw), dcol = PB - drow * tw;
+            int row = div_small(tid, tw), col = tid - row * tw;
+            for (int j = tid; j < tlen; j += PB) {
+                const long long v = s.tile[j];
+                if (v != 0) {
+                    s.tile[j] = 0;
+                    int spoke = ref.spoke + d0 + col;
+                    if (spoke < 0) spoke += na;
+                    else if (spoke >= na) spoke -= na;
+                    if (spoke >= na) spoke -= na;
+                    atomicAdd((unsigned long long *)&a.mfx[ref.zone - 1][mo + (r0 + row) * na + spoke],
+                              (unsigned long long)v);
+                }
+                row += drow;
+                col += dcol;
+                if (col >= tw) {
+                    col -= tw;
+                    row++;
+                }
             }
         }
-        if (last) break;
+        const unsigned long long kref = s.ref[pass & 1];
+        if (kref == ~0ull || pass + 1 >= PUSH_PASSES) break;   // uniform
+        ref.zone = (int)((kref >> 28) & 0xF);
+        ref.ring = (int)((kref >> 16) & 0xFFF);
+        ref.spoke = (int)(kref & 0xFFFF);
     }
     // what no pass took (and cells on the last ring): global atomics
 #pragma unroll
     for (int k = 0; k < PPT; k++) {
-        const int z = dc_zone(dcell[k]), ring = dc_ring(dcell[k]);
-        if (z == 0 || (ring + 1 < nr && !pend[k])) continue;
+        const int z = (int)(dzone >> (4 * k) & 15u);
+        R w[4];
+        int ring, spoke;
+        cic(cu[k].x, cu[k].y, nr, na, ring, spoke, w);
+        if (z == 0 || (ring + 1 < nr && !(pend >> k & 1u))) continue;
         long long qv[4];
-        quant_n<R, 4>(dw[k], qbits, true, qv);
-        atomicMin(&s_jr[z - 1], ring);
-        atomicMax(&s_kr[z - 1], ring);
+        quant_n<R, 4>(w, qbits, true, qv);
+        atomicMin(&s.jr[z - 1], ring);
+        atomicMax(&s.kr[z - 1], ring);
         int ic[4];
-        corners_rs(ring, dc_spoke(dcell[k]), na, ic);
+        corners_rs(ring, spoke, na, ic);
 #pragma unroll
         for (int q = 0; q < 4; q++)
             if (qv[q] != 0) deposit_global(a.mfx, nz, a.mesh, z, ic[q], qv[q], mo);
     }
-    __syncthreads();
-    if (tid < nz && s_kr[tid] >= 0) {
-        atomicMin(&jrad[tid], s_jr[tid] + 1);
-        int k = s_kr[tid] + 2;
-        atomicMax(&krad[tid], k < nr ? k : nr);
+}
+
+// The block's ring ranges join the grid's (after a barrier).
+template <int TILE>
+__device__ __forceinline__ void deposit_ranges(const DepositLds<TILE> &s, int nz, int nr, int *jrad,
+                                               int *krad, int rstride) {
+    const int tid = threadIdx.x;
+    if (tid < nz && s.kr[tid] >= 0) {
+        const int k = s.kr[tid] + 2;
+        widen_range(jrad, krad, rstride, blockIdx.x, tid + 1, s.jr[tid] + 1, k < nr ? k : nr);
     }
+}
+
+// ENS: an ensemble launch, the block's particles and member from a.blk.
+// COMP: compensated positions (a.xlo holds the low words).
+// PPT: particles per thread (see push_ppt).
+template <typename R, bool ENS, bool COMP, int PPT>
+__global__ __launch_bounds__(PB, (PushShape<R, COMP, PPT>::waves)) void push_kernel(PushArgs<R> a) {
+    typedef typename Vec2<R>::T R2;
+    typedef typename Vec4<R>::T R4;
+    __shared__ DepositLds<PushShape<R, COMP, PPT>::tile> s_dep;
+    __shared__ int s_dnoff, s_pushes;
+    // the logarithm and arc-tangent tables, read per particle by ut_push
+    __shared__ double s_tab[UtTab<R>::n];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    // the block's particles and its grid (ensembles: member eb.x)
+    const int4 eb = ENS ? a.blk[blockIdx.x] : make_int4(0, 0, 0, 0);
+    const long long base = ENS ? (long long)eb.y : (long long)blockIdx.x * (PB * PPT);
+    const long long mo = ENS ? (long long)eb.x * a.mesh : 0;
+    const R2 *const fld = a.fld + mo;
+    int *const jrad = a.jrad + (ENS ? eb.x * GH_MAXZ : 0);
+    int *const krad = a.krad + (ENS ? eb.x * GH_MAXZ : 0);
+    long long *const counters = a.counters + (ENS ? eb.x * 4 : 0);
+    const int qbits = ENS ? a.qbits_m[eb.x] : a.qbits;
+    const int nz = a.nz, nlists = a.nz + 1, na = a.na, nr = a.nr;
+    // the block's particles through block-based pointers and 32-bit
+    // offsets (uniform base, per-lane offset: no 64-bit address arithmetic)
+    R4 *const xvb = a.xv + base;
+    R2 *const utb = a.ut + base;
+    R2 *const lob = COMP ? a.xlo + base : nullptr;
+    uint8_t *const zb = a.zone + base;
+    const int nblk = ENS ? eb.z : (int)min((long long)(PB * PPT), a.n - base);
+    // On a full step every list moves: the particles are loaded without
+    // waiting for their zones, one memory latency instead of two.  Other
+    // steps look at the zones first, since many blocks have nothing to move.
+    const bool full = a.mzone == nz;
+    int zin[PPT];
+    R4 st[PPT];
+    R2 cu[PPT], lo_[COMP ? PPT : 1];
+#pragma unroll
+    for (int k = 0; k < PPT; k++) zin[k] = zb[min(k * PB + tid, nblk - 1)];
+    const int zmid = zb[nblk >> 1];
+    const R2 umid = utb[nblk >> 1];
+    auto load_state = [&]() {
+#pragma unroll
+        for (int k = 0; k < PPT; k++) {
+            const int j = min(k * PB + tid, nblk - 1);
+            cu[k] = utb[j];
+            st[k] = xvb[j];
+            if (COMP) lo_[k] = lob[j];
+        }
+    };
+    if (full) load_state();
+    // LDS set-up while the loads are in flight
+    for (int j = tid; j < UtTab<R>::n; j += PB) s_tab[j] = ut_tab_entry<R>(j);
+    deposit_init(s_dep);
+    if (tid == 0) s_dnoff = s_pushes = 0;
+    unsigned mv = 0;   // bit k: particle k moves
+    if (!full)
+#pragma unroll
+        for (int k = 0; k < PPT; k++)
+            if (k * PB + tid < nblk && zin[k] <= a.mzone) mv |= 1u << k;
+    // every thread reaches this barrier; a block with nothing to move exits
+    if (!__syncthreads_or(full ? 1 : (int)mv)) return;
+    if (full) {
+#pragma unroll
+        for (int k = 0; k < PPT; k++)
+            if (k * PB + tid < nblk && (zin[k] != nlists || a.offanal)) mv |= 1u << k;
+    } else {
+        load_state();
+    }
+    const PushRef ref = push_ref(umid, zmid, nz, nr, na);
+
+    // grdacc's reads for particle k: the four field corners of its old cell
+    // (weights of the old position from its (u, t)) and its interval of the
+    // fixed-force table, straight from the L2 (particles are ordered by cell,
+    // so a wavefront touches a few lines).  Staging the block's field window
+    // in LDS cost two more barriers and a wavefront reduction for its box,
+    // and held the registers and the LDS of a sixth wavefront per SIMD.
+    R2 f[4];
+    double4 fc;
+    auto gather = [&](int k) {
+        R w[4];
+        int ring, spoke, ic[4];
+        const bool grid = (mv >> k & 1u) && zin[k] != nlists;
+        cic(grid ? cu[k].x : (R)0, grid ? cu[k].y : (R)0, nr, na, ring, spoke, w);
+        corners_rs(ring, spoke, na, ic);
+#pragma unroll
+        for (int q = 0; q < 4; q++) f[q] = fld[ic[q] < a.mesh ? ic[q] : 0];
+        if (a.fixforce) {
+            const R rr = sqrt_rn(st[k].x * st[k].x + st[k].y * st[k].y);
+            fc = a.fr_c[fixforce_index((double)rr, a.nfr, a.fr_inv_dr)];
+        }
+    };
+    // zones of the deposits, four bits per particle (0: none); the new
+    // state takes the registers of the old one, stored once every load has
+    // been used: a load waits for the stores issued before it
+    unsigned dzone = 0, zch = 0;
+    int npush = 0, nplus = 0, nminus = 0;   // lane counts by ballot (uniform)
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        gather(k);
+        bool plus = false, minus = false;   // leaving the grid, returning
+        const bool move = mv >> k & 1u;
+        npush += __popcll(__ballot(move));
+        if (move) {
+            opaque(cu[k]);
+            const int z0 = zin[k];
+            const bool offlist = z0 == nlists;
+            R ox = st[k].x, oy = st[k].y, ovx = st[k].z, ovy = st[k].w;
+            const R rr = sqrt_rn(ox * ox + oy * oy);
+            R ax_ = 0, ay_ = 0;
+            if (!offlist) {
+                R w[4];
+                int ring, spoke, ic[4];
+                cic(cu[k].x, cu[k].y, nr, na, ring, spoke, w);
+                corners_rs(ring, spoke, na, ic);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    // the last ring with t == na points past the field: 0
+                    const R wq = ic[q] < a.mesh ? w[q] : (R)0;
+                    ax_ = ax_ + f[q].x * wq;
+                    ay_ = ay_ + f[q].y * wq;
+                }
+                if (a.fixforce) {
+                    const int kf = fixforce_index((double)rr, a.nfr, a.fr_inv_dr);
+                    const R fr = (R)fixforce_at((double)rr, kf, a.nfr, a.fr_inv_dr, &fc, kf);
+                    if (fr != (R)0) {
+                        const R fo = div_rn(fr, rr);
+                        ax_ = ax_ + fo * ox;
+                        ay_ = ay_ + fo * oy;
+                    }
+                }
+            }
+            if (nz > 1 && z0 > 1) {
+                R t = tsfac(a, z0);
+                t = t * t;
+                ax_ = t * ax_;
+                ay_ = t * ay_;
+            }
+            R nvx = ovx + ax_, nvy = ovy + ay_;
+            R nx = ox + nvx, ny = oy + nvy;
+            R2 lo = zero2<R>(), elo = zero2<R>();
+            if (COMP) {
+                lo = lo_[k];
+                nx = comp_add(ox, nvx, lo.x, elo.x);
+                ny = comp_add(oy, nvy, lo.y, elo.y);
+            }
+            int znew = z0;
+            R rnew = sqrt_rn(nx * nx + ny * ny);
+            bool off = rnew > a.rgrid;
+            if (!offlist) {
+                if (off) {
+                    znew = nlists;
+                    plus = true;
+                    if (a.offanal && z0 < nz) {
+                        R tfac = tsfac(a, nz) / tsfac(a, z0);
+                        chstep(tfac, ox, oy, ovx, ovy, ax_, ay_, nx, ny, nvx, nvy);
+                        if (COMP) {
+                            nx = comp_add(ox, nvx, lo.x, elo.x);
+                            ny = comp_add(oy, nvy, lo.y, elo.y);
+                        }
+                        rnew = sqrt(nx * nx + ny * ny);
+                    }
+                }
+            } else if (!off) {
+                minus = true;
+                znew = nz;
+            }
+            if (a.mzone > 1 && !offlist && znew <= a.mzone) {
+                int kz = zone_of(a, rnew);
+                if (kz > a.mzone) kz = a.mzone;
+                if (kz > znew) kz = zone_of(a, rr);
+                if (kz != znew) {
+                    R tfac = tsfac(a, kz) / tsfac(a, znew);
+                    chstep(tfac, ox, oy, ovx, ovy, ax_, ay_, nx, ny, nvx, nvy);
+                    if (COMP) {
+                        nx = comp_add(ox, nvx, lo.x, elo.x);
+                        ny = comp_add(oy, nvy, lo.y, elo.y);
+                    }
+                    rnew = sqrt(nx * nx + ny * ny);
+                    znew = kz;
+                }
+            }
+            st[k] = mk4(nx, ny, nvx, nvy);
+            if (COMP) lo_[k] = elo;
+            if (znew != z0) zch |= 1u << k;
+            zin[k] = znew;
+            if (znew >= 1 && znew <= nz) {
+                R u, t;
+                ut_push(nx, ny, rnew, a.k, u, t, s_tab);
+                cu[k] = mk2(u, t);
+                dzone |= (unsigned)znew << (4 * k);
+            }
+        }
+        nplus += __popcll(__ballot(plus));
+        nminus += __popcll(__ballot(minus));
+    }
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        const int j = k * PB + tid;
+        if (mv >> k & 1u) {
+            xvb[j] = st[k];
+            if (COMP) lob[j] = lo_[k];
+            if (zch >> k & 1u) zb[j] = (uint8_t)zin[k];
+            if (dzone >> (4 * k) & 15u) utb[j] = cu[k];
+        }
+        // the deposit's angle is folded into the sector
+        if (a.nsect > 1) cu[k].y = (R)fmod(cu[k].y, a.thmax);
+    }
+    // the wave's pushes and off-grid change, added to the block's counters by
+    // one lane
+    if (lane == 0) {
+        if (npush) atomicAdd(&s_pushes, npush);
+        if (nplus != nminus) atomicAdd(&s_dnoff, nplus - nminus);
+    }
+    deposit_block<R, PPT>(a, s_dep, cu, dzone, ref, qbits, mo);
+    __syncthreads();
+    deposit_ranges(s_dep, nz, nr, jrad, krad, a.rstride);
     if (tid == 0) {
         if (s_dnoff) atomicAdd((unsigned long long *)&counters[0],
                                (unsigned long long)(long long)s_dnoff);
-        if (s_pushes) atomicAdd((unsigned long long *)&counters[1],
-                                (unsigned long long)s_pushes);
+        count_pushes(a.pushes, blockIdx.x, s_pushes);
     }
 }
 
 // masset / massgn for every on-grid particle without a push: also fills the
-// particles' (u, t) so the next push finds them.  Global atomics after the
-// wavefront reduction.
-template <typename R>
-__global__ __launch_bounds__(GH_BLOCK) void massgn_kernel(PushArgs<R> a) {
-    typedef typename Vec4<R>::T R4;
-    __shared__ int s_jr[GH_MAXZ], s_kr[GH_MAXZ];
-    const int tid = threadIdx.x, lane = tid & 63;
-    if (tid < GH_MAXZ) {
-        s_jr[tid] = INT_MAX;
-        s_kr[tid] = -1;
-    }
-    __syncthreads();
-    long long i = (long long)blockIdx.x * GH_BLOCK + tid;
-    int z = i < a.n ? a.zone[i] : 0;
-    bool on = z >= 1 && z <= a.nz;
-    R w[4];
-    int ring = 0, spoke = 0;
-    if (on) {
-        R rr, u, t;
-        const R4 st = a.xv[i];
-        (void)weight1<R>(st.x, st.y, a.nr, a.k, false, a.thmax, w, rr, u, t);
-        a.ut[i] = mk2(u, t);
-        R tf = a.nsect > 1 ? (R)fmod(t, a.thmax) : t;
-        cic(u, tf, a.nr, a.na, ring, spoke, w);
-        atomicMin(&s_jr[z - 1], ring);
-        atomicMax(&s_kr[z - 1], ring);
-    }
-    __syncthreads();
-    // one global min/max per zone and block (ring ranges are 1-based)
-    if (tid < a.nz && s_kr[tid] >= 0) {
-        atomicMin(&a.jrad[tid], s_jr[tid] + 1);
-        int k = s_kr[tid] + 2;
-        atomicMax(&a.krad[tid], k < a.nr ? k : a.nr);
-    }
-    const int key = on ? ((z - 1) * (a.nr + 1) + ring) * a.na + spoke : -1;
-    long long qv[4];
-    quant_n<R, 4>(w, a.qbits, on, qv);
-    unsigned long long pend = __ballot(key >= 0);
-    while (pend) {
-        const int leader = __ffsll((long long)pend) - 1;
-        const int lk = __shfl(key, leader, 64);
-        const bool mine = key == lk;
-        const unsigned long long mm = __ballot(mine);
-        long long s[4];
-        for (int q = 0; q < 4; q++) s[q] = wave_sum64(mine ? qv[q] : 0);
-        if (lane == leader) {
-            int ic[4];
-            corners_rs(ring, spoke, a.na, ic);
-            for (int q = 0; q < 4; q++)
-                if (s[q] != 0) deposit_global(a.mfx, a.nz, a.mesh, z, ic[q], s[q]);
+// particles' (u, t) so the next push finds them.  ENS: the members' blocks
+// of a.blk.  The push's deposit, one particle per thread (with a reduction
+// over the wavefront per cell and global atomics it took 530 us for 1e7
+// particles, 108 us now).
+template <typename R, bool ENS, int PPT>
+__global__ __launch_bounds__(PB, (PushShape<R, false, PPT>::waves)) void massgn_kernel(PushArgs<R> a) {
+    typedef typename Vec2<R>::T R2;
+    __shared__ DepositLds<PushShape<R, false, PPT>::tile> s_dep;
+    __shared__ R2 s_mid;
+    __shared__ int s_zmid;
+    const int tid = threadIdx.x;
+    const int4 eb = ENS ? a.blk[blockIdx.x] : make_int4(0, 0, 0, 0);
+    const long long base = ENS ? (long long)eb.y : (long long)blockIdx.x * (PB * PPT);
+    const int nblk = ENS ? eb.z : (int)min((long long)(PB * PPT), a.n - base);
+    R2 cu[PPT];
+    unsigned dzone = 0;
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        const int j = k * PB + tid;
+        cu[k] = zero2<R>();
+        const int z = j < nblk ? a.zone[base + j] : 0;
+        if (z >= 1 && z <= a.nz) {
+            const typename Vec4<R>::T st = a.xv[base + j];
+            R u, t;
+            ut_of(st.x, st.y, sqrt(st.x * st.x + st.y * st.y), a.k, u, t);
+            a.ut[base + j] = mk2(u, t);
+            cu[k] = mk2(u, a.nsect > 1 ? (R)fmod(t, a.thmax) : t);
+            dzone |= (unsigned)z << (4 * k);
         }
-        pend &= ~mm;
     }
+    // the middle particle's cell from the thread that has formed it
+#pragma unroll
+    for (int k = 0; k < PPT; k++)
+        if (k * PB + tid == nblk >> 1) {
+            s_mid = cu[k];
+            s_zmid = (int)(dzone >> (4 * k) & 15u);
+        }
+    deposit_init(s_dep);
+    __syncthreads();
+    const PushRef ref = push_ref(s_mid, s_zmid, a.nz, a.nr, a.na);
+    deposit_block<R, PPT>(a, s_dep, cu, dzone, ref, ENS ? a.qbits_m[eb.x] : a.qbits,
+                          ENS ? (long long)eb.x * a.mesh : 0);
+    __syncthreads();
+    deposit_ranges(s_dep, a.nz, a.nr, a.jrad + (ENS ? eb.x * GH_MAXZ : 0),
+                   a.krad + (ENS ? eb.x * GH_MAXZ : 0), a.rstride);
 }
 
 // (u, t) of every particle's position (after a load)
@@ -1072,36 +1020,52 @@ static inline unsigned nblocks(long long n, long long per) {
     return (unsigned)((n + per - 1) / per);
 }
 
-template <typename R, bool COMP>
+template <typename R, bool COMP, int PPT>
 static void launch_push_c(const PushArgs<R> &a, hipStream_t s) {
-    if (a.blk) {
-        if (a.nblocks > 0)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(push_kernel<R, true, COMP>), dim3(a.nblocks),
-                               dim3(PB), 0, s, a);
-    } else {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(push_kernel<R, false, COMP>),
+    if (a.blk)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(push_kernel<R, true, COMP, PPT>), dim3(a.nblocks),
+                           dim3(PB), 0, s, a);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(push_kernel<R, false, COMP, PPT>),
                            dim3(nblocks(a.n, PB * PPT)), dim3(PB), 0, s, a);
-    }
 }
 
+// a.ppt: push_ppt's choice (an ensemble's block table is made for it)
 template <typename R>
 hipError_t launch_push(const PushArgs<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
     if constexpr (sizeof(R) == 4) {
-        if (a.xlo) launch_push_c<R, true>(a, s);
-        else launch_push_c<R, false>(a, s);
+        if (a.ppt == 1) {
+            if (a.xlo) launch_push_c<R, true, 1>(a, s);
+            else launch_push_c<R, false, 1>(a, s);
+        } else {
+            if (a.xlo) launch_push_c<R, true, 4>(a, s);
+            else launch_push_c<R, false, 4>(a, s);
+        }
     } else {
         if (a.xlo) return hipErrorInvalidValue;   // compensated positions are FP32 only
-        launch_push_c<R, false>(a, s);
+        if (a.ppt != 1) return hipErrorInvalidValue;
+        launch_push_c<R, false, 1>(a, s);
     }
     return hipGetLastError();
+}
+
+template <typename R, int PPT>
+static void launch_massgn_p(const PushArgs<R> &a, hipStream_t s) {
+    if (a.blk)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(massgn_kernel<R, true, PPT>), dim3(a.nblocks), dim3(PB),
+                           0, s, a);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(massgn_kernel<R, false, PPT>),
+                           dim3(nblocks(a.n, PB * PPT)), dim3(PB), 0, s, a);
 }
 
 template <typename R>
 hipError_t launch_massgn(const PushArgs<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(massgn_kernel<R>, dim3(nblocks(a.n, GH_BLOCK)),
-                       dim3(GH_BLOCK), 0, s, a);
+    if (a.ppt == 1) launch_massgn_p<R, 1>(a, s);
+    else if constexpr (sizeof(R) == 4) launch_massgn_p<R, 4>(a, s);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

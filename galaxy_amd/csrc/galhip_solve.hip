@@ -39,7 +39,7 @@ template <typename R>
 __global__ __launch_bounds__(SOLVE_BLOCK) void analyse_kernel(AnaArgs<R> a) {
     __shared__ R rho_s[MAX_NA];
     __shared__ R tws[2 * MAX_NA];
-    __shared__ int s_rng[4], s_ok;
+    __shared__ int s_rng[4], s_ok, s_jr[GH_MAXZ], s_kr[GH_MAXZ];
     const int tid = threadIdx.x, na = a.na, ir = blockIdx.x + 1;
     const int h = blockIdx.y, mem = blockIdx.z;
     // member mem's grids
@@ -51,9 +51,10 @@ __global__ __launch_bounds__(SOLVE_BLOCK) void analyse_kernel(AnaArgs<R> a) {
     R *const coef = a.coef + (size_t)mem * a.ncoef * a.nr;
     const double q = a.qbits_m ? ldexp(1.0, -a.qbits_m[mem]) : a.q;
     const double pmass = a.pmass_m ? a.pmass_m[mem] : a.pmass;
+    if (tid < 64) combine_ranges(jrad, krad, a.rstride, a.nz, s_jr, s_kr);
     if (tid == 0) {
         int kr[GH_MAXZ], rg[4] = {0, 0, 0, 0};
-        bool ok = solve_ranges(jrad, krad, a.nz, a.nr, a.mzone, a.lpot,
+        bool ok = solve_ranges(s_jr, s_kr, a.nz, a.nr, a.mzone, a.lpot,
                                a.explicit_zones, a.jzone, a.kzone, kr, rg);
         s_ok = ok;
         for (int q = 0; q < 4; q++) s_rng[q] = rg[q];
@@ -138,9 +139,11 @@ __global__ __launch_bounds__(SOLVE_BLOCK) void synth_kernel(SynArgs<R> a) {
                 a.mfx[z - 1][idx] = 0;
             }
         }
-        if (blockIdx.x == 0 && q == 0 && tid < a.masscl_z) {
-            a.jrad[mem * GH_MAXZ + tid] = nr;
-            a.krad[mem * GH_MAXZ + tid] = 0;
+        if (blockIdx.x == 0 && q == 0 && tid < a.masscl_z * GH_RANGE_STRIPES) {
+            const int z = tid / GH_RANGE_STRIPES;
+            const int e = (tid & (GH_RANGE_STRIPES - 1)) * a.rstride + mem * GH_MAXZ + z;
+            a.jrad[e] = nr;
+            a.krad[e] = 0;
         }
     }
     const int jrs = ranges[0], krs = ranges[1];
@@ -341,7 +344,7 @@ __global__ void fill_kernel(T *__restrict__ p, T v, long long n) {
 // reset jrad/krad of those zones, for the ncell = nmem x mesh cells of nmem
 // grids (ring ranges GH_MAXZ apart).
 __global__ void masscl_kernel(ZonePtrs zp, int mz, long long ncell, int *jrad,
-                              int *krad, int nr, int nmem) {
+                              int *krad, int rstride, int nr, int nmem) {
     long long i = (long long)blockIdx.x * GH_BLOCK + threadIdx.x;
     if (i < ncell) {
         for (int z = 1; z <= mz; z++) {
@@ -349,10 +352,11 @@ __global__ void masscl_kernel(ZonePtrs zp, int mz, long long ncell, int *jrad,
             zp.mfx[z - 1][i] = 0;
         }
     }
-    if (i < (long long)mz * nmem) {
-        const int m = (int)(i / mz), z = (int)(i - (long long)m * mz);
-        jrad[m * GH_MAXZ + z] = nr;
-        krad[m * GH_MAXZ + z] = 0;
+    if (i < (long long)mz * nmem * GH_RANGE_STRIPES) {
+        const int s = (int)(i & (GH_RANGE_STRIPES - 1)), r = (int)(i / GH_RANGE_STRIPES);
+        const int m = r / mz, e = s * rstride + m * GH_MAXZ + (r - m * mz);
+        jrad[e] = nr;
+        krad[e] = 0;
     }
 }
 
@@ -613,11 +617,11 @@ hipError_t launch_fill_i32(int *p, int v, long long n, hipStream_t s) {
 }
 
 hipError_t launch_masscl(const ZonePtrs &zp, int mz, long long mesh, int *jrad,
-                         int *krad, int nr, int nmem, hipStream_t s) {
-    const long long ncell = mesh * nmem, nz = (long long)mz * nmem;
+                         int *krad, int rstride, int nr, int nmem, hipStream_t s) {
+    const long long ncell = mesh * nmem, nz = (long long)mz * nmem * GH_RANGE_STRIPES;
     long long n = ncell > nz ? ncell : nz;
     hipLaunchKernelGGL(masscl_kernel, dim3((unsigned)((n + GH_BLOCK - 1) / GH_BLOCK)),
-                       dim3(GH_BLOCK), 0, s, zp, mz, ncell, jrad, krad, nr, nmem);
+                       dim3(GH_BLOCK), 0, s, zp, mz, ncell, jrad, krad, rstride, nr, nmem);
     return hipGetLastError();
 }
 
