@@ -330,6 +330,18 @@ __device__ __forceinline__ int weight1(R x, R y, int nr, const UtConst &k,
     return ring * k.na + spoke;
 }
 
+// step ratio of list iz (the off-grid list has the top zone's): the first
+// three zones by selection between uniform values (an indexed read of the
+// argument block is a load, and a load after the particle stores waits for
+// them)
+__device__ __forceinline__ int step_ratio(const int *nstep, int nz, int iz) {
+    const int i = iz < nz ? iz : nz;
+    int n = i == 1 ? nstep[0] : i == 2 ? nstep[1] : nstep[2];
+    for (int q = 4; q <= nz; q++)
+        if (i == q) n = nstep[q - 1];
+    return n;
+}
+
 // Fixed-point weight: w * 2^qbits, rounded to nearest even.
 template <typename R>
 __device__ __forceinline__ long long quant(R w, int qbits) {

@@ -6,7 +6,7 @@
 // per cell, (F_x, F_y, F_z, potential), so that an interpolation corner is
 // one 16-byte (FP32) load.
 //
-// Particle kernels (one thread per particle):
+// Particle kernels:
 //   p3_massgn_kernel  massgn of every on-grid particle (massgn.f:140-172)
 //   p3_push_kernel    getacc (grdacc.f:189-211, getacc.f:106-151) + stpgrp
 //                     + offgrd (|z| > zm or R > rgrid, offgrd.f:69-72) +
@@ -58,6 +58,28 @@ __device__ __forceinline__ void ut3(R x, R y, const P3Args<R> &a, R &u, R &t) {
     if (!(rr > (R)0)) t = (R)0;
 }
 
+// A position's grid coordinates (weight.f:210-230): u, t (folded into the
+// sector for mass assignment) and zz = (z + zm) / dzg.
+template <typename R> struct P3Pos {
+    R u, t, zz;
+};
+template <typename R>
+__device__ __forceinline__ P3Pos<R> pos3(R u, R t, R z, const P3Args<R> &a, bool fold) {
+    P3Pos<R> p;
+    p.u = u;
+    p.t = fold ? (R)fmod(t, a.thmax) : t;
+    p.zz = div_rn(z + a.zm, a.dzg);
+    return p;
+}
+
+// Hides a position's origin from the optimiser (no instruction is issued).
+__device__ __forceinline__ void opaque3(P3Pos<float> &p) {
+    asm volatile("" : "+v"(p.u), "+v"(p.t), "+v"(p.zz));
+}
+__device__ __forceinline__ void opaque3(P3Pos<double> &p) {
+    asm volatile("" : "+v"(p.u), "+v"(p.t), "+v"(p.zz));
+}
+
 // ut3 in the push (ut_push); rr the position's cylindrical radius
 template <typename R>
 __device__ __forceinline__ void ut3_push(R x, R y, R rr, const P3Args<R> &a, R &u, R &t,
@@ -66,22 +88,34 @@ __device__ __forceinline__ void ut3_push(R x, R y, R rr, const P3Args<R> &a, R &
     if (!(rr > (R)0)) t = (R)0;
 }
 
-// weight() for one position given its (u, t), p3d jmass = 2
-// (weight.f:219-248): returns the 0-based cell (ju ngz + jz) na + jt and the
-// 8 weights in the reference's order (bit 0 = dt, bit 1 = dz, bit 2 = du).
+// The cell of a position: ring and plane of the low corner (jmass 2,
+// weight.f:219-231) or the nearest node (jmass 3, ring >= 1, t rounding to
+// na folded to spoke 0; weight.f:281-292).  For jmass 2 the spoke is na when t
+// has rounded to na.
+template <typename R, int J>
+__device__ __forceinline__ void loc3(const P3Pos<R> &p, const P3Args<R> &a, int &ring, int &plane,
+                                     int &spoke) {
+    const R h = J == 3 ? (R)0.5 : (R)0;
+    ring = J == 3 ? (int)(p.u + h) : (int)p.u;
+    plane = J == 3 ? (int)(p.zz + h) : (int)p.zz;
+    spoke = J == 3 ? (int)(p.t + h) : (int)p.t;
+    if (ring > a.nr - 2) ring = a.nr - 2;
+    if (J == 3 && ring < 1) ring = 1;
+    if (plane < 0) plane = 0;
+    if (plane > a.ngz - 2) plane = a.ngz - 2;
+    if (J == 3 && spoke == a.na) spoke = 0;
+}
 template <typename R>
-__device__ __forceinline__ int cell3(R u, R t, R z, const P3Args<R> &a, bool fold, R w[8],
-                                     int &ring, int &plane, int &spoke) {
-    R zz = z + a.zm;
-    if (fold) t = (R)fmod(t, a.thmax);
-    int ju = (int)u;
-    if (ju > a.nr - 2) ju = a.nr - 2;
-    int jt = (int)t;
-    zz = div_rn(zz, a.dzg);
-    int jz = (int)zz;
-    if (jz < 0) jz = 0;
-    if (jz > a.ngz - 2) jz = a.ngz - 2;
-    const R du = u - (R)ju, dt = t - (R)jt, dz = zz - (R)jz;
+__device__ __forceinline__ int cell_index(const P3Args<R> &a, int ring, int plane, int spoke) {
+    return (ring * a.ngz + plane) * a.na + spoke;
+}
+
+// The weights of a position in cell (ring, plane): 8 in the reference's order
+// (bit 0 = dt, bit 1 = dz, bit 2 = du; weight.f:232-248), or 27, spoke
+// offset -1, 0, +1 fastest, then plane, then ring (weight.f:281-300).
+template <typename R>
+__device__ __forceinline__ void weights3(const P3Pos<R> &p, int ring, int plane, R (&w)[8]) {
+    const R du = p.u - (R)ring, dt = p.t - (R)(int)p.t, dz = p.zz - (R)plane;
     const R one = (R)1;
     w[0] = (one - dt) * (one - dz) * (one - du);
     w[1] = dt * (one - dz) * (one - du);
@@ -91,46 +125,15 @@ __device__ __forceinline__ int cell3(R u, R t, R z, const P3Args<R> &a, bool fol
     w[5] = dt * (one - dz) * du;
     w[6] = (one - dt) * dz * du;
     w[7] = dt * dz * du;
-    ring = ju;
-    plane = jz;
-    spoke = jt;
-    return (ju * a.ngz + jz) * a.na + jt;
 }
-
 template <typename R>
-__device__ __forceinline__ int weight3(R x, R y, R z, const P3Args<R> &a, bool fold, R w[8]) {
-    R u, t;
-    int rg, pl, sp;
-    ut3(x, y, a, u, t);
-    return cell3(u, t, z, a, fold, w, rg, pl, sp);
-}
-
-// weight() for jmass = 3 given (u, t) (weight.f:281-300): the central cell
-// of the 27 (nearest node, ju >= 1, jt == na folded to spoke 0) and their
-// weights, spoke offset -1, 0, +1 fastest, then plane, then ring.
-template <typename R>
-__device__ __forceinline__ int cell3q(R u, R t, R z, const P3Args<R> &a, bool fold, R w[27],
-                                      int &ring, int &plane, int &spoke) {
-    R zz = z + a.zm;
-    if (fold) t = (R)fmod(t, a.thmax);
+__device__ __forceinline__ void weights3(const P3Pos<R> &p, int ring, int plane, R (&w)[27]) {
     const R h = (R)0.5;
-    int ju = (int)(u + h);
-    if (ju > a.nr - 2) ju = a.nr - 2;
-    if (ju < 1) ju = 1;
-    const int jt = (int)(t + h);
-    zz = div_rn(zz, a.dzg);
-    int jz = (int)(zz + h);
-    if (jz < 0) jz = 0;
-    if (jz > a.ngz - 2) jz = a.ngz - 2;
-    int c = (ju * a.ngz + jz) * a.na + jt;
-    if (jt == a.na) c -= a.na;
-    ring = ju;
-    plane = jz;
-    spoke = jt == a.na ? 0 : jt;
     R dp[3][3];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const R dd = i == 0 ? t + h - (R)jt : i == 1 ? zz + h - (R)jz : u + h - (R)ju;
+        const R dd = i == 0 ? p.t + h - (R)(int)(p.t + h) : i == 1 ? p.zz + h - (R)plane
+                                                                    : p.u + h - (R)ring;
         dp[0][i] = (R)1 - (R)2 * dd + dd * dd;
         dp[1][i] = (R)1 + (R)2 * dd - (R)2 * (dd * dd);
         dp[2][i] = dd * dd;
@@ -142,22 +145,19 @@ __device__ __forceinline__ int cell3q(R u, R t, R z, const P3Args<R> &a, bool fo
 #pragma unroll
             for (int i = 0; i < 3; i++)
                 w[9 * k + 3 * j + i] = (R)0.125 * dp[i][0] * dp[j][1] * dp[k][2];
-    return c;
 }
 
 // weights per particle of interpolation scheme J (jmass 2 or 3)
 template <int J> struct P3NW { static constexpr int v = J == 3 ? 27 : 8; };
 
+// cell index, its parts and the weights of a position given its (u, t)
 template <typename R, int J>
-__device__ __forceinline__ int cellJ(R u, R t, R z, const P3Args<R> &a, bool fold, R *w,
-                                     int &ring, int &plane, int &spoke) {
-    if constexpr (J == 3) return cell3q<R>(u, t, z, a, fold, w, ring, plane, spoke);
-    else return cell3<R>(u, t, z, a, fold, w, ring, plane, spoke);
-}
-template <typename R, int J>
-__device__ __forceinline__ int cellJ(R u, R t, R z, const P3Args<R> &a, bool fold, R *w) {
-    int rg, pl, sp;
-    return cellJ<R, J>(u, t, z, a, fold, w, rg, pl, sp);
+__device__ __forceinline__ int cellJ(R u, R t, R z, const P3Args<R> &a, bool fold,
+                                     R (&w)[P3NW<J>::v], int &ring, int &plane, int &spoke) {
+    const P3Pos<R> p = pos3(u, t, z, a, fold);
+    loc3<R, J>(p, a, ring, plane, spoke);
+    weights3(p, ring, plane, w);
+    return cell_index(a, ring, plane, spoke);
 }
 
 // grdacc's corners (grdacc.f:193-203): c, c+1 (wrapped when c+1 is a
@@ -200,7 +200,7 @@ template <int J> __device__ __forceinline__ void cornersJ(int c, int spoke, int 
 
 template <typename R>
 __device__ __forceinline__ R tsfac3(const P3Args<R> &a, int iz) {
-    return (R)a.nstep[(iz < a.nz ? iz : a.nz) - 1];
+    return (R)step_ratio(a.nstep, a.nz, iz);
 }
 
 // zoneno with spherical boundaries (zoneno.f:40-55, setrun.f:810)
@@ -240,18 +240,25 @@ __device__ __forceinline__ void getacc3(const P3Args<R> &a, R ox, R oy, R oz, R 
         const int c = cellJ<R, J>(u, t, oz, a, false, w, rg, pl, sp);
         cornersJ<J>(c, sp, a.na, a.ngz, ic);
         R sx = (R)0, sy = (R)0, sz = (R)0;
+        // a corner outside the field array (the last ring with t == na; for
+        // jmass 3 also the first ring's bottom plane) reads 0: cell 0 is read
+        // instead and its weight is 0.  Only a wavefront with such a lane
+        // tests its corners.
+        const int reach = (a.ngz + 1) * a.na + 1;   // largest corner offset
+        if (any_lane(c + reach >= a.mesh || (J == 3 && c < reach))) {
+#pragma unroll
+            for (int q = 0; q < NW; q++)
+                if (ic[q] < 0 || ic[q] >= a.mesh) {
+                    ic[q] = 0;
+                    w[q] = (R)0;
+                }
+        }
 #pragma unroll
         for (int q = 0; q < NW; q++) {
-            // a corner outside the field array (the last ring with t == na;
-            // for jmass 3 also the first ring's bottom plane) reads 0: cell 0
-            // is read instead and its value multiplied by 0 (unconditional
-            // loads, no per-corner branch)
-            const bool in = ic[q] >= 0 && ic[q] < a.mesh;
-            const R4 f = a.fld[in ? ic[q] : 0];
-            const R wq = in ? w[q] : (R)0;
-            sx = sx + f.x * wq;
-            sy = sy + f.y * wq;
-            sz = sz + f.z * wq;
+            const R4 f = a.fld[ic[q]];
+            sx = sx + f.x * w[q];
+            sy = sy + f.y * w[q];
+            sz = sz + f.z * w[q];
         }
         if (a.fixforce) {
             R r2 = (R)0;
@@ -280,173 +287,224 @@ __device__ __forceinline__ void getacc3(const P3Args<R> &a, R ox, R oy, R oz, R 
     }
 }
 
-__device__ __forceinline__ int p3_wave_min(int v) { return wave_min_i32(v); }
-__device__ __forceinline__ int p3_wave_max(int v) { return wave_max_i32(v); }
+// Launch shape of the push and the mass assignment.  Linear FP32: two
+// particles per thread share the window's reductions, clearing and flush, and
+// 20 KB of LDS leave seven wavefronts per SIMD (2e7 particles on 200 x 256 x
+// 125, push averaged over an eight-step sort cycle, us: one particle per
+// thread in blocks of 512 with 4096 cells 686; two in blocks of 256 with 4096,
+// 3072, 2560, 2048 cells 708, 640, 633, 736; four 697; two in blocks of 512
+// 689-706; 749 before, at one per thread).  The 27 weights of the quadratic
+// scheme and FP64 keep one.
+template <typename R, int J> struct P3Shape {
+    static constexpr bool two = J == 2 && sizeof(R) == 4;
+    static constexpr int ppt = two ? 2 : 1;
+    static constexpr int block = two ? 256 : 512;
+    static constexpr int tile = two ? 2560 : 4096;
+    static constexpr int waves = two ? 7 : 4;
+};
+constexpr int P3_PASSES = 8;   // window passes before the direct fallback
 
-#ifndef GH_P3_TILE
-#define GH_P3_TILE 4096
-#endif
-#ifndef GH_P3_PASSES
-#define GH_P3_PASSES 8
-#endif
-constexpr int P3_TILE = GH_P3_TILE;       // cells of a block's LDS deposit window
-constexpr int P3_PASSES = GH_P3_PASSES;   // window passes before the direct fallback
-constexpr int P3_SB = 13;                 // ints of the block scratch s_b
+// LDS of a block's deposit.
+template <int TILE> struct Deposit3Lds {
+    long long tile[TILE];
+    int jr[GH_MAXZ], kr[GH_MAXZ];    // central ring ranges by zone
+    int box[12];                     // two (min, max) x (ring, plane, spoke) boxes
+    unsigned long long ref[2];       // two reference keys
+};
+template <int TB, int TILE>
+__device__ __forceinline__ void deposit3_init(Deposit3Lds<TILE> &s) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < TILE; j += TB) s.tile[j + tid] = 0;
+    if (tid < GH_MAXZ) {
+        s.jr[tid] = INT_MAX;
+        s.kr[tid] = -1;
+    }
+    if (tid < 12) s.box[tid] = (tid & 1) ? -1 : INT_MAX;
+    if (tid < 2) s.ref[tid] = ~0ull;
+}
+
+struct P3Ref {
+    int zone, ring, plane, spoke;
+};
 
 // Block-level fixed-point deposit.  The block's particles (sorted by cell,
 // so a block covers a few neighbouring cells) are accumulated into an LDS
 // window spanning the (ring, plane, spoke) box of their corners, then the
 // window's non-zero cells are added to the zone array with one global atomic
-// each (consecutive cells of a row, so the atomics of a wave coalesce).  The
-// corners of a central cell are the next ring, plane and spoke (jmass 2) or
-// the cells one either side (jmass 3); spokes wrap around the ring, so the
-// window's spoke axis runs past na (or below 0) and the flush folds it back.
-// A box larger than P3_TILE cells is clipped to at most 8 rings and 8
-// planes, then as many spokes as fit, placed about a reference particle:
-// the middle thread's, or the first pending one after it in thread order.
+// each (consecutive cells of a row, so the atomics of a wave coalesce) and
+// cleared.  The corners of a central cell are the next ring, plane and spoke
+// (jmass 2) or the cells one either side (jmass 3); spokes wrap around the
+// ring, so the window's spoke axis runs past na (or below 0) and the flush
+// folds it back.  A box larger than TILE cells is clipped to at most 8 rings
+// and 8 planes, then as many spokes as fit, placed about a reference cell.
 // The particles it leaves out (outliers that have moved away from the
-// block's cells, or the far rows of a block in a sparse region) get the
-// next pass's window over what remains, up to P3_PASSES passes; the
-// reference particle is always inside its window.
+// block's cells, the far rows of a block in a sparse region, other zones)
+// get the next pass's window, up to P3_PASSES passes: the first pass takes
+// the zone and cell of the block's middle particle, a later one those of the
+// first pending particle in particle order from there, which is always
+// inside its own window.
 // Particles whose corners leave the row structure (the plane next to the
-// last or, for jmass 3, the first; a linear cell at t == na), those of
-// another zone than the block's lowest, and those still left after the last
-// pass add their corners to the zone array directly.  Integer sums: the
-// result does not depend on the grouping.  Every thread of the block must
-// call it (on = false for threads without a deposit).  s_b: P3_SB ints,
-// s_b[0] = INT_MAX on entry; s_jr/s_kr receive the block's central-ring
-// minimum and maximum per zone.
-template <typename R, int J>
-__device__ __forceinline__ void deposit3_block(const P3Args<R> &a, bool on, int z, int c,
-                                               int ring, int plane, int spoke,
-                                               const R *w, long long *tile, int *s_b,
-                                               unsigned long long *s_ref, int *s_jr,
-                                               int *s_kr) {
+// last or, for jmass 3, the first; a linear cell at t == na) and those still
+// left after the last pass add their corners to the zone array directly.
+// Integer sums: the result does not depend on the grouping.  Every thread of
+// the block must call it; dz[k]: the deposit's zone (0: none).
+template <typename R, int J, int PPT, int TB, int TILE>
+__device__ __forceinline__ void deposit3_block(const P3Args<R> &a, Deposit3Lds<TILE> &s,
+                                               P3Pos<R> (&pos)[PPT], unsigned dzone, P3Ref ref) {
     constexpr int NW = P3NW<J>::v;
     constexpr int LO = J == 3 ? 1 : 0;   // corner cells below the central one
     const int tid = threadIdx.x, lane = tid & 63;
-    // reference key: thread order from the middle thread, then the cell
-    const unsigned long long rkey =
-        ((unsigned long long)((tid - P3_PBLOCK / 2) & (P3_PBLOCK - 1)) << 40) |
-        ((unsigned long long)(unsigned)ring << 26) | ((unsigned long long)(unsigned)plane << 13) |
-        (unsigned long long)(unsigned)spoke;
-    if (!on) ring = plane = spoke = 0;
-    // the block's zone: the lowest among its deposits
-    int zw = p3_wave_min(on ? z : INT_MAX);
-    if (lane == 0 && zw != INT_MAX) atomicMin(&s_b[0], zw);
-    if (tid == 0) {
-        // two (min, max) x (ring, plane, spoke) box buffers, used by
-        // alternate passes so that one can be reset while the other is read
+    unsigned pend = 0;
 #pragma unroll
-        for (int k = 1; k < P3_SB; k++) s_b[k] = (k & 1) ? INT_MAX : -1;
-        s_ref[0] = s_ref[1] = ~0ull;
+    for (int k = 0; k < PPT; k++) {
+        int ring, plane, spoke;
+        loc3<R, J>(pos[k], a, ring, plane, spoke);
+        if ((dzone >> (4 * k) & 15u) && plane - LO >= 0 && plane + 1 < a.ngz && spoke < a.na &&
+            ring - LO >= 0)
+            pend |= 1u << k;
     }
-    __syncthreads();
-    const int tz = s_b[0];
-    bool pend = on && z == tz && plane - LO >= 0 && plane + 1 < a.ngz && spoke < a.na &&
-                ring - LO >= 0;
-    {
-        // ring ranges: the block zone's by wave reduction, others directly
-        const int jr = p3_wave_min(on && z == tz ? ring : INT_MAX);
-        const int kr = p3_wave_max(on && z == tz ? ring : -1);
-        if (lane == 0 && kr >= 0) {
-            atomicMin(&s_jr[tz - 1], jr);
-            atomicMax(&s_kr[tz - 1], kr);
-        }
-        if (on && z != tz) {
-            atomicMin(&s_jr[z - 1], ring);
-            atomicMax(&s_kr[z - 1], ring);
-        }
-    }
-    long long v[NW];
-    quant_n<R, NW>(w, a.qbits, on, v);
-    bool direct = on && !pend;
+    unsigned direct = 0;
+#pragma unroll
+    for (int k = 0; k < PPT; k++)
+        if ((dzone >> (4 * k) & 15u) && !(pend >> k & 1u)) direct |= 1u << k;
+    auto in_zone = [&](int k, int z) {
+        return (pend >> k & 1u) && (int)(dzone >> (4 * k) & 15u) == z;
+    };
+#pragma unroll 1
     for (int pass = 0;; pass++) {
-        int *const sb = s_b + 1 + 6 * (pass & 1);
+        int *const sb = s.box + 6 * (pass & 1);
+        // cells and weights are formed again from the grid coordinates
+#pragma unroll
+        for (int k = 0; k < PPT; k++) opaque3(pos[k]);
         {
-            const int r0 = p3_wave_min(pend ? ring : INT_MAX), r1 = p3_wave_max(pend ? ring : -1);
-            const int p0 = p3_wave_min(pend ? plane : INT_MAX), p1 = p3_wave_max(pend ? plane : -1);
-            const int q0 = p3_wave_min(pend ? spoke : INT_MAX), q1 = p3_wave_max(pend ? spoke : -1);
-            // the wave's first pending lane holds its lowest reference key
-            const unsigned long long bal = __ballot(pend);
-            const int fl = bal ? __ffsll((long long)bal) - 1 : 0;
-            const unsigned klo = __builtin_amdgcn_readlane((unsigned)rkey, fl);
-            const unsigned khi = __builtin_amdgcn_readlane((unsigned)(rkey >> 32), fl);
+            int r0 = INT_MAX, r1 = -1, p0 = INT_MAX, p1 = -1, q0 = INT_MAX, q1 = -1;
+#pragma unroll
+            for (int k = 0; k < PPT; k++) {
+                int ring, plane, spoke;
+                loc3<R, J>(pos[k], a, ring, plane, spoke);
+                if (in_zone(k, ref.zone)) {
+                    r0 = min(r0, ring);
+                    r1 = max(r1, ring);
+                    p0 = min(p0, plane);
+                    p1 = max(p1, plane);
+                    q0 = min(q0, spoke);
+                    q1 = max(q1, spoke);
+                }
+            }
+            r0 = wave_min_i32(r0);
+            r1 = wave_max_i32(r1);
+            p0 = wave_min_i32(p0);
+            p1 = wave_max_i32(p1);
+            q0 = wave_min_i32(q0);
+            q1 = wave_max_i32(q1);
             if (lane == 0 && r1 >= 0) {
-                atomicMin(&sb[0], r0); atomicMax(&sb[1], r1);
-                atomicMin(&sb[2], p0); atomicMax(&sb[3], p1);
-                atomicMin(&sb[4], q0); atomicMax(&sb[5], q1);
-                atomicMin(&s_ref[pass & 1], ((unsigned long long)khi << 32) | klo);
+                atomicMin(&sb[0], r0);
+                atomicMax(&sb[1], r1);
+                atomicMin(&sb[2], p0);
+                atomicMax(&sb[3], p1);
+                atomicMin(&sb[4], q0);
+                atomicMax(&sb[5], q1);
             }
         }
         __syncthreads();
-        // the box of the pending corners, clipped from its low corner
+        // the box of the pending corners, clipped about the reference cell
         int r0 = sb[0] - LO, p0 = sb[2] - LO, q0 = sb[4] - LO;
         int NR = sb[1] - sb[0] + 2 + LO, NP = sb[3] - sb[2] + 2 + LO;
         int NQ = sb[5] - sb[4] + 2 + LO;
-        const bool use = sb[1] >= 0;
-        const unsigned long long kref = s_ref[pass & 1];
+        const bool some = sb[1] >= 0;
         if (tid == 0) {
-            int *const nb = s_b + 1 + 6 * ((pass + 1) & 1);   // last read in the previous pass
+            if (some) {
+                atomicMin(&s.jr[ref.zone - 1], sb[0]);
+                atomicMax(&s.kr[ref.zone - 1], sb[1]);
+            }
+            // the other box and key were last read before this barrier
+            int *const nb = s.box + 6 * ((pass + 1) & 1);
 #pragma unroll
             for (int k = 0; k < 6; k++) nb[k] = (k & 1) ? -1 : INT_MAX;
-            s_ref[(pass + 1) & 1] = ~0ull;
+            s.ref[(pass + 1) & 1] = ~0ull;
         }
-        if (use && NR * NP * NQ > P3_TILE) {
-            // about the reference cell, inside the box
-            const int rr = (int)((kref >> 26) & 0x1FFF), rp = (int)((kref >> 13) & 0x1FFF);
-            const int rq = (int)(kref & 0x1FFF);
+        if (some && (long long)NR * NP * NQ > TILE) {
             if (NR > 8) {
-                r0 = min(max(rr - LO - 3, r0), r0 + NR - 8);
+                r0 = min(max(ref.ring - LO - 3, r0), r0 + NR - 8);
                 NR = 8;
             }
             if (NP > 8) {
-                p0 = min(max(rp - LO - 3, p0), p0 + NP - 8);
+                p0 = min(max(ref.plane - LO - 3, p0), p0 + NP - 8);
                 NP = 8;
             }
-            const int mq = P3_TILE / (NR * NP);
+            const int mq = TILE / (NR * NP);
             if (NQ > mq) {
-                q0 = min(max(rq - LO - (mq - 2 - LO) / 2, q0), q0 + NQ - mq);
+                q0 = min(max(ref.spoke - LO - (mq - 2 - LO) / 2, q0), q0 + NQ - mq);
                 NQ = mq;
             }
         }
-        const int ncell = use ? NR * NP * NQ : 0;
-        for (int e = tid; e < ncell; e += P3_PBLOCK) tile[e] = 0;
-        __syncthreads();
-        const bool inside = pend && ring - LO >= r0 && ring - r0 + 1 < NR && plane - LO >= p0 &&
-                            plane - p0 + 1 < NP && spoke - LO >= q0 && spoke - q0 + 1 < NQ;
-        if (inside) {
-            const int b = ((ring - r0) * NP + (plane - p0)) * NQ + (spoke - q0);
+        const int ncell = some ? NR * NP * NQ : 0;
 #pragma unroll
-            for (int q = 0; q < NW; q++) {
-                int o;
-                if constexpr (J == 3)
-                    o = b + (q % 3 - 1) + ((q / 3) % 3 - 1) * NQ + (q / 9 - 1) * NP * NQ;
-                else
-                    o = b + ((q & 1) ? 1 : 0) + ((q & 2) ? NQ : 0) + ((q & 4) ? NP * NQ : 0);
-                if (v[q] != 0) atomicAdd((unsigned long long *)&tile[o], (unsigned long long)v[q]);
+        for (int k = 0; k < PPT; k++) {
+            int ring, plane, spoke;
+            loc3<R, J>(pos[k], a, ring, plane, spoke);
+            const bool inside = in_zone(k, ref.zone) && ring - LO >= r0 && ring - r0 + 1 < NR &&
+                                plane - LO >= p0 && plane - p0 + 1 < NP && spoke - LO >= q0 &&
+                                spoke - q0 + 1 < NQ;
+            if (inside) {
+                R w[NW];
+                weights3(pos[k], ring, plane, w);
+                long long v[NW];
+                quant_n<R, NW>(w, a.qbits, true, v);
+                const int b = ((ring - r0) * NP + (plane - p0)) * NQ + (spoke - q0);
+#pragma unroll
+                for (int q = 0; q < NW; q++) {
+                    int o;
+                    if constexpr (J == 3)
+                        o = b + (q % 3 - 1) + ((q / 3) % 3 - 1) * NQ + (q / 9 - 1) * NP * NQ;
+                    else
+                        o = b + ((q & 1) ? 1 : 0) + ((q & 2) ? NQ : 0) + ((q & 4) ? NP * NQ : 0);
+                    atomicAdd((unsigned long long *)&s.tile[o], (unsigned long long)v[q]);
+                }
+                pend &= ~(1u << k);
             }
-            pend = false;
+        }
+        // the next reference: the lowest particle index, counted from the
+        // block's middle, among the pending deposits
+        if (any_lane(pend != 0)) {
+            int myrot = INT_MAX;
+            unsigned lo = 0, hi = 0;
+#pragma unroll
+            for (int k = 0; k < PPT; k++) {
+                const int rot = (k * TB + tid - TB * PPT / 2) & (TB * PPT - 1);
+                int ring, plane, spoke;
+                loc3<R, J>(pos[k], a, ring, plane, spoke);
+                if ((pend >> k & 1u) && rot < myrot) {
+                    myrot = rot;
+                    lo = ((unsigned)plane << 13) | (unsigned)spoke;
+                    hi = ((unsigned)rot << 16) | ((dzone >> (4 * k) & 15u) << 11) | (unsigned)ring;
+                }
+            }
+            const int wmin = wave_min_i32(myrot);
+            const int fl = __ffsll((long long)__ballot(myrot == wmin)) - 1;
+            const unsigned wl = __builtin_amdgcn_readlane(lo, fl);
+            const unsigned wh = __builtin_amdgcn_readlane(hi, fl);
+            if (lane == 0) atomicMin(&s.ref[pass & 1], ((unsigned long long)wh << 32) | wl);
         }
         __syncthreads();
-        // flush: the window's cells over all threads in storage order (a
-        // row's cells are consecutive spokes, so a wave's atomics coalesce),
-        // one global atomic per non-zero cell; the (ring, plane, spoke)
-        // offsets of cell e advanced by the block size with carries instead
-        // of divided out per cell; window spokes q0 + dq lie in [-1, na],
-        // folded back onto the ring
-        if (use) {
-            const int t1 = div_small(P3_PBLOCK, NQ), sq = P3_PBLOCK - t1 * NQ;
+        // flush: the window's cells over all threads in storage order, one
+        // global atomic per non-zero cell; the (ring, plane, spoke) offsets of
+        // cell e advanced by the block size with carries instead of divided
+        // out per cell; window spokes q0 + dq lie in [-1, na]
+        if (tid < ncell) {
+            const int t1 = div_small(TB, NQ), sq = TB - t1 * NQ;
             const int sr = div_small(t1, NP), spl = t1 - sr * NP;
             const int u1 = div_small(tid, NQ);
             int dq = tid - u1 * NQ, dr = div_small(u1, NP);
             int dp = u1 - dr * NP;
-            for (int e = tid; e < ncell; e += P3_PBLOCK) {
-                const long long tv = tile[e];
+            for (int e = tid; e < ncell; e += TB) {
+                const long long tv = s.tile[e];
                 if (tv != 0) {
+                    s.tile[e] = 0;
                     int sp = q0 + dq;
                     sp = sp >= a.na ? sp - a.na : sp < 0 ? sp + a.na : sp;
-                    atomicAdd((unsigned long long *)&a.mfx[tz - 1][((r0 + dr) * a.ngz + (p0 + dp)) * a.na + sp],
+                    atomicAdd((unsigned long long *)&a.mfx[ref.zone - 1][((r0 + dr) * a.ngz + (p0 + dp)) * a.na + sp],
                               (unsigned long long)tv);
                 }
                 dq += sq;
@@ -458,106 +516,155 @@ __device__ __forceinline__ void deposit3_block(const P3Args<R> &a, bool on, int 
                 dr += sr + c2;
             }
         }
-        if (pass + 1 >= P3_PASSES) {
-            direct = direct || pend;
-            break;
-        }
-        // every thread reads the flag of the same barrier: a uniform exit
-        if (!__syncthreads_or(pend ? 1 : 0)) break;
+        const unsigned long long kref = s.ref[pass & 1];
+        if (kref == ~0ull || pass + 1 >= P3_PASSES) break;   // uniform
+        const unsigned rh = (unsigned)(kref >> 32), rl = (unsigned)kref;
+        ref.zone = (int)((rh >> 11) & 0xF);
+        ref.ring = (int)(rh & 0x7FF);
+        ref.plane = (int)(rl >> 13);
+        ref.spoke = (int)(rl & 0x1FFF);
     }
-    if (direct) {
-        int ic[NW];
-        cornersJ<J>(c, spoke, a.na, a.ngz, ic);
+    direct |= pend;
+    if (any_lane(direct != 0)) {
 #pragma unroll
-        for (int q = 0; q < NW; q++)
-            if (v[q] != 0) deposit_global(a.mfx, a.nz, a.mesh, z, ic[q], v[q]);
+        for (int k = 0; k < PPT; k++) {
+            if (!(direct >> k & 1u)) continue;
+            const int z = (int)(dzone >> (4 * k) & 15u);
+            int ring, plane, spoke;
+            loc3<R, J>(pos[k], a, ring, plane, spoke);
+            R w[NW];
+            weights3(pos[k], ring, plane, w);
+            long long v[NW];
+            quant_n<R, NW>(w, a.qbits, true, v);
+            atomicMin(&s.jr[z - 1], ring);
+            atomicMax(&s.kr[z - 1], ring);
+            int ic[NW];
+            cornersJ<J>(cell_index(a, ring, plane, spoke), spoke, a.na, a.ngz, ic);
+#pragma unroll
+            for (int q = 0; q < NW; q++)
+                if (v[q] != 0) deposit_global(a.mfx, a.nz, a.mesh, z, ic[q], v[q]);
+        }
     }
 }
 
 // jrad/krad from the block's central rings: 1-based rings j+1..j+2 about a
 // central ring j (massgn.f:146-149), j..j+2 for jmass 3 (massgn.f:176-179)
-__device__ __forceinline__ void flush_ranges(int nz, int nr, int lo, const int *s_jr,
-                                             const int *s_kr, int *jrad, int *krad,
-                                             int rstride) {
+template <int TILE>
+__device__ __forceinline__ void deposit3_ranges(const Deposit3Lds<TILE> &s, int nz, int nr, int lo,
+                                                int *jrad, int *krad, int rstride) {
     const int tid = threadIdx.x;
-    if (tid < nz && s_kr[tid] >= 0) {
-        const int k = s_kr[tid] + 2;
-        widen_range(jrad, krad, rstride, blockIdx.x, tid + 1, s_jr[tid] + 1 - lo, k < nr ? k : nr);
+    if (tid < nz && s.kr[tid] >= 0) {
+        const int k = s.kr[tid] + 2;
+        widen_range(jrad, krad, rstride, blockIdx.x, tid + 1, s.jr[tid] + 1 - lo, k < nr ? k : nr);
     }
 }
 
 template <typename R, int J>
-__global__ __launch_bounds__(P3_PBLOCK) void p3_massgn_kernel(P3Args<R> a) {
-    __shared__ int s_jr[GH_MAXZ], s_kr[GH_MAXZ], s_b[P3_SB];
-    __shared__ unsigned long long s_ref[2];
-    __shared__ long long tile[P3_TILE];
+__global__ __launch_bounds__((P3Shape<R, J>::block), (P3Shape<R, J>::waves)) void p3_massgn_kernel(P3Args<R> a) {
+    constexpr int TB = P3Shape<R, J>::block, PPT = P3Shape<R, J>::ppt, TILE = P3Shape<R, J>::tile;
+    __shared__ Deposit3Lds<TILE> s_dep;
+    __shared__ P3Ref s_ref0;
     const int tid = threadIdx.x;
-    if (tid < GH_MAXZ) {
-        s_jr[tid] = INT_MAX;
-        s_kr[tid] = -1;
-    }
-    if (tid == 0) s_b[0] = INT_MAX;
-    __syncthreads();
-    const long long i = (long long)blockIdx.x * P3_PBLOCK + tid;
-    bool on = false;
-    int z = 0, c = 0, rg = 0, pl = 0, sp = 0;
-    R w[P3NW<J>::v];
-    if (i < a.n) {
-        z = a.zone[i];
-        const typename Vec4<R>::T p = a.rec[2 * i];
-        R u, t;
-        ut3(p.x, p.y, a, u, t);
-        p3_set_ut(a, i, u, t);
-        if (z >= 1 && z <= a.nz) {
-            c = cellJ<R, J>(u, t, p.z, a, a.nsect > 1, w, rg, pl, sp);
-            on = true;
+    const long long base = (long long)blockIdx.x * (TB * PPT);
+    const int nblk = (int)min((long long)(TB * PPT), a.n - base);
+    P3Pos<R> pos[PPT];
+    unsigned dzone = 0;
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        const int j = k * TB + tid;
+        pos[k].u = pos[k].t = pos[k].zz = (R)0;
+        if (j < nblk) {
+            const int z = a.zone[base + j];
+            const typename Vec4<R>::T p = a.rec[2 * (base + j)];
+            R u, t;
+            ut3(p.x, p.y, a, u, t);
+            p3_set_ut(a, base + j, u, t);
+            if (z >= 1 && z <= a.nz) {
+                pos[k] = pos3(u, t, p.z, a, a.nsect > 1);
+                dzone |= (unsigned)z << (4 * k);
+            }
+        }
+        if (j == nblk >> 1) {
+            s_ref0.zone = max(1, (int)(dzone >> (4 * k) & 15u));
+            loc3<R, J>(pos[k], a, s_ref0.ring, s_ref0.plane, s_ref0.spoke);
         }
     }
-    deposit3_block<R, J>(a, on, z, c, rg, pl, sp, w, tile, s_b, s_ref, s_jr, s_kr);
+    deposit3_init<TB>(s_dep);
     __syncthreads();
-    flush_ranges(a.nz, a.nr, J == 3 ? 1 : 0, s_jr, s_kr, a.jrad, a.krad, a.rstride);
+    const P3Ref ref = s_ref0;
+    deposit3_block<R, J, PPT, TB>(a, s_dep, pos, dzone, ref);
+    __syncthreads();
+    deposit3_ranges(s_dep, a.nz, a.nr, J == 3 ? 1 : 0, a.jrad, a.krad, a.rstride);
 }
 
 template <typename R, int J>
-__global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
+__global__ __launch_bounds__((P3Shape<R, J>::block), (P3Shape<R, J>::waves)) void p3_push_kernel(P3Args<R> a) {
     typedef typename Vec4<R>::T R4;
-    typedef typename Vec2<R>::T R2;
-    __shared__ int s_jr[GH_MAXZ], s_kr[GH_MAXZ], s_b[P3_SB];
-    __shared__ unsigned long long s_ref[2];
+    constexpr int TB = P3Shape<R, J>::block, PPT = P3Shape<R, J>::ppt, TILE = P3Shape<R, J>::tile;
+    __shared__ Deposit3Lds<TILE> s_dep;
     __shared__ int s_dn, s_np;
-    __shared__ long long tile[P3_TILE];
     __shared__ double s_tab[UtTab<R>::n];
-    const int tid = threadIdx.x;
-    if (tid < GH_MAXZ) {
-        s_jr[tid] = INT_MAX;
-        s_kr[tid] = -1;
+    const int tid = threadIdx.x, nz = a.nz, nlists = nz + 1;
+    const long long base = (long long)blockIdx.x * (TB * PPT);
+    const int nblk = (int)min((long long)(TB * PPT), a.n - base);
+    R4 *const rec = a.rec + 2 * base;
+    uint8_t *const zb = a.zone + base;
+    // on a full step every list moves: no wait for the zones before the load
+    const bool full = a.mzone == nz;
+    int zin[PPT];
+    R4 st[PPT], sv[PPT];   // (x, y, z, vx), (vy, vz, u, t)
+#pragma unroll
+    for (int k = 0; k < PPT; k++) zin[k] = zb[min(k * TB + tid, nblk - 1)];
+    const int zmid = zb[nblk >> 1];
+    const R4 m0 = rec[2 * (nblk >> 1)], m1 = rec[2 * (nblk >> 1) + 1];
+    auto load_state = [&]() {
+#pragma unroll
+        for (int k = 0; k < PPT; k++) {
+            const int j = min(k * TB + tid, nblk - 1);
+            st[k] = rec[2 * j];
+            sv[k] = rec[2 * j + 1];
+        }
+    };
+    if (full) load_state();
+    for (int j = tid; j < UtTab<R>::n; j += TB) s_tab[j] = ut_tab_entry<R>(j);
+    deposit3_init<TB>(s_dep);
+    if (tid == 0) s_dn = s_np = 0;
+    unsigned mv = 0;   // bit k: particle k moves
+    if (!full)
+#pragma unroll
+        for (int k = 0; k < PPT; k++)
+            if (k * TB + tid < nblk && zin[k] <= a.mzone) mv |= 1u << k;
+    if (!__syncthreads_or(full ? 1 : (int)mv)) return;
+    if (full) {
+#pragma unroll
+        for (int k = 0; k < PPT; k++)
+            if (k * TB + tid < nblk && (zin[k] != nlists || a.offanal)) mv |= 1u << k;
+    } else {
+        load_state();
     }
-    if (tid == 0) {
-        s_dn = s_np = 0;
-        s_b[0] = INT_MAX;
-    }
-    if (tid < UtTab<R>::n) s_tab[tid] = ut_tab_entry<R>(tid);
-    __syncthreads();
-    const long long i = (long long)blockIdx.x * P3_PBLOCK + tid;
-    int dn = 0, np = 0;
-    bool don = false;
-    int dz = 0, dc = 0, drg = 0, dpl = 0, dsp = 0;
-    R dw[P3NW<J>::v];
-    if (i < a.n) {
-        const int nz = a.nz, nlists = nz + 1;
-        const int z0 = a.zone[i];
-        const bool offlist = z0 == nlists;
-        const bool move = offlist ? (a.offanal && a.mzone == nz) : z0 <= a.mzone;
+    P3Ref ref;
+    ref.zone = min(max(zmid, 1), nz);
+    loc3<R, J>(pos3(m1.z, m1.w, m0.z, a, a.nsect > 1), a, ref.ring, ref.plane, ref.spoke);
+    ref.ring = max(ref.ring, 0);
+    ref.spoke = min(max(ref.spoke, 0), a.na);
+    // the new states take the old ones' registers and are stored after every
+    // load has been used
+    P3Pos<R> pos[PPT];
+    unsigned dzone = 0, zch = 0;
+    int np = 0, nplus = 0, nminus = 0;
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        bool plus = false, minus = false;
+        const bool move = mv >> k & 1u;
+        np += __popcll(__ballot(move));
+        pos[k].u = pos[k].t = pos[k].zz = (R)0;
         if (move) {
-            np = 1;
-            const R4 p = a.rec[2 * i];
-            const R4 q4 = a.rec[2 * i + 1];
-            const R2 q = mk2(q4.x, q4.y);
-            const R2 ut0 = mk2(q4.z, q4.w);
-            R o[3] = {p.x, p.y, p.z};
-            R ov[3] = {p.w, q.x, q.y};
+            const int z0 = zin[k];
+            const bool offlist = z0 == nlists;
+            R o[3] = {st[k].x, st[k].y, st[k].z};
+            R ov[3] = {st[k].w, sv[k].x, sv[k].y};
             R acc[3], nv[3], nx[3];
-            getacc3<R, J>(a, o[0], o[1], o[2], ut0.x, ut0.y, z0, acc);
+            getacc3<R, J>(a, o[0], o[1], o[2], sv[k].z, sv[k].w, z0, acc);
             // stpgrp
 #pragma unroll
             for (int d = 0; d < 3; d++) {
@@ -565,22 +672,22 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
                 nx[d] = o[d] + nv[d];
             }
             int znew = z0;
-            const R nx0 = nx[0], nx1 = nx[1];
-            R rnew = sqrt_rn(nx0 * nx0 + nx1 * nx1);
+            R rnew = sqrt_rn(nx[0] * nx[0] + nx[1] * nx[1]);
             const R az = nx[2] < (R)0 ? -nx[2] : nx[2];
             const bool off = (az > a.zm) || (rnew > a.rgrid);
             if (!offlist) {
                 if (off) {
                     znew = nlists;
-                    dn = 1;
+                    plus = true;
                     if (a.offanal && z0 < nz) {
                         const R tfac = tsfac3(a, nz) / tsfac3(a, z0);
 #pragma unroll
                         for (int d = 0; d < 3; d++) chstep1(tfac, o[d], ov[d], acc[d], nx[d], nv[d]);
+                        rnew = sqrt(nx[0] * nx[0] + nx[1] * nx[1]);
                     }
                 }
             } else if (!off) {
-                dn = -1;
+                minus = true;
                 znew = nz;
             }
             // rezgrp
@@ -592,32 +699,41 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_push_kernel(P3Args<R> a) {
                     const R tfac = tsfac3(a, kz) / tsfac3(a, znew);
 #pragma unroll
                     for (int d = 0; d < 3; d++) chstep1(tfac, o[d], ov[d], acc[d], nx[d], nv[d]);
+                    rnew = sqrt(nx[0] * nx[0] + nx[1] * nx[1]);
                     znew = kz;
                 }
             }
             R un, tn;
-            if (nx0 != nx[0] || nx1 != nx[1]) rnew = sqrt_rn(nx[0] * nx[0] + nx[1] * nx[1]);
             ut3_push(nx[0], nx[1], rnew, a, un, tn, s_tab);
-            a.rec[2 * i] = mk4(nx[0], nx[1], nx[2], nv[0]);
-            a.rec[2 * i + 1] = mk4(nv[1], nv[2], un, tn);
-            a.zone[i] = (uint8_t)znew;
+            st[k] = mk4(nx[0], nx[1], nx[2], nv[0]);
+            sv[k] = mk4(nv[1], nv[2], un, tn);
+            if (znew != z0) zch |= 1u << k;
+            zin[k] = znew;
             if (znew >= 1 && znew <= nz) {
-                dc = cellJ<R, J>(un, tn, nx[2], a, a.nsect > 1, dw, drg, dpl, dsp);
-                dz = znew;
-                don = true;
+                pos[k] = pos3(un, tn, nx[2], a, a.nsect > 1);
+                dzone |= (unsigned)znew << (4 * k);
             }
         }
+        nplus += __popcll(__ballot(plus));
+        nminus += __popcll(__ballot(minus));
     }
-    deposit3_block<R, J>(a, don, dz, dc, drg, dpl, dsp, dw, tile, s_b, s_ref, s_jr, s_kr);
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        const int j = k * TB + tid;
+        if (mv >> k & 1u) {
+            rec[2 * j] = st[k];
+            rec[2 * j + 1] = sv[k];
+            if (zch >> k & 1u) zb[j] = (uint8_t)zin[k];
+        }
+    }
     // block sums of the off-grid change and the pushes
-    dn = wave_sum_i32(dn);
-    np = wave_sum_i32(np);
     if ((tid & 63) == 0) {
-        if (dn) atomicAdd(&s_dn, dn);
+        if (nplus != nminus) atomicAdd(&s_dn, nplus - nminus);
         if (np) atomicAdd(&s_np, np);
     }
+    deposit3_block<R, J, PPT, TB>(a, s_dep, pos, dzone, ref);
     __syncthreads();
-    flush_ranges(a.nz, a.nr, J == 3 ? 1 : 0, s_jr, s_kr, a.jrad, a.krad, a.rstride);
+    deposit3_ranges(s_dep, nz, a.nr, J == 3 ? 1 : 0, a.jrad, a.krad, a.rstride);
     if (tid == 0) {
         if (s_dn) atomicAdd((unsigned long long *)&a.counters[0], (unsigned long long)(long long)s_dn);
         count_pushes(a.pushes, blockIdx.x, s_np);
@@ -788,8 +904,9 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_key_kernel(P3Args<R> a, int kshi
         const typename Vec4<R>::T p = a.rec[2 * i];
         const typename Vec4<R>::T q = a.rec[2 * i + 1];
         const typename Vec2<R>::T ut = mk2(q.z, q.w);
-        R w[P3NW<J>::v];
-        k = (unsigned)(cellJ<R, J>(ut.x, ut.y, p.z, a, false, w) >> kshift);
+        int ring, plane, spoke;
+        loc3<R, J>(pos3(ut.x, ut.y, p.z, a, false), a, ring, plane, spoke);
+        k = (unsigned)(cell_index(a, ring, plane, spoke) >> kshift);
     }
     key[i] = k;
     perm[i] = (unsigned)i;
@@ -1245,22 +1362,30 @@ __global__ __launch_bounds__(GREEN3_BLOCK) void p3_green_kernel(
 // ---- launchers ------------------------------------------------------------------------
 
 static unsigned p3_blocks(long long n) { return (unsigned)((n + P3_PBLOCK - 1) / P3_PBLOCK); }
+template <typename R, int J> static dim3 p3_grid(long long n) {
+    const int per = P3Shape<R, J>::block * P3Shape<R, J>::ppt;
+    return dim3((unsigned)((n + per - 1) / per));
+}
 
 template <typename R> hipError_t launch_p3_massgn(const P3Args<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
     if (a.jmass == 3)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, 3>), dim3(p3_blocks(a.n)), dim3(P3_PBLOCK), 0, s, a);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, 3>), (p3_grid<R, 3>(a.n)),
+                           dim3(P3Shape<R, 3>::block), 0, s, a);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, 2>), dim3(p3_blocks(a.n)), dim3(P3_PBLOCK), 0, s, a);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, 2>), (p3_grid<R, 2>(a.n)),
+                           dim3(P3Shape<R, 2>::block), 0, s, a);
     return hipGetLastError();
 }
 
 template <typename R> hipError_t launch_p3_push(const P3Args<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
     if (a.jmass == 3)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, 3>), dim3(p3_blocks(a.n)), dim3(P3_PBLOCK), 0, s, a);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, 3>), (p3_grid<R, 3>(a.n)),
+                           dim3(P3Shape<R, 3>::block), 0, s, a);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, 2>), dim3(p3_blocks(a.n)), dim3(P3_PBLOCK), 0, s, a);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, 2>), (p3_grid<R, 2>(a.n)),
+                           dim3(P3Shape<R, 2>::block), 0, s, a);
     return hipGetLastError();
 }
 

@@ -56,18 +56,9 @@ template <typename R, bool COMP, int PPT> struct PushShape {
 constexpr int PUSH_PASSES = 8;         // deposit window passes before global atomics
 constexpr int CLIP_RINGS = 16;          // rings of a window that had to be clipped
 
-// step ratio of list iz: the first three by selection between uniform values
-// (an indexed read of the argument block is a load, and a load after the
-// particle stores waits for them)
 template <typename R>
 __device__ __forceinline__ R tsfac(const PushArgs<R> &a, int iz) {
-    const int i = iz < a.nz ? iz : a.nz;
-    int n = i == 1 ? a.nstep[0] : i == 2 ? a.nstep[1] : a.nstep[2];
-    if (a.nz > 3) {
-        for (int q = 4; q <= a.nz; q++)
-            if (i == q) n = a.nstep[q - 1];
-    }
-    return (R)n;
+    return (R)step_ratio(a.nstep, a.nz, iz);
 }
 
 // zoneno for a position of known radius (zoneno.f:40-55)

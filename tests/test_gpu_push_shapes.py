@@ -47,6 +47,22 @@ def test_run_masses_equal_masset(n, nr, na, prec, comp):
     g.close()
 
 
+@pytest.mark.parametrize("n,nr,na,ngz", [(1, 24, 64, 16), (511, 24, 64, 16), (513, 64, 128, 45),
+                                          (30_000, 90, 128, 61), (600_123, 40, 90, 31)])
+@pytest.mark.parametrize("prec,jmass", [("fp32", 2), ("fp64", 2), ("fp32", 3)])
+def test_run_masses_equal_masset_p3d(n, nr, na, ngz, prec, jmass):
+    from galaxy_amd.lib15 import P3DGrid
+    print("[case] masses p3d", n, nr, na, ngz, prec, jmass, flush=True)
+    w = configs.Workload3("p3d-shapes", nr=nr, na=na, hash=2, n=n, steps=1, dt=0.05, ngz=ngz,
+                          dz_model=0.08, eps_model=0.2, seed=8)
+    g = P3DGrid(precision=prec, jmass=jmass, **configs.grid_kwargs3(w))
+    g.greenm()
+    g.restrt(*configs.particles3(w, None, None, g.rgrid))
+    g.masset()
+    _check(g, 4)
+    g.close()
+
+
 def test_ensemble_equals_lone_discs_across_shapes():
     """Three members of 6e5 particles (four per thread together) against the
     same discs alone (one per thread)."""
