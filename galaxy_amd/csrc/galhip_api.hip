@@ -206,6 +206,7 @@ static int p2d_create(const galhip_p2d_params *p, int nmem, const double *pmass,
     rc |= dalloc(&c->ranges, sizeof(int) * 4 * nm);
     rc |= dalloc(&c->lg_d, sizeof(int) * c->mmax);
     rc |= dalloc(&c->counters, sizeof(long long) * 4 * nm);
+    rc |= dalloc(&c->load_chk, sizeof(long long) * 4 * (nm + 1));
     rc |= dalloc(&c->push_cnt, sizeof(long long) * 8 * GH_PUSH_STRIPES);
     rc |= dalloc(&c->rho, es * cells);
     rc |= dalloc(&c->coef, es * c->ncoef * c->nr * nm);
@@ -285,7 +286,7 @@ extern "C" int galhip_free(galhip_ctx *c) {
     if (c->p3d) p3_free(c);
     free_particles(c);
     for (int z = 0; z < GH_MAXZ; z++) { dfree(c->mfx[z]); dfree(c->moz[z]); }
-    dfree(c->jrad); dfree(c->krad); dfree(c->ranges); dfree(c->lg_d); dfree(c->counters);
+    dfree(c->jrad); dfree(c->krad); dfree(c->ranges); dfree(c->lg_d); dfree(c->counters); dfree(c->load_chk);
     dfree(c->push_cnt);
     dfree(c->fp_c);
     dfree(c->rho); dfree(c->coef); dfree(c->fld2); dfree(c->pot); dfree(c->tw); dfree(c->twd);
@@ -528,8 +529,11 @@ static int load_xv(galhip_ctx *c, long long n, const void *x, const void *y, con
     const size_t es = esize(c);
     unsigned char *stage = (unsigned char *)c->xv2;
     const void *src[4] = {x, y, vx, vy};
+    CopySegment seg[4];
     for (int k = 0; k < 4; k++)
-        HIPCHK(hipMemcpy(stage + k * es * n, src[k], es * n, hipMemcpyHostToDevice));
+        seg[k] = {(void *)src[k], stage + k * es * n, es * (size_t)n};
+    int rc = copy_segments(c, seg, 4, false);
+    if (rc) return rc;
     if (c->prec == GALHIP_FP32)
         HIPCHK(launch_interleave<float>((const float *)stage, (float4 *)c->xv, c->id, n, c->s));
     else
@@ -550,23 +554,14 @@ extern "C" int galhip_restrt(galhip_ctx *c, int64_t n, const void *x,
     int rc = ensure_particles(c, n);
     if (rc) return rc;
     size_t es = esize(c);
-    std::vector<uint8_t> z(n);
-    long long cnt[4] = {0, 0, 0, 0};   // counters: [0] noff
-    for (long long i = 0; i < n; i++) {
-        int v = iz[i];
-        if (v < 1 || v > c->nz + 1)
-            return gh_fail(GALHIP_EINVAL, "particle %lld has zone %d outside 1..%d", i, v, c->nz + 1);
-        z[i] = (uint8_t)v;
-        if (v == c->nz + 1) cnt[0]++;    // /admin/ noff: the off-grid list
-    }
-    HIPCHK(hipMemcpy(c->counters, cnt, sizeof cnt, hipMemcpyHostToDevice));
+    rc = load_zones(c, n, iz);
+    if (rc) return rc;
     HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     c->qbits = qbits_for(n);
     c->order_ver++;
     if (n == 0) return 0;
     rc = load_xv(c, n, x, y, vx, vy);
     if (rc) return rc;
-    HIPCHK(hipMemcpy(c->zone, z.data(), n, hipMemcpyHostToDevice));
     if (c->xlo) HIPCHK(hipMemset(c->xlo, 0, 2 * es * n));
     c->qbits = qbits_for(n);
     rc = compute_ut(c);
@@ -595,7 +590,6 @@ static int unload_all(galhip_ctx *c, void *x, void *y, void *vx, void *vy, int32
     if (n <= 0) return 0;
     // planar, in load order, into the second particle buffer and the sort
     // keys (both free outside a sort), then straight to the caller's arrays
-    void *dst[4] = {x, y, vx, vy};
     const size_t es = esize(c);
     unsigned char *stage = (unsigned char *)c->xv2;
     int *zs = (int *)c->key;
@@ -605,11 +599,12 @@ static int unload_all(galhip_ctx *c, void *x, void *y, void *vx, void *vy, int32
     else
         HIPCHK(launch_deinterleave<double>((const double4 *)c->xv, c->zone, c->id,
                                            (double *)stage, zs, n, c->s));
-    HIPCHK(hipStreamSynchronize(c->s));
-    for (int k = 0; k < 4; k++)
-        if (dst[k]) HIPCHK(hipMemcpy(dst[k], stage + k * es * n, es * n, hipMemcpyDeviceToHost));
-    if (iz) HIPCHK(hipMemcpy(iz, zs, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    return 0;
+    const CopySegment seg[5] = {{x, stage, es * n},
+                                {y, stage + es * n, es * n},
+                                {vx, stage + 2 * es * n, es * n},
+                                {vy, stage + 3 * es * n, es * n},
+                                {iz, zs, sizeof(int32_t) * n}};
+    return copy_segments(c, seg, 5, true);
 }
 
 // ---- zone bookkeeping (host) -----------------------------------------------------
@@ -1668,23 +1663,13 @@ extern "C" int galhip_ens_restrt(galhip_ctx *c, const int64_t *count, const void
         HIPCHK(hipMemcpy(c->blk_d, blk.data(), sizeof(int4) * blk.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->m_qbits_d, c->m_qbits.data(), sizeof(int) * c->nmem, hipMemcpyHostToDevice));
     size_t es = esize(c);
-    std::vector<uint8_t> z(n);
-    std::vector<long long> cnt(4 * (size_t)c->nmem, 0);   // per member: [0] noff
-    for (int m = 0; m < c->nmem; m++)
-        for (long long i = c->m_off[m]; i < c->m_off[m + 1]; i++) {
-            int v = iz[i];
-            if (v < 1 || v > c->nz + 1)
-                return gh_fail(GALHIP_EINVAL, "particle %lld has zone %d outside 1..%d", i, v, c->nz + 1);
-            z[i] = (uint8_t)v;
-            if (v == c->nz + 1) cnt[4 * m]++;
-        }
-    HIPCHK(hipMemcpy(c->counters, cnt.data(), sizeof(long long) * cnt.size(), hipMemcpyHostToDevice));
+    rc = load_zones(c, n, iz);
+    if (rc) return rc;
     HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     drop_graphs(c);
     if (n == 0) return 0;
     rc = load_xv(c, n, x, y, vx, vy);
     if (rc) return rc;
-    HIPCHK(hipMemcpy(c->zone, z.data(), n, hipMemcpyHostToDevice));
     if (c->xlo) HIPCHK(hipMemset(c->xlo, 0, 2 * es * n));
     rc = compute_ut(c);
     if (rc) return rc;
@@ -1794,14 +1779,9 @@ extern "C" int galhip_get_position_lo(const galhip_ctx *c, void *xlo, void *ylo)
         memset(ylo, 0, es * n);
         return 0;
     }
-    std::vector<unsigned> ids(n);
-    std::vector<float> lo(2 * n);
-    HIPCHK(hipMemcpy(ids.data(), c->id, sizeof(unsigned) * n, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(lo.data(), c->xlo, sizeof(float) * 2 * n, hipMemcpyDeviceToHost));
-    float *xo = (float *)xlo, *yo = (float *)ylo;
-    for (long long i = 0; i < n; i++) {
-        xo[ids[i]] = lo[2 * i];
-        yo[ids[i]] = lo[2 * i + 1];
-    }
-    return 0;
+    // through the second buffer (free outside a sort), planar in load order
+    float *stage = (float *)c->xlo2;
+    HIPCHK(launch_planar_lo((const float2 *)c->xlo, c->id, stage, n, c->s));
+    const CopySegment seg[2] = {{xlo, stage, es * n}, {ylo, stage + n, es * n}};
+    return copy_segments(c, seg, 2, true);
 }

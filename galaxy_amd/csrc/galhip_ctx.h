@@ -18,7 +18,22 @@ int gh_fail(int code, const char *fmt, ...);
                         hipGetErrorString(e_), __FILE__, __LINE__);           \
     } while (0)
 
+// Copies of particle arrays (galhip_copy.hip)
+struct CopySegment {
+    void *host, *dev;   // a null host pointer skips the segment
+    size_t bytes;
+};
+
+// Every context is a user of the pinned buffers that the copies share.
+struct CopyUser {
+    CopyUser();
+    ~CopyUser();
+    CopyUser(const CopyUser &) = delete;
+    CopyUser &operator=(const CopyUser &) = delete;
+};
+
 struct galhip_ctx {
+    CopyUser copy_user;
     int prec;
     int nr, na, ng, mmax, nsect, mesh, tsoft, nz, offanal;
     int nstep[GH_MAXZ];
@@ -51,6 +66,7 @@ struct galhip_ctx {
     int *jrad, *krad, *ranges, *lg_d;   // ring ranges in stripes (widen_range)
     int rstride;
     long long *counters;              // [0] off-grid count (per grid)
+    long long *load_chk;              // zone_load_kernel: [0] first bad index, 4 m + 4 noff
     long long *push_cnt;              // pushes, striped (count_pushes)
     void *rho, *coef, *fld2, *pot, *G, *tw;
     double *Gd, *twd;
@@ -181,8 +197,11 @@ void set_mzone(galhip_ctx *c);
 void masscl_host(galhip_ctx *c, bool normal);
 int zoncmb_host(galhip_ctx *c);
 hipEvent_t take_event(galhip_ctx *c);
+int copy_segments(const galhip_ctx *c, const CopySegment *seg, int nseg, bool to_host);
+int load_zones(galhip_ctx *c, long long n, const int32_t *iz);
 
 namespace gh {
+hipError_t launch_planar_lo(const float2 *, const unsigned *, float *, long long, hipStream_t);
 hipError_t launch_d2f(const double *, float *, long long, hipStream_t);
 hipError_t launch_fill_i64(long long *, long long, long long, hipStream_t);
 hipError_t launch_fill_i32(int *, int, long long, hipStream_t);

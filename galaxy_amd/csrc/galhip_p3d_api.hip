@@ -146,6 +146,7 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
     rc |= dalloc(&c->slot_p_d, sizeof(int) * (nm > 0 ? nm : 1));
     rc |= dalloc(&c->slot_of_d, sizeof(int) * c->mmax);
     rc |= dalloc(&c->counters, sizeof(long long) * 4);
+    rc |= dalloc(&c->load_chk, sizeof(long long) * 8);
     rc |= dalloc(&c->push_cnt, sizeof(long long) * 8 * GH_PUSH_STRIPES);
     rc |= dalloc(&c->rho, es * c->mesh);
     rc |= dalloc(&c->A3, es * c->nr * nm * c->ngz);
@@ -300,34 +301,25 @@ extern "C" int galhip_restrt3(galhip_ctx *c, int64_t n, const void *x, const voi
     int rc = p3_ensure(c, n);
     if (rc) return rc;
     const size_t es = esize(c);
-    std::vector<uint8_t> zz(n);
-    long long cnt[4] = {0, 0, 0, 0};
-    for (long long i = 0; i < n; i++) {
-        const int v = iz[i];
-        if (v < 1 || v > c->nz + 1)
-            return gh_fail(GALHIP_EINVAL, "particle %lld has zone %d outside 1..%d", i, v, c->nz + 1);
-        zz[i] = (uint8_t)v;
-        if (v == c->nz + 1) cnt[0]++;
-    }
-    HIPCHK(hipMemcpy(c->counters, cnt, sizeof cnt, hipMemcpyHostToDevice));
+    rc = load_zones(c, n, iz);
+    if (rc) return rc;
     HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     if (n > 0) {
         // the planar arrays through the second record buffer (free outside a
         // sort, 8 n values), interleaved on the device
         unsigned char *t4 = (unsigned char *)c->xv2, *t2 = t4 + 4 * es * n;
-        const void *s4[4] = {x, y, z, vx};
-        const void *s2[2] = {vy, vz};
-        for (int k = 0; k < 4; k++)
-            HIPCHK(hipMemcpy(t4 + k * es * n, s4[k], es * n, hipMemcpyHostToDevice));
-        for (int k = 0; k < 2; k++)
-            HIPCHK(hipMemcpy(t2 + k * es * n, s2[k], es * n, hipMemcpyHostToDevice));
+        const void *src[6] = {x, y, z, vx, vy, vz};
+        CopySegment seg[6];
+        for (int k = 0; k < 6; k++)
+            seg[k] = {(void *)src[k], t4 + k * es * n, es * (size_t)n};
+        rc = copy_segments(c, seg, 6, false);
+        if (rc) return rc;
         if (c->prec == GALHIP_FP32)
             HIPCHK(launch_p3_interleave<float>((const float *)t4, (const float *)t2,
                                                (float4 *)c->xv, c->id, n, c->s));
         else
             HIPCHK(launch_p3_interleave<double>((const double *)t4, (const double *)t2,
                                                 (double4 *)c->xv, c->id, n, c->s));
-        HIPCHK(hipMemcpy(c->zone, zz.data(), n, hipMemcpyHostToDevice));
     }
     c->qbits = qbits_for(n);
     if (c->prec == GALHIP_FP32) HIPCHK(launch_p3_ut<float>(p3_args<float>(c), c->s));
@@ -356,15 +348,11 @@ extern "C" int galhip_unload3(galhip_ctx *c, void *x, void *y, void *z, void *vx
     else
         HIPCHK(launch_p3_deinterleave<double>((const double4 *)c->xv, c->zone, c->id,
                                               (double *)t4, (double *)t2, zs, n, c->s));
-    HIPCHK(hipStreamSynchronize(c->s));
-    void *d4[4] = {x, y, z, vx};
-    void *d2[2] = {vy, vz};
-    for (int k = 0; k < 4; k++)
-        if (d4[k]) HIPCHK(hipMemcpy(d4[k], t4 + k * es * n, es * n, hipMemcpyDeviceToHost));
-    for (int k = 0; k < 2; k++)
-        if (d2[k]) HIPCHK(hipMemcpy(d2[k], t2 + k * es * n, es * n, hipMemcpyDeviceToHost));
-    if (iz) HIPCHK(hipMemcpy(iz, zs, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    return 0;
+    void *dst[6] = {x, y, z, vx, vy, vz};
+    CopySegment seg[7];
+    for (int k = 0; k < 6; k++) seg[k] = {dst[k], t4 + k * es * n, es * (size_t)n};
+    seg[6] = {iz, zs, sizeof(int32_t) * (size_t)n};
+    return copy_segments(c, seg, 7, true);
 }
 
 // Regroup the particles by cell (the storage order sets the locality of the
