@@ -47,8 +47,8 @@ template <typename R> struct P3SolveArgs {
     int *jrad, *krad, rstride, *ranges;
     R *rho;          // [mesh] combined, scaled mass
     R *A;            // [nr][nm][ngz] azimuthal components per plane
-    R *M;            // [nr][nm][2 ngz] after the vertical transform
-    R *W;            // [4][nr][nm][2 ngz] contracted
+    R *M;            // [nm][2 ngz][nr] after the vertical transform
+    R *W;            // [4][nm][2 ngz][nr] contracted
     R *Z;            // [4][nr][ngz][nm] after the inverse vertical transform
     const R *G;      // [4][ngz+1][ng][nr(source)][nr(field)]
     const R *tw;     // [na][2] cos, sin of 2 pi k / na

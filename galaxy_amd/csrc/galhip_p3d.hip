@@ -15,22 +15,23 @@
 //   p3_tmcent_kernel  tmcent's half-step velocity shift
 //   p3_gather_kernel  weight / grdacc for given positions (parity checks)
 // Solve (p3fndf.f:37-104), FP32 or FP64:
-//   p3_analyse_kernel block (plane, ring): zoncmb + scaled, then the
+//   p3_analyse_kernel wavefront per (planes, ring): zoncmb + scaled, then the
 //                     azimuthal components of the active harmonics
 //                     (p3manl.f:60-89) as direct sums
-//   p3_zfwd_kernel    block per ring: the doubled vertical transform of each
+//   p3_zfwd_kernel    block per (columns, ring): the doubled vertical transform of each
 //                     component column, zero-padded to 2 ngz (p3manl.f:90-101)
 //   p3_conv_kernel    block per (type, k_z, m): the radial contraction with
 //                     that Green's matrix (p3conv.f:139-226); table streamed
 //                     once, field ring per thread
-//   p3_zinv_kernel    block per (type, ring): inverse vertical transform,
+//   p3_zinv_kernel    block per (columns, type, ring): inverse vertical transform,
 //                     first ngz planes (p3fsyn.f:59-91)
-//   p3_synth_kernel   block per (plane, ring): inverse azimuthal transform,
+//   p3_synth_kernel   block per (planes, ring): inverse azimuthal transform,
 //                     1/(2 ngz na) (p3fsyn.f:92-129) and polcat
 // p3_green_kernel: p3grnm's tables in FP64 (p3grnm.f:93-263), p3gwrt's
 //   per-(k_z, m) matrices with the field ring fastest (p3gwrt.f:46-64).
 #include "galhip_p3d.h"
 
+#include <algorithm>
 #include <climits>
 
 namespace gh {
@@ -966,14 +967,47 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_deinterleave_kernel(
 
 // ---- field solve ------------------------------------------------------------------
 
-// grid (ngz, nr): block (plane, ring-1)
+// Solve shapes.  All transforms are direct sums in the order of one sum per
+// output (j, p or k ascending), whatever the shape, so that results do not
+// depend on it; what the shapes share is the twiddle, read from LDS once for
+// several planes or columns.  200 rings x 125 planes x 256 spokes, 9 harmonics:
+//   analysis  `planes` planes a wavefront, cosine and sine sums of a harmonic
+//             together (sums once per component before, each formed twice):
+//             100 -> 50 us; 4 planes 56 (registers: 4 wavefronts a SIMD instead
+//             of 7), 1 plane 65.  Floor: 77 MB, 15 us; conversions and the
+//             wavefront sums are what is left.
+//   synthesis `splanes` planes a block: 101 -> 48 us; 2 planes 48, 8 planes 52.
+//             It stores the three force components only (57 us when it reads
+//             the potential to store whole vectors): 77 MB.
+template <typename R> struct P3Solve {
+    static constexpr int planes = sizeof(R) == 4 ? 2 : 1;
+    static constexpr int splanes = sizeof(R) == 4 ? 4 : 2;
+    static constexpr int harm = 9;
+};
+
+// combined, scaled mass of a cell (zoncmb + scaled)
+template <typename R>
+__device__ __forceinline__ R p3_cell_mass(const P3SolveArgs<R> &a, size_t idx) {
+    double acc = (double)a.mfx[0][idx] * a.q;
+    for (int z = 2; z <= a.nz; z++) {
+        if (a.use_new[z - 1]) acc = acc + a.fnew[z - 1] * ((double)a.mfx[z - 1][idx] * a.q);
+        if (a.use_old[z - 1]) acc = acc + a.fold[z - 1] * ((double)a.moz[z - 1][idx] * a.q);
+    }
+    return (R)(acc * a.pmass);
+}
+
+// grid (planes / (4 wavefronts x P3Solve::planes), nr): a wavefront takes some
+// planes of a ring
 template <typename R>
 __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) {
-    __shared__ R rho_s[P3_MAX_NA];
-    __shared__ R tws[2 * P3_MAX_NA];
+    constexpr int PL = P3Solve<R>::planes, HB = P3Solve<R>::harm;
+    typedef typename Vec2<R>::T R2;
+    extern __shared__ unsigned char p3_lds[];
+    R2 *tws = (R2 *)p3_lds;                   // [na]
     __shared__ int s_rng[4], s_ok, s_jr[GH_MAXZ], s_kr[GH_MAXZ];
-    const int tid = threadIdx.x, na = a.na;
-    const int plane = blockIdx.x, ir = blockIdx.y + 1;
+    const int tid = threadIdx.x, na = a.na, nm = a.nm, lane = tid & 63;
+    const int ir = blockIdx.y + 1;
+    const int plane0 = (blockIdx.x * (P3_BLOCK / 64) + (tid >> 6)) * PL;
     if (tid < 64) combine_ranges(a.jrad, a.krad, a.rstride, a.nz, s_jr, s_kr);
     if (tid == 0) {
         int kr[GH_MAXZ], rg[4] = {0, 0, 0, 0};
@@ -981,49 +1015,85 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
                                      a.explicit_zones, a.jzone, a.kzone, kr, rg);
         s_ok = ok;
         for (int q = 0; q < 4; q++) s_rng[q] = rg[q];
-        if (plane == 0 && ir == 1) {
+        if (blockIdx.x == 0 && ir == 1) {
             for (int q = 0; q < 4; q++) a.ranges[q] = ok ? rg[q] : -1;
             if (ok)
                 for (int z = 1; z < a.nz; z++) a.krad[z] = kr[z];
         }
     }
+    for (int j = tid; j < na; j += P3_BLOCK) tws[j] = mk2(a.tw[2 * j], a.tw[2 * j + 1]);
     __syncthreads();
-    // zoncmb + scaled for this ring and plane
-    const size_t row = ((size_t)(ir - 1) * a.ngz + plane) * na;
-    for (int j = tid; j < na; j += P3_BLOCK) {
-        const size_t idx = row + j;
-        double acc = (double)a.mfx[0][idx] * a.q;
-        for (int z = 2; z <= a.nz; z++) {
-            if (a.use_new[z - 1]) acc = acc + a.fnew[z - 1] * ((double)a.mfx[z - 1][idx] * a.q);
-            if (a.use_old[z - 1]) acc = acc + a.fold[z - 1] * ((double)a.moz[z - 1][idx] * a.q);
+    if (plane0 >= a.ngz) return;
+    const bool active = s_ok && ir >= s_rng[0] && ir <= s_rng[1];
+    size_t row[PL];
+#pragma unroll
+    for (int p = 0; p < PL; p++)
+        row[p] = ((size_t)(ir - 1) * a.ngz + min(plane0 + p, a.ngz - 1)) * na;
+    int s = 0;
+    bool first = true;
+    do {
+        // the next HB harmonics of the slot list
+        int k[HB], step[HB], sn = s;
+#pragma unroll
+        for (int h = 0; h < HB; h++) {
+            int m = 0;
+            if (sn < nm) {
+                m = a.slot_m[sn];
+                sn += sn + 1 < nm && a.slot_p[sn + 1] ? 2 : 1;
+            }
+            k[h] = (int)(((long long)m * lane) % na);
+            step[h] = (int)(((long long)m * 64) % na);
         }
-        const R v = (R)(acc * a.pmass);
-        rho_s[j] = v;
-        a.rho[idx] = v;
-    }
-    for (int j = tid; j < 2 * na; j += P3_BLOCK) tws[j] = a.tw[j];
-    __syncthreads();
-    if (!s_ok || ir < s_rng[0] || ir > s_rng[1]) return;
-    const int wave = tid >> 6, lane = tid & 63, nw = P3_BLOCK / 64;
-    for (int s = wave; s < a.nm; s += nw) {
-        const int m = a.slot_m[s], part = a.slot_p[s];
-        R sa = 0, sb = 0;
-        int k = (int)(((long long)m * lane) % na);
-        const int step = (int)(((long long)m * 64) % na);
+        R sa[HB][PL], sb[HB][PL];
+#pragma unroll
+        for (int h = 0; h < HB; h++)
+#pragma unroll
+            for (int p = 0; p < PL; p++) sa[h][p] = sb[h][p] = (R)0;
         for (int j = lane; j < na; j += 64) {
-            const R rv = rho_s[j];
-            sa += rv * tws[2 * k];
-            sb += rv * tws[2 * k + 1];
-            k += step;
-            if (k >= na) k -= na;
+            R rv[PL];
+#pragma unroll
+            for (int p = 0; p < PL; p++) rv[p] = first ? p3_cell_mass(a, row[p] + j) : a.rho[row[p] + j];
+            if (first)
+#pragma unroll
+                for (int p = 0; p < PL; p++)
+                    if (plane0 + p < a.ngz) a.rho[row[p] + j] = rv[p];
+            if (!active) continue;
+#pragma unroll
+            for (int h = 0; h < HB; h++) {
+                const R2 w = tws[k[h]];
+#pragma unroll
+                for (int p = 0; p < PL; p++) {
+                    sa[h][p] += rv[p] * w.x;
+                    sb[h][p] += rv[p] * w.y;
+                }
+                k[h] += step[h];
+                if (k[h] >= na) k[h] -= na;
+            }
         }
-        sa = p3_wave_sum(sa);
-        sb = p3_wave_sum(sb);
-        if (lane == 0) a.A[((size_t)(ir - 1) * a.nm + s) * a.ngz + plane] = part ? -sb : sa;
-    }
+        if (!active) return;
+#pragma unroll
+        for (int h = 0; h < HB; h++) {
+            const bool pair = s + 1 < nm && a.slot_p[s + 1];
+            R va = 0, vb = 0;
+#pragma unroll
+            for (int p = 0; p < PL; p++) {
+                const R ta = p3_wave_sum(sa[h][p]), tb = p3_wave_sum(sb[h][p]);
+                if (lane == p) {
+                    va = ta;
+                    vb = -tb;
+                }
+            }
+            R *out = a.A + ((size_t)(ir - 1) * nm + s) * a.ngz + plane0 + lane;
+            if (s < nm && lane < PL && plane0 + lane < a.ngz) {
+                out[0] = va;
+                if (pair) out[a.ngz] = vb;
+            }
+            s += pair ? 2 : 1;
+        }
+        first = false;
+    } while (s < nm);
 }
 
-// grid (nr): the doubled vertical transform of each component column
 // The vertical twiddles (cos, sin of 2 pi k / P) in LDS with one pad entry
 // after every 256 bytes: the transforms read them at index p k mod P across
 // consecutive k (or q), a stride that puts many lanes on one bank when it is
@@ -1037,52 +1107,83 @@ template <typename R> __device__ __forceinline__ int tz_at(int idx) {
 }
 template <typename R>
 __device__ __forceinline__ void tz_stage(const R *twz, int P, R *tz) {
-    for (int e = threadIdx.x; e < P; e += P3_BLOCK) {
+    for (int e = threadIdx.x; e < P; e += blockDim.x) {
         tz[tz_at<R>(e)] = twz[2 * e];
         tz[tz_at<R>(e) + 1] = twz[2 * e + 1];
     }
 }
 
-template <typename R>
+// The ring of a vertical transform's block: consecutive blocks go to the eight
+// XCDs in turn, and neighbouring rings, which share the lines of the
+// [column][k][ring] arrays, to one of them.
+__device__ __forceinline__ int p3_ring(int nr) {
+    const int b = blockIdx.x, x = b & 7, q = nr >> 3, r = nr & 7;
+    return x * q + min(x, r) + (b >> 3);
+}
+
+// grid (nr, columns / CB): the doubled vertical transform of some component
+// columns of one ring
+template <typename R, int CB>
 __global__ __launch_bounds__(P3_BLOCK) void p3_zfwd_kernel(P3SolveArgs<R> a) {
     extern __shared__ unsigned char p3_lds[];
-    R *col = (R *)p3_lds;                     // [nm][ngz]
     const int ngz = a.ngz, P = 2 * ngz, nm = a.nm;
-    R *tz = col + (size_t)nm * ngz;           // [P][2]
-    const int ir = blockIdx.x + 1, tid = threadIdx.x;
+    const int s0 = blockIdx.y * CB, ncol = min(CB, nm - s0);
+    R *tz = (R *)p3_lds;                      // [P][2]
+    R *col = tz + tz_words<R>(P);             // [ngz][CB]
+    const int ir = p3_ring(a.nr) + 1, tid = threadIdx.x;
     const int jrs = a.ranges[0], krs = a.ranges[1];
     if (jrs < 1 || ir < jrs || ir > krs) return;
-    const R *src = a.A + (size_t)(ir - 1) * nm * ngz;
-    for (int e = tid; e < nm * ngz; e += P3_BLOCK) col[e] = src[e];
+    const R *src = a.A + ((size_t)(ir - 1) * nm + s0) * ngz;
+    for (int e = tid; e < CB * ngz; e += blockDim.x) {
+        const int c = e / ngz, p = e - c * ngz;
+        col[p * CB + c] = c < ncol ? src[e] : (R)0;
+    }
     tz_stage<R>(a.twz, P, tz);
     __syncthreads();
-    R *dst = a.M + (size_t)(ir - 1) * nm * P;
-    for (int o = tid; o < nm * (ngz + 1); o += P3_BLOCK) {
-        const int s = o / (ngz + 1), k = o - s * (ngz + 1);
-        const R *c = col + (size_t)s * ngz;
-        R sa = 0, sb = 0;
+    // [column][k][ring]: the contraction reads and writes rings
+    R *dst = a.M + (size_t)s0 * P * a.nr + (ir - 1);
+    const size_t nr = a.nr;
+    for (int k = tid; k <= ngz; k += blockDim.x) {
+        R sa[CB], sb[CB];
+#pragma unroll
+        for (int c = 0; c < CB; c++) sa[c] = sb[c] = (R)0;
         int idx = 0;
+#pragma unroll 4
         for (int p = 0; p < ngz; p++) {
             const int t = tz_at<R>(idx);
-            sa += c[p] * tz[t];
-            sb += c[p] * tz[t + 1];
+            const R w0 = tz[t], w1 = tz[t + 1];
+#pragma unroll
+            for (int c = 0; c < CB; c++) {
+                const R v = col[p * CB + c];
+                sa[c] += v * w0;
+                sb[c] += v * w1;
+            }
             idx += k;
             if (idx >= P) idx -= P;
         }
-        R *h = dst + (size_t)s * P;
-        if (k == 0) h[0] = sa;
-        else if (k == ngz) h[P - 1] = sa;
-        else {
-            h[2 * k - 1] = sa;
-            h[2 * k] = -sb;
+#pragma unroll
+        for (int c = 0; c < CB; c++) {
+            if (c >= ncol) break;
+            R *h = dst + (size_t)c * P * nr;
+            if (k == 0) h[0] = sa[c];
+            else if (k == ngz) h[(P - 1) * nr] = sa[c];
+            else {
+                h[(2 * k - 1) * nr] = sa[c];
+                h[2 * k * nr] = -sb[c];
+            }
         }
     }
 }
 
-// grid (ng, ngz + 1, ntypes): block (m, k_z, type) applies one Green's matrix
+// grid (ng, ngz + 1, ntypes): block (m, k_z, type) applies one Green's matrix.
+// Reading the tables bounds it: three types of 9 x 126 matrices of 200 x 200,
+// 544 MB, in 128 us (4.2 TB/s; a copy reaches 5.3).  With M and W by ring
+// first the 4-byte accesses of the source rings and results, a line each, made
+// it 154.
 template <typename R>
 __global__ __launch_bounds__(P3_BLOCK) void p3_conv_kernel(P3SolveArgs<R> a) {
-    __shared__ R rhs[4][P3_MAX_NR];
+    typedef typename Vec4<R>::T R4;
+    __shared__ R4 rhs[P3_MAX_NR];
     const int im = blockIdx.x + 1, iz = blockIdx.y + 1, type = blockIdx.z;
     const int ng = a.ng, ngz = a.ngz, mmax = a.mmax, nm = a.nm, nr = a.nr;
     if (type == 1 && (im < 2 || im > min(ng, mmax - 1))) return;
@@ -1114,7 +1215,7 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_conv_kernel(P3SolveArgs<R> a) {
     const int nrs = krs - jrs + 1;
     for (int e = threadIdx.x; e < 4 * nrs; e += P3_BLOCK) {
         const int q = e / nrs, is = jrs + (e - q * nrs);
-        rhs[q][is - 1] = val[q] ? sgn[q] * a.M[(size_t)(is - 1) * nm * P + src[q]] : (R)0;
+        reinterpret_cast<R *>(rhs)[4 * (is - 1) + q] = val[q] ? sgn[q] * a.M[(size_t)src[q] * nr + (is - 1)] : (R)0;
     }
     __syncthreads();
     const R *Gm = a.G + ((((size_t)type * (ngz + 1) + (iz - 1)) * ng + (im - 1)) * nr) * nr;
@@ -1124,110 +1225,135 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_conv_kernel(P3SolveArgs<R> a) {
 #pragma unroll 8
         for (int is = jrs; is <= krs; is++) {
             const R gv = g[(size_t)(is - 1) * nr];
-            s0 += gv * rhs[0][is - 1];
-            s1 += gv * rhs[1][is - 1];
-            s2 += gv * rhs[2][is - 1];
-            s3 += gv * rhs[3][is - 1];
+            const R4 r = rhs[is - 1];
+            s0 += gv * r.x;
+            s1 += gv * r.y;
+            s2 += gv * r.z;
+            s3 += gv * r.w;
         }
-        R *w = a.W + ((size_t)type * nr + (ir - 1)) * nm * P;
-        if (val[0]) w[dst[0]] = s0;
-        if (val[1]) w[dst[1]] = s1;
-        if (val[2]) w[dst[2]] = s2;
-        if (val[3]) w[dst[3]] = s3;
+        R *w = a.W + (size_t)type * nm * P * nr + (ir - 1);
+        if (val[0]) w[(size_t)dst[0] * nr] = s0;
+        if (val[1]) w[(size_t)dst[1] * nr] = s1;
+        if (val[2]) w[(size_t)dst[2] * nr] = s2;
+        if (val[3]) w[(size_t)dst[3] * nr] = s3;
     }
 }
 
-// grid (nr, ntypes): inverse vertical transform of one ring's columns
-template <typename R>
+// grid (nr, ntypes, columns / CB): inverse vertical transform of
+// some columns of one ring
+template <typename R, int CB>
 __global__ __launch_bounds__(P3_BLOCK) void p3_zinv_kernel(P3SolveArgs<R> a) {
     extern __shared__ unsigned char p3_lds[];
     const int ngz = a.ngz, P = 2 * ngz, nm = a.nm;
-    R *h = (R *)p3_lds;                       // [nm][P]
-    R *tz = h + (size_t)nm * P;               // [P][2]
-    const int ir = blockIdx.x + 1, type = blockIdx.y, tid = threadIdx.x;
+    const int s0 = blockIdx.z * CB, ncol = min(CB, nm - s0);
+    R *tz = (R *)p3_lds;                      // [P][2]
+    R *h = tz + tz_words<R>(P);               // [P][CB]
+    const int ir = p3_ring(a.nr) + 1, type = blockIdx.y, tid = threadIdx.x;
     const int jrs = a.ranges[0], jrf = a.ranges[2], krf = a.ranges[3];
     if (jrs < 1 || ir < jrf || ir > krf) return;
-    const R *src = a.W + ((size_t)type * a.nr + (ir - 1)) * nm * P;
-    for (int e = tid; e < nm * P; e += P3_BLOCK) h[e] = src[e];
+    const R *src = a.W + ((size_t)type * nm + s0) * P * a.nr + (ir - 1);
+    for (int e = tid; e < CB * P; e += blockDim.x) {
+        const int c = e / P, k = e - c * P;
+        h[k * CB + c] = c < ncol ? src[(size_t)e * a.nr] : (R)0;
+    }
     tz_stage<R>(a.twz, P, tz);
     __syncthreads();
-    R *dst = a.Z + ((size_t)type * a.nr + (ir - 1)) * ngz * nm;
-    for (int o = tid; o < nm * ngz; o += P3_BLOCK) {
-        const int s = o / ngz, q = o - s * ngz;
-        const R *c = h + (size_t)s * P;
-        R v = c[0] + ((q & 1) ? -c[P - 1] : c[P - 1]);
+    R *dst = a.Z + ((size_t)type * a.nr + (ir - 1)) * ngz * nm + s0;
+    for (int q = tid; q < ngz; q += blockDim.x) {
+        R v[CB];
+#pragma unroll
+        for (int c = 0; c < CB; c++) {
+            const R e = h[(P - 1) * CB + c];
+            v[c] = h[c] + ((q & 1) ? -e : e);
+        }
         int idx = q;
+#pragma unroll 4
         for (int k = 1; k < ngz; k++) {
             const int t = tz_at<R>(idx);
-            v += (R)2 * (c[2 * k - 1] * tz[t] - c[2 * k] * tz[t + 1]);
+            const R w0 = tz[t], w1 = tz[t + 1];
+            const R *hk = h + (2 * k - 1) * CB;
+            // (v + 2 x rounds as the fused product does: 2 x is exact)
+#pragma unroll
+            for (int c = 0; c < CB; c++)
+                v[c] = fma((R)2, hk[c] * w0 - hk[CB + c] * w1, v[c]);
             idx += q;
             if (idx >= P) idx -= P;
         }
-        dst[(size_t)q * nm + s] = v;
+#pragma unroll
+        for (int c = 0; c < CB; c++)
+            if (c < ncol) dst[(size_t)q * nm + c] = v[c];
     }
 }
 
-// grid (ngz, nr): block (plane, ring-1): inverse azimuthal transform of the
-// active components, scale, polcat; interleaved field store
-template <typename R>
+// grid (planes / P3Solve::planes, nr): inverse azimuthal transform of the
+// active components of some planes of a ring, scale, polcat; interleaved
+// field store
+template <typename R, bool LPOT>
 __global__ __launch_bounds__(P3_BLOCK) void p3_synth_kernel(P3SolveArgs<R> a) {
     typedef typename Vec4<R>::T R4;
-    __shared__ R zc[4][P3_MAX_NM];
-    __shared__ R tws[2 * P3_MAX_NA];
-    __shared__ int sm[P3_MAX_NM], sp[P3_MAX_NM];
-    const int plane = blockIdx.x, ir = blockIdx.y + 1, tid = threadIdx.x;
+    typedef typename Vec2<R>::T R2;
+    constexpr int PL = P3Solve<R>::splanes, NT = LPOT ? 4 : 3;
+    extern __shared__ unsigned char p3_lds[];
+    R4 *zc = (R4 *)p3_lds;                    // [nm][PL]
+    R2 *tws = (R2 *)(zc + a.nm * PL);         // [na]
+    const int plane0 = blockIdx.x * PL, ir = blockIdx.y + 1, tid = threadIdx.x;
     const int na = a.na, nm = a.nm, ngz = a.ngz, mmax = a.mmax;
     const int jrs = a.ranges[0], jrf = a.ranges[2], krf = a.ranges[3];
     if (jrs < 1 || ir < jrf || ir > krf) return;
-    for (int e = tid; e < 4 * nm; e += P3_BLOCK) {
-        const int t = e / nm, s = e - t * nm;
+    for (int e = tid; e < 4 * PL * nm; e += blockDim.x) {
+        const int t = e / (PL * nm), r = e - t * (PL * nm), p = r / nm, s = r - p * nm;
         R v = (R)0;
-        if (t < a.ntypes && !(t == 1 && a.ng == 1))
-            v = a.Z[(((size_t)t * a.nr + (ir - 1)) * ngz + plane) * nm + s];
-        zc[t][s] = v;
+        if (t < NT && !(t == 1 && a.ng == 1) && plane0 + p < ngz)
+            v = a.Z[(((size_t)t * a.nr + (ir - 1)) * ngz + plane0 + p) * nm + s];
+        reinterpret_cast<R *>(zc)[4 * (s * PL + p) + t] = v;
     }
-    for (int e = tid; e < nm; e += P3_BLOCK) {
-        sm[e] = a.slot_m[e];
-        sp[e] = a.slot_p[e];
-    }
-    for (int j = tid; j < 2 * na; j += P3_BLOCK) tws[j] = a.tw[j];
+    for (int j = tid; j < na; j += blockDim.x) tws[j] = mk2(a.tw[2 * j], a.tw[2 * j + 1]);
     __syncthreads();
     const R scale = (R)1 / (R)(2 * ngz * na);
-    const size_t row = ((size_t)(ir - 1) * ngz + plane) * na;
-    for (int j = tid; j < na; j += P3_BLOCK) {
-        R F0 = 0, F1 = 0, F2 = 0, F3 = 0;
+    const size_t row = ((size_t)(ir - 1) * ngz + plane0) * na;
+    for (int j = tid; j < na; j += blockDim.x) {
+        R F[PL][NT];
+#pragma unroll
+        for (int p = 0; p < PL; p++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) F[p][t] = (R)0;
         // k = (m j) mod na, advanced with m (the slots come in ascending m)
         int mcur = 0, k = 0;
         for (int s = 0; s < nm; s++) {
-            const int m = sm[s];
-            if (m < mcur) {
-                mcur = 0;
-                k = 0;
-            }
+            const int m = a.slot_m[s], part = a.slot_p[s];
             for (; mcur < m; mcur++) {
                 k += j;
                 if (k >= na) k -= na;
             }
-            R b;
+            const R2 w = tws[k];
+            R b = part ? (R)-2 * w.y : (R)2 * w.x;
             if (m == 0) b = (R)1;
-            else if (m == mmax - 1) b = (j & 1) ? (R)-1 : (R)1;
-            else b = sp[s] ? (R)-2 * tws[2 * k + 1] : (R)2 * tws[2 * k];
-            F0 += zc[0][s] * b;
-            F1 += zc[1][s] * b;
-            F2 += zc[2][s] * b;
-            F3 += zc[3][s] * b;
+            if (m == mmax - 1) b = (j & 1) ? (R)-1 : (R)1;
+#pragma unroll
+            for (int p = 0; p < PL; p++) {
+                const R4 z = zc[s * PL + p];
+                F[p][0] += z.x * b;
+                F[p][1] += z.y * b;
+                F[p][2] += z.z * b;
+                if (LPOT) F[p][3] += z.w * b;
+            }
         }
-        F0 *= scale;
-        F1 *= scale;
-        F2 *= scale;
-        F3 *= scale;
-        const R cp = tws[2 * j], sn = tws[2 * j + 1];
-        R4 out;
-        out.x = F0 * cp - F1 * sn;
-        out.y = F0 * sn + F1 * cp;
-        out.z = F2;
-        out.w = a.lpot ? F3 : a.fld[row + j].w;
-        a.fld[row + j] = out;
+        const R cp = tws[j].x, sn = tws[j].y;
+#pragma unroll
+        for (int p = 0; p < PL; p++) {
+            if (plane0 + p >= ngz) break;
+            const R F0 = F[p][0] * scale, F1 = F[p][1] * scale;
+            R *f = reinterpret_cast<R *>(a.fld + row + (size_t)p * na + j);
+            const R x = F0 * cp - F1 * sn, y = F0 * sn + F1 * cp, z = F[p][2] * scale;
+            if (LPOT) {
+                *reinterpret_cast<R4 *>(f) = mk4(x, y, z, F[p][NT - 1] * scale);
+            } else {
+                // the potential of the last solve that formed it stays
+                f[0] = x;
+                f[1] = y;
+                f[2] = z;
+            }
+        }
     }
 }
 
@@ -1470,6 +1596,7 @@ hipError_t launch_p3_integrals(const P3Args<R> &a, int with_pot, const double4 *
 }
 
 // Limits the launches below rely on (checked again by the context set-up).
+// (the limits of whole-ring transforms; contexts beyond them are refused)
 template <typename R> bool p3_solve_fits(const P3SolveArgs<R> &a) {
     const size_t P = 2 * (size_t)a.ngz;
     return a.na <= P3_MAX_NA && a.nm <= P3_MAX_NM && a.nr <= P3_MAX_NR &&
@@ -1477,22 +1604,54 @@ template <typename R> bool p3_solve_fits(const P3SolveArgs<R> &a) {
            ((size_t)a.nm * P + tz_words<R>(P)) * sizeof(R) <= 48 * 1024;
 }
 
+// block of whole wavefronts for n lanes
+static dim3 p3_lanes(int n) { return dim3(std::min(P3_BLOCK, (n + 63) / 64 * 64)); }
+
+// The vertical transforms by CB columns a block.  The forward transform takes
+// three.  The inverse reads a column twice as often as it multiplies it, from
+// LDS: nine columns share a twiddle (three types of 200 rings, 17 columns:
+// 49 us, three at a time 60) if that leaves four blocks a CU, else three, for
+// more blocks (three types of 61 rings, 9 columns, FP64: 22 us and 10 us).
+// With fewer columns in the context, no more of them than it has stand in LDS.
+template <typename R, int CB>
+static hipError_t p3_vertical(const P3SolveArgs<R> &a, bool inverse, hipStream_t s) {
+    const size_t P = 2 * (size_t)a.ngz;
+    const unsigned nc = (a.nm + CB - 1) / CB;
+    if (inverse)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_zinv_kernel<R, CB>), dim3(a.nr, a.ntypes, nc),
+                           p3_lanes(a.ngz), (CB * P + tz_words<R>(P)) * sizeof(R), s, a);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_zfwd_kernel<R, CB>), dim3(a.nr, nc),
+                           p3_lanes(a.ngz + 1), (CB * a.ngz + tz_words<R>(P)) * sizeof(R), s, a);
+    return hipGetLastError();
+}
+template <typename R>
+static hipError_t p3_vertical(const P3SolveArgs<R> &a, bool inverse, hipStream_t s) {
+    if (a.nm == 0) return hipSuccess;
+    if (inverse && a.nm >= 9 && (long long)a.nr * a.ntypes * ((a.nm + 8) / 9) >= 1024)
+        return p3_vertical<R, 9>(a, inverse, s);
+    return a.nm >= 3 ? p3_vertical<R, 3>(a, inverse, s) : p3_vertical<R, 1>(a, inverse, s);
+}
+
 template <typename R> hipError_t launch_p3_solve(const P3SolveArgs<R> &a, hipStream_t s) {
     if (!p3_solve_fits(a)) return hipErrorInvalidValue;
-    const size_t P = 2 * (size_t)a.ngz;
-    hipLaunchKernelGGL(p3_analyse_kernel<R>, dim3(a.ngz, a.nr), dim3(P3_BLOCK), 0, s, a);
+    constexpr unsigned PL = P3Solve<R>::planes, per = P3_BLOCK / 64 * PL;
+    hipLaunchKernelGGL(p3_analyse_kernel<R>, dim3((a.ngz + per - 1) / per, a.nr), dim3(P3_BLOCK),
+                       2 * a.na * sizeof(R), s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(p3_zfwd_kernel<R>, dim3(a.nr), dim3(P3_BLOCK),
-                       ((size_t)a.nm * a.ngz + tz_words<R>(P)) * sizeof(R), s, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = p3_vertical(a, false, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(p3_conv_kernel<R>, dim3(a.ng, a.ngz + 1, a.ntypes), dim3(P3_BLOCK),
                        0, s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(p3_zinv_kernel<R>, dim3(a.nr, a.ntypes), dim3(P3_BLOCK),
-                       ((size_t)a.nm * P + tz_words<R>(P)) * sizeof(R), s, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(p3_synth_kernel<R>, dim3(a.ngz, a.nr), dim3(P3_BLOCK), 0, s, a);
+    if ((e = p3_vertical(a, true, s)) != hipSuccess) return e;
+    constexpr int SL = P3Solve<R>::splanes;
+    const dim3 grid((a.ngz + SL - 1) / SL, a.nr);
+    const size_t lds = (4 * (size_t)a.nm * SL + 2 * a.na) * sizeof(R);
+    if (a.lpot)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_synth_kernel<R, true>), grid, p3_lanes(a.na), lds, s, a);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_synth_kernel<R, false>), grid, p3_lanes(a.na), lds, s, a);
     return hipGetLastError();
 }
 
