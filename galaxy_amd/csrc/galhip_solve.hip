@@ -17,6 +17,8 @@
 //   circle, harmonic filter, p2gwrt's [m][field ring][source ring] layout.
 #include "galhip_kern.h"
 
+#include <algorithm>
+
 namespace gh {
 
 constexpr int MAX_NA = 2048;
@@ -118,11 +120,12 @@ __global__ __launch_bounds__(SOLVE_BLOCK) void analyse_kernel(AnaArgs<R> a) {
 // (q+1) na/SYN_SPLIT) of grid mem.
 // PRE: the contraction was done beforehand (the ensemble's MFMA GEMM):
 // W is read from a.wpre[mem][type][cos/sin][m][ring] instead.
-template <typename R, bool PRE>
-__global__ __launch_bounds__(SOLVE_BLOCK) void synth_kernel(SynArgs<R> a) {
+template <typename R, bool PRE, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void synth_kernel(SynArgs<R> a) {
     typedef typename Vec2<R>::T R2;
     __shared__ R W[3][2][MAX_NG];
-    __shared__ R tws[2 * MAX_NA];
+    extern __shared__ unsigned char solve_lds[];
+    R *tws = (R *)solve_lds;                  // [na][2]
     const int tid = threadIdx.x, na = a.na, nr = a.nr, ir = blockIdx.x + 1;
     const int q = blockIdx.y, mem = blockIdx.z;
     const int jlo = (q * na) / SYN_SPLIT, jhi = ((q + 1) * na) / SYN_SPLIT;
@@ -132,30 +135,31 @@ __global__ __launch_bounds__(SOLVE_BLOCK) void synth_kernel(SynArgs<R> a) {
     // masscl of the coming push, on this block's cells
     if (a.masscl_z > 0) {
         const size_t row = mo + (size_t)(ir - 1) * na;
-        for (int j = jlo + tid; j < jhi; j += SOLVE_BLOCK) {
+        for (int j = jlo + tid; j < jhi; j += BLOCK) {
             const size_t idx = row + j;
             for (int z = 1; z <= a.masscl_z; z++) {
                 if (z >= 2) a.moz[z - 1][idx] = a.mfx[z - 1][idx];
                 a.mfx[z - 1][idx] = 0;
             }
         }
-        if (blockIdx.x == 0 && q == 0 && tid < a.masscl_z * GH_RANGE_STRIPES) {
-            const int z = tid / GH_RANGE_STRIPES;
-            const int e = (tid & (GH_RANGE_STRIPES - 1)) * a.rstride + mem * GH_MAXZ + z;
-            a.jrad[e] = nr;
-            a.krad[e] = 0;
-        }
+        if (blockIdx.x == 0 && q == 0)
+            for (int t = tid; t < a.masscl_z * GH_RANGE_STRIPES; t += BLOCK) {
+                const int z = t / GH_RANGE_STRIPES;
+                const int e = (t & (GH_RANGE_STRIPES - 1)) * a.rstride + mem * GH_MAXZ + z;
+                a.jrad[e] = nr;
+                a.krad[e] = 0;
+            }
     }
     const int jrs = ranges[0], krs = ranges[1];
     const int jrf = ranges[2], krf = ranges[3];
     if (jrs < 1 || ir < jrf || ir > krf) return;
-    for (int j = tid; j < 2 * na; j += SOLVE_BLOCK) tws[j] = a.tw[j];
+    for (int j = tid; j < 2 * na; j += BLOCK) tws[j] = a.tw[j];
     const int ntypes = a.lpot ? 3 : 2;
-    const int wave = tid >> 6, lane = tid & 63, nw = SOLVE_BLOCK / 64;
+    const int wave = tid >> 6, lane = tid & 63, nw = BLOCK / 64;
     const int mmax = a.mmax;
     const int maz = min(mmax - 2, a.ng - 1);
     if (PRE) {
-        for (int t = tid; t < ntypes * 2 * a.ng; t += SOLVE_BLOCK) {
+        for (int t = tid; t < ntypes * 2 * a.ng; t += BLOCK) {
             const int type = t / (2 * a.ng), r = t - type * 2 * a.ng, cs = r / a.ng;
             const int m = r - cs * a.ng;
             W[type][cs][m] = (R)a.wpre[((((size_t)mem * 3 + type) * 2 + cs) * a.ng + m) * nr +
@@ -226,7 +230,7 @@ __global__ __launch_bounds__(SOLVE_BLOCK) void synth_kernel(SynArgs<R> a) {
     }
     __syncthreads();
     const R inv = (R)1 / (R)na;
-    for (int j = jlo + tid; j < jhi; j += SOLVE_BLOCK) {
+    for (int j = jlo + tid; j < jhi; j += BLOCK) {
         R F[3] = {0, 0, 0};
         for (int type = 0; type < ntypes; type++) {
             R s = W[type][0][0];
@@ -360,11 +364,241 @@ __global__ void masscl_kernel(ZonePtrs zp, int mz, long long ncell, int *jrad,
     }
 }
 
+// ---- many rings at once (ensembles) -------------------------------------------
+//
+// A block of 16 wavefronts per ring suits one grid, whose few rings leave most
+// of the chip idle; with the rings of many discs the harmonics of a ring keep
+// only some of the wavefronts busy and every ring loads its twiddles.  Here a
+// wavefront (analysis) or a block (synthesis) takes several rings of a member
+// and shares the twiddles.  Every sum keeps its order, so that a member's
+// results stay those of the same disc alone.  64 discs of 128 x 256, 9
+// harmonics: analysis 46.7 -> 15.7 us (four rings a wavefront 19.8, one 16.0),
+// synthesis 40.9 -> 15.6 (two rings a block 17.0, eight 20.0).
+constexpr int ROWS_BLOCK = 256;
+constexpr int ROWS_HARM = 9;     // harmonics per pass of the analysis
+template <typename R> constexpr int ana_rows() { return sizeof(R) == 4 ? 2 : 1; }
+constexpr int SYN_ROWS = 4;
+
+// grid (rings / (4 wavefronts x ana_rows), nmem)
+template <typename R>
+__global__ __launch_bounds__(ROWS_BLOCK) void analyse_rows_kernel(AnaArgs<R> a) {
+    constexpr int RW = ana_rows<R>(), HB = ROWS_HARM;
+    typedef typename Vec2<R>::T R2;
+    extern __shared__ unsigned char rows_lds[];
+    R2 *tws = (R2 *)rows_lds;                 // [na]
+    __shared__ int s_rng[4], s_ok, s_jr[GH_MAXZ], s_kr[GH_MAXZ];
+    const int tid = threadIdx.x, na = a.na, nr = a.nr, mem = blockIdx.y, lane = tid & 63;
+    const int ring0 = (blockIdx.x * (ROWS_BLOCK / 64) + (tid >> 6)) * RW;   // 0-based
+    const size_t mo = (size_t)mem * nr * na;
+    int *const jrad = a.jrad + mem * GH_MAXZ;
+    int *const krad = a.krad + mem * GH_MAXZ;
+    R *const rho = a.rho + mo;
+    R *const coef = a.coef + (size_t)mem * a.ncoef * nr;
+    const double q = a.qbits_m ? ldexp(1.0, -a.qbits_m[mem]) : a.q;
+    const double pmass = a.pmass_m ? a.pmass_m[mem] : a.pmass;
+    if (tid < 64) combine_ranges(jrad, krad, a.rstride, a.nz, s_jr, s_kr);
+    if (tid == 0) {
+        int kr[GH_MAXZ], rg[4] = {0, 0, 0, 0};
+        const bool ok = solve_ranges(s_jr, s_kr, a.nz, nr, a.mzone, a.lpot, a.explicit_zones,
+                                     a.jzone, a.kzone, kr, rg);
+        s_ok = ok;
+        for (int e = 0; e < 4; e++) s_rng[e] = rg[e];
+        if (blockIdx.x == 0) {
+            int *const ranges = a.ranges + mem * 4;
+            for (int e = 0; e < 4; e++) ranges[e] = ok ? rg[e] : -1;
+            if (ok)
+                for (int z = 1; z < a.nz; z++) krad[z] = kr[z];
+        }
+    }
+    for (int j = tid; j < na; j += ROWS_BLOCK) tws[j] = mk2(a.tw[2 * j], a.tw[2 * j + 1]);
+    __syncthreads();
+    if (ring0 >= nr) return;
+    const int jrs = s_ok ? s_rng[0] : nr + 1, krs = s_ok ? s_rng[1] : 0;
+    const bool active = ring0 + RW >= jrs && ring0 + 1 <= krs;   // any ring of the wavefront
+    size_t row[RW];
+#pragma unroll
+    for (int p = 0; p < RW; p++) row[p] = (size_t)min(ring0 + p, nr - 1) * na;
+    for (int m0 = 0; m0 < a.ng; m0 += HB) {
+        int k[HB], step[HB];
+#pragma unroll
+        for (int h = 0; h < HB; h++) {
+            const int m = m0 + h < a.ng ? m0 + h : 0;
+            k[h] = (m * lane) % na;
+            step[h] = (m * 64) % na;
+        }
+        R sa[HB][RW], sb[HB][RW];
+#pragma unroll
+        for (int h = 0; h < HB; h++)
+#pragma unroll
+            for (int p = 0; p < RW; p++) sa[h][p] = sb[h][p] = (R)0;
+        for (int j = lane; j < na; j += 64) {
+            R rv[RW];
+#pragma unroll
+            for (int p = 0; p < RW; p++) {
+                if (m0) {
+                    rv[p] = rho[row[p] + j];
+                    continue;
+                }
+                // zoncmb + scaled
+                const size_t idx = mo + row[p] + j;
+                double acc = (double)a.mfx[0][idx] * q;
+                for (int z = 2; z <= a.nz; z++) {
+                    if (a.use_new[z - 1])
+                        acc = acc + a.fnew[z - 1] * ((double)a.mfx[z - 1][idx] * q);
+                    if (a.use_old[z - 1])
+                        acc = acc + a.fold[z - 1] * ((double)a.moz[z - 1][idx] * q);
+                }
+                rv[p] = (R)(acc * pmass);
+            }
+            if (m0 == 0)
+#pragma unroll
+                for (int p = 0; p < RW; p++)
+                    if (ring0 + p < nr) rho[row[p] + j] = rv[p];
+            if (!active) continue;
+#pragma unroll
+            for (int h = 0; h < HB; h++) {
+                const R2 w = tws[k[h]];
+#pragma unroll
+                for (int p = 0; p < RW; p++) {
+                    sa[h][p] += rv[p] * w.x;
+                    sb[h][p] += rv[p] * w.y;
+                }
+                k[h] += step[h];
+                if (k[h] >= na) k[h] -= na;
+            }
+        }
+        if (!active) return;
+#pragma unroll
+        for (int h = 0; h < HB; h++) {
+            const int m = m0 + h;
+            R va = 0, vb = 0;
+#pragma unroll
+            for (int p = 0; p < RW; p++) {
+                const R ta = wave_sum(sa[h][p]), tb = wave_sum(sb[h][p]);
+                if (lane == p) {
+                    va = ta;
+                    vb = -tb;
+                }
+            }
+            const int ir = ring0 + 1 + lane;
+            if (m < a.ng && lane < RW && ir >= jrs && ir <= krs) {
+                if (a.lg[m]) {
+                    va = 0;
+                    vb = -(R)0;
+                }
+                if (m == 0) {
+                    coef[ir - 1] = va;
+                } else {
+                    coef[(size_t)(2 * m - 1) * nr + ir - 1] = va;
+                    if (2 * m != na) coef[(size_t)(2 * m) * nr + ir - 1] = vb;
+                }
+            }
+        }
+    }
+}
+
+// grid (rings / SYN_ROWS, nmem), after a contraction done beforehand
+template <typename R, bool LPOT>
+__global__ __launch_bounds__(ROWS_BLOCK) void synth_rows_kernel(SynArgs<R> a) {
+    typedef typename Vec2<R>::T R2;
+    constexpr int RW = SYN_ROWS, NT = LPOT ? 3 : 2;
+    extern __shared__ unsigned char rows_lds[];
+    R2 *W = (R2 *)rows_lds;                   // [ng][RW][NT]: (cos, sin) parts
+    R2 *tws = W + a.ng * RW * NT;             // [na]
+    const int tid = threadIdx.x, na = a.na, nr = a.nr, ng = a.ng, mem = blockIdx.y;
+    const int ring0 = blockIdx.x * RW;        // 0-based
+    const size_t mo = (size_t)mem * nr * na;
+    // masscl of the coming push, on this block's cells
+    if (a.masscl_z > 0) {
+        const size_t lo = mo + (size_t)ring0 * na, hi = mo + (size_t)min(ring0 + RW, nr) * na;
+        for (size_t idx = lo + tid; idx < hi; idx += blockDim.x)
+            for (int z = 1; z <= a.masscl_z; z++) {
+                if (z >= 2) a.moz[z - 1][idx] = a.mfx[z - 1][idx];
+                a.mfx[z - 1][idx] = 0;
+            }
+        if (blockIdx.x == 0)
+            for (int e = tid; e < a.masscl_z * GH_RANGE_STRIPES; e += blockDim.x) {
+                const int z = e / GH_RANGE_STRIPES;
+                const int o = (e & (GH_RANGE_STRIPES - 1)) * a.rstride + mem * GH_MAXZ + z;
+                a.jrad[o] = nr;
+                a.krad[o] = 0;
+            }
+    }
+    const int *const ranges = a.ranges + mem * 4;
+    const int jrs = ranges[0], jrf = ranges[2], krf = ranges[3];
+    if (jrs < 1 || ring0 + RW < jrf || ring0 + 1 > krf) return;
+    for (int e = tid; e < NT * 2 * ng * RW; e += blockDim.x) {
+        const int p = e % RW, r = e / RW, type = r / (2 * ng), cm = r - type * 2 * ng;
+        const int cs = cm / ng, m = cm - cs * ng;
+        reinterpret_cast<R *>(W)[2 * ((m * RW + p) * NT + type) + cs] =
+            (R)a.wpre[((((size_t)mem * 3 + type) * 2 + cs) * ng + m) * nr + min(ring0 + p, nr - 1)];
+    }
+    for (int j = tid; j < na; j += blockDim.x) tws[j] = mk2(a.tw[2 * j], a.tw[2 * j + 1]);
+    __syncthreads();
+    const R inv = (R)1 / (R)na;
+    for (int j = tid; j < na; j += blockDim.x) {
+        R s[RW][NT];
+#pragma unroll
+        for (int p = 0; p < RW; p++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) s[p][t] = W[p * NT + t].x;
+        int k = j;
+        for (int m = 1; m < ng; m++) {
+            const R2 w = tws[k];
+            const bool nyq = 2 * m >= na;
+#pragma unroll
+            for (int p = 0; p < RW; p++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const R2 c = W[(m * RW + p) * NT + t];
+                    // (s + 2 x rounds as the fused product does: 2 x is exact)
+                    if (!nyq) s[p][t] = fma((R)2, c.x * w.x - c.y * w.y, s[p][t]);
+                    else s[p][t] += (j & 1) ? -c.x : c.x;
+                }
+            k += j;
+            if (k >= na) k -= na;
+        }
+        const R cp = tws[j].x, sp = tws[j].y;
+#pragma unroll
+        for (int p = 0; p < RW; p++) {
+            const int ir = ring0 + p + 1;
+            if (ir < jrf || ir > krf) continue;
+            const R F0 = s[p][0] * inv, F1 = s[p][1] * inv;
+            const size_t idx = mo + (size_t)(ir - 1) * na + j;
+            a.fld[idx] = mk2(F0 * cp - F1 * sp, F0 * sp + F1 * cp);
+            if (LPOT) a.pot[idx] = s[p][NT - 1] * inv;
+        }
+    }
+}
+
 // ---- host launchers ----
+
+// The rows kernels' time hardly depends on the number of rings until they fill
+// the chip; a block per ring costs the same for every 512 rings.  The lines lie
+// where the two were equal (rings x members):
+//   analysis  1200 at 256 spokes x 9 harmonics (10.7 us against 9.6 at 1536),
+//             1900 at 512 x 9, 3200 at 512 x 17 (14 discs of 256 rings 31.6 and
+//             28.3), 4400 at 1024 x 17: the passes over a ring grow with both;
+//   synthesis after a contraction 1000 to 1450 (1536 rings of 256 spokes 10.1
+//             and 7.9 us, 1024 8.0 and 7.5, 512 4.6 and 7.1).
+// The synthesis with its own contraction keeps its blocks, of 256 threads
+// instead of 1024 once there are enough of them that a block's idle wavefronts
+// keep others off the CU: 64 discs of 128 x 256 99 -> 52 us, FP64 195 -> 80;
+// 768 rings of 512 21.2 and 23.7, FP64 37.9 and 31.3.
+template <typename R> static bool ana_by_rows(const AnaArgs<R> &a) {
+    return 10LL * a.nr * a.nmem >= 5000 + 3LL * a.na * a.ng;
+}
+constexpr int SYN_ROWS_MIN = 1400;
 
 template <typename R>
 hipError_t launch_analyse(const AnaArgs<R> &a, hipStream_t s) {
     if (a.na > MAX_NA) return hipErrorInvalidValue;
+    if (ana_by_rows(a)) {
+        const unsigned per = ROWS_BLOCK / 64 * ana_rows<R>();
+        hipLaunchKernelGGL(analyse_rows_kernel<R>, dim3((a.nr + per - 1) / per, a.nmem),
+                           dim3(ROWS_BLOCK), 2 * a.na * sizeof(R), s, a);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(analyse_kernel<R>, dim3(a.nr, ANA_SPLIT, a.nmem), dim3(SOLVE_BLOCK), 0,
                        s, a);
     return hipGetLastError();
@@ -373,12 +607,27 @@ hipError_t launch_analyse(const AnaArgs<R> &a, hipStream_t s) {
 template <typename R>
 hipError_t launch_synth(const SynArgs<R> &a, hipStream_t s) {
     if (a.ng > MAX_NG) return hipErrorInvalidValue;
+    if (a.wpre && a.nr * a.nmem >= SYN_ROWS_MIN) {
+        const dim3 grid((a.nr + SYN_ROWS - 1) / SYN_ROWS, a.nmem);
+        const dim3 block(std::min(ROWS_BLOCK, (a.na + 63) / 64 * 64));
+        const size_t lds = (2 * (size_t)a.ng * SYN_ROWS * (a.lpot ? 3 : 2) + 2 * a.na) * sizeof(R);
+        if (a.lpot)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_rows_kernel<R, true>), grid, block, lds, s, a);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_rows_kernel<R, false>), grid, block, lds, s, a);
+        return hipGetLastError();
+    }
+    const dim3 grid(a.nr, SYN_SPLIT, a.nmem);
+    const size_t lds = 2 * a.na * sizeof(R);
     if (a.wpre)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_kernel<R, true>), dim3(a.nr, SYN_SPLIT, a.nmem),
-                           dim3(SOLVE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_kernel<R, true, SOLVE_BLOCK>), grid,
+                           dim3(SOLVE_BLOCK), lds, s, a);
+    else if ((size_t)a.nr * a.nmem * sizeof(R) >= 5120)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_kernel<R, false, ROWS_BLOCK>), grid,
+                           dim3(ROWS_BLOCK), lds, s, a);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_kernel<R, false>), dim3(a.nr, SYN_SPLIT, a.nmem),
-                           dim3(SOLVE_BLOCK), 0, s, a);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(synth_kernel<R, false, SOLVE_BLOCK>), grid,
+                           dim3(SOLVE_BLOCK), lds, s, a);
     return hipGetLastError();
 }
 
@@ -397,7 +646,10 @@ hipError_t launch_synth(const SynArgs<R> &a, hipStream_t s) {
 // FP32 and the matrix cores accumulate them in FP32.  The dropped terms are
 // below 2^-24 of the product, so the result has the error of an FP32 dot
 // product.  The instructions are gfx950's K = 32 (16 x 16 tiles) and
-// K = 16 (32 x 32 tiles) bf16 forms.
+// K = 16 (32 x 32 tiles) bf16 forms.  About one wavefront a SIMD: the latency
+// of the operand loads bounds it.  With loads behind the tests of a source
+// range each and two bytes wide for G, 128 columns of 2 x 9 matrices of
+// 128 x 128 took 25.5 us, now 9.6.
 
 typedef __bf16 gh_v8bf __attribute__((ext_vector_type(8)));
 typedef float gh_v4f __attribute__((ext_vector_type(4)));
@@ -437,18 +689,26 @@ __global__ void split_bf16_kernel(const double *__restrict__ G, unsigned short *
     w[2 * tot + i] = bf16_rn((float)g2);
 }
 
-// element (source ring k, column col) of the (type, m) right-hand side
-__device__ __forceinline__ float ens_rhs(const EnsGemmArgs &a, int type, int m, bool pair,
-                                         int off, int k, int col) {
-    const int mem = col >> 1, cs = col & 1;
-    if (mem >= a.nmem || k >= a.nr) return 0.f;
+// A column (member, cos/sin) of the (type, m) right-hand side: source rings
+// lo..hi of p (0-based), negated if neg; zero elsewhere.
+struct EnsCol {
+    const float *p;
+    int lo, hi, last;
+    bool neg;
+};
+__device__ __forceinline__ EnsCol ens_col(const EnsGemmArgs &a, int type, bool pair, int off,
+                                          int col) {
+    const int mem = min(col >> 1, a.nmem - 1), cs = col & 1;
     const int jrs = a.ranges[4 * mem], krs = a.ranges[4 * mem + 1];
-    if (jrs < 1 || k + 1 < jrs || k + 1 > krs) return 0.f;
-    const float *cf = a.coef + (size_t)mem * a.ncoef * a.nr;
-    const float mc = cf[(size_t)off * a.nr + k];
-    const float ms = pair ? cf[(size_t)(off + 1) * a.nr + k] : 0.f;
-    if (type == 1) return cs == 0 ? ms : -mc;
-    return cs == 0 ? mc : ms;
+    // F_R and the potential: (Mc, Ms); F_phi: (Ms, -Mc)
+    const bool sine = (cs == 1) != (type == 1);
+    EnsCol c;
+    c.p = a.coef + ((size_t)mem * a.ncoef + off + (sine && pair ? 1 : 0)) * a.nr;
+    c.lo = jrs - 1;
+    c.hi = (col >> 1) < a.nmem && jrs >= 1 && (pair || !sine) ? krs - 1 : -1;
+    c.last = a.nr - 1;
+    c.neg = type == 1 && cs == 1;
+    return c;
 }
 
 __device__ __forceinline__ bool ens_valid(const EnsGemmArgs &a, int type, int m) {
@@ -470,14 +730,20 @@ struct SplitOps {
 };
 
 __device__ __forceinline__ void load_ops(const EnsGemmArgs &a, SplitOps &o, size_t rowoff,
-                                         size_t wstride, int type, int m, bool pair, int off,
-                                         int k, int col) {
+                                         size_t wstride, const EnsCol &c, int k) {
+    // (rows are a multiple of 32 words long: 16-byte loads.  The column's
+    // loads are unconditional, within its ring row: none waits for a test.)
+    const unsigned short *g = a.gsp + rowoff + k;
+    o.a1 = *reinterpret_cast<const gh_v8bf *>(g);
+    o.a2 = *reinterpret_cast<const gh_v8bf *>(g + wstride);
+    o.a3 = *reinterpret_cast<const gh_v8bf *>(g + 2 * wstride);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = c.p[min(k + j, c.last)];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        o.a1[j] = bf16_bits(a.gsp[rowoff + k + j]);
-        o.a2[j] = bf16_bits(a.gsp[wstride + rowoff + k + j]);
-        o.a3[j] = bf16_bits(a.gsp[2 * wstride + rowoff + k + j]);
-        const float b = ens_rhs(a, type, m, pair, off, k + j, col);
+        float b = k + j >= c.lo && k + j <= c.hi ? v[j] : 0.f;
+        if (c.neg) b = -b;
         const unsigned short h1 = bf16_rn(b);
         const float r1 = b - bf16_to_f(h1);
         const unsigned short h2 = bf16_rn(r1);
@@ -504,11 +770,12 @@ __global__ __launch_bounds__(64 * WPB) void ens_gemm16_kernel(EnsGemmArgs a) {
     gh_v4f acc = {0.f, 0.f, 0.f, 0.f}, lo = acc;   // x1 y1 terms; the five corrections
     const int col = tn * 16 + (lane & 15), kq = 8 * (lane >> 4);
     if (valid) {
+        const EnsCol c = ens_col(a, type, pair, off, col);
         const size_t wstride = 3ull * a.ng * a.nrp * a.nrp;
         const size_t rowoff = ((size_t)(type * a.ng + m) * a.nrp + tm * 16 + (lane & 15)) * a.nrp;
         for (int k0 = 0; k0 < a.nrp; k0 += 32) {
             SplitOps o;
-            load_ops(a, o, rowoff, wstride, type, m, pair, off, k0 + kq, col);
+            load_ops(a, o, rowoff, wstride, c, k0 + kq);
             lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a3, o.b1, lo, 0, 0, 0);
             lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a2, o.b2, lo, 0, 0, 0);
             lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a1, o.b3, lo, 0, 0, 0);
@@ -538,11 +805,12 @@ __global__ __launch_bounds__(64) void ens_gemm32_kernel(EnsGemmArgs a) {
     for (int i = 0; i < 16; i++) acc[i] = lo[i] = 0.f;
     const int col = tn * 32 + (lane & 31), kq = 8 * (lane >> 5);
     if (valid) {
+        const EnsCol c = ens_col(a, type, pair, off, col);
         const size_t wstride = 3ull * a.ng * a.nrp * a.nrp;
         const size_t rowoff = ((size_t)(type * a.ng + m) * a.nrp + tm * 32 + (lane & 31)) * a.nrp;
         for (int k0 = 0; k0 < a.nrp; k0 += 16) {
             SplitOps o;
-            load_ops(a, o, rowoff, wstride, type, m, pair, off, k0 + kq, col);
+            load_ops(a, o, rowoff, wstride, c, k0 + kq);
             lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.a3, o.b1, lo, 0, 0, 0);
             lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.a2, o.b2, lo, 0, 0, 0);
             lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.a1, o.b3, lo, 0, 0, 0);
