@@ -589,15 +589,16 @@ static int unload_all(galhip_ctx *c, void *x, void *y, void *vx, void *vy, int32
     long long n = c->n;
     if (n <= 0) return 0;
     // planar, in load order, into the second particle buffer and the sort
-    // keys (both free outside a sort), then straight to the caller's arrays
+    // keys, through the sort's index (all free outside a sort), then straight to the caller's arrays
     const size_t es = esize(c);
     unsigned char *stage = (unsigned char *)c->xv2;
     int *zs = (int *)c->key;
+    HIPCHK(launch_inverse_order(c->id, c->perm, n, c->s));
     if (c->prec == GALHIP_FP32)
-        HIPCHK(launch_deinterleave<float>((const float4 *)c->xv, c->zone, c->id, (float *)stage,
+        HIPCHK(launch_deinterleave<float>((const float4 *)c->xv, c->zone, c->perm, (float *)stage,
                                           zs, n, c->s));
     else
-        HIPCHK(launch_deinterleave<double>((const double4 *)c->xv, c->zone, c->id,
+        HIPCHK(launch_deinterleave<double>((const double4 *)c->xv, c->zone, c->perm,
                                            (double *)stage, zs, n, c->s));
     const CopySegment seg[5] = {{x, stage, es * n},
                                 {y, stage + es * n, es * n},
