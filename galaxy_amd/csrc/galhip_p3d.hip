@@ -1112,14 +1112,11 @@ template <typename R> __host__ __device__ constexpr size_t tz_words(size_t P) {
     return 2 * (P + (P >> tz_shift<R>()) + 1);
 }
 template <typename R> __device__ __forceinline__ int tz_at(int idx) {
-    return 2 * (idx + (idx >> tz_shift<R>()));
+    return idx + (idx >> tz_shift<R>());
 }
 template <typename R>
-__device__ __forceinline__ void tz_stage(const R *twz, int P, R *tz) {
-    for (int e = threadIdx.x; e < P; e += blockDim.x) {
-        tz[tz_at<R>(e)] = twz[2 * e];
-        tz[tz_at<R>(e) + 1] = twz[2 * e + 1];
-    }
+__device__ __forceinline__ void tz_stage(const R *twz, int P, typename Vec2<R>::T *tz) {
+    for (int e = threadIdx.x; e < P; e += blockDim.x) tz[tz_at<R>(e)] = mk2(twz[2 * e], twz[2 * e + 1]);
 }
 
 // The ring of a vertical transform's block: consecutive blocks go to the eight
@@ -1137,8 +1134,9 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_zfwd_kernel(P3SolveArgs<R> a) {
     extern __shared__ unsigned char p3_lds[];
     const int ngz = a.ngz, P = 2 * ngz, nm = a.nm;
     const int s0 = blockIdx.y * CB, ncol = min(CB, nm - s0);
-    R *tz = (R *)p3_lds;                      // [P][2]
-    R *col = tz + tz_words<R>(P);             // [ngz][CB]
+    typedef typename Vec2<R>::T R2;
+    R2 *tz = (R2 *)p3_lds;                    // [P]
+    R *col = (R *)p3_lds + tz_words<R>(P);             // [ngz][CB]
     const int ir = p3_ring(a.nr) + 1, tid = threadIdx.x;
     const int jrs = a.ranges[0], krs = a.ranges[1];
     if (jrs < 1 || ir < jrs || ir > krs) return;
@@ -1159,13 +1157,12 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_zfwd_kernel(P3SolveArgs<R> a) {
         int idx = 0;
 #pragma unroll 4
         for (int p = 0; p < ngz; p++) {
-            const int t = tz_at<R>(idx);
-            const R w0 = tz[t], w1 = tz[t + 1];
+            const R2 w = tz[tz_at<R>(idx)];
 #pragma unroll
             for (int c = 0; c < CB; c++) {
                 const R v = col[p * CB + c];
-                sa[c] += v * w0;
-                sb[c] += v * w1;
+                sa[c] += v * w.x;
+                sb[c] += v * w.y;
             }
             idx += k;
             if (idx >= P) idx -= P;
@@ -1255,8 +1252,9 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_zinv_kernel(P3SolveArgs<R> a) {
     extern __shared__ unsigned char p3_lds[];
     const int ngz = a.ngz, P = 2 * ngz, nm = a.nm;
     const int s0 = blockIdx.z * CB, ncol = min(CB, nm - s0);
-    R *tz = (R *)p3_lds;                      // [P][2]
-    R *h = tz + tz_words<R>(P);               // [P][CB]
+    typedef typename Vec2<R>::T R2;
+    R2 *tz = (R2 *)p3_lds;                    // [P]
+    R *h = (R *)p3_lds + tz_words<R>(P);               // [P][CB]
     const int ir = p3_ring(a.nr) + 1, type = blockIdx.y, tid = threadIdx.x;
     const int jrs = a.ranges[0], jrf = a.ranges[2], krf = a.ranges[3];
     if (jrs < 1 || ir < jrf || ir > krf) return;
@@ -1278,13 +1276,12 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_zinv_kernel(P3SolveArgs<R> a) {
         int idx = q;
 #pragma unroll 4
         for (int k = 1; k < ngz; k++) {
-            const int t = tz_at<R>(idx);
-            const R w0 = tz[t], w1 = tz[t + 1];
+            const R2 w = tz[tz_at<R>(idx)];
             const R *hk = h + (2 * k - 1) * CB;
             // (v + 2 x rounds as the fused product does: 2 x is exact)
 #pragma unroll
             for (int c = 0; c < CB; c++)
-                v[c] = fma((R)2, hk[c] * w0 - hk[CB + c] * w1, v[c]);
+                v[c] = fma((R)2, hk[c] * w.x - hk[CB + c] * w.y, v[c]);
             idx += q;
             if (idx >= P) idx -= P;
         }
@@ -1619,8 +1616,8 @@ static dim3 p3_lanes(int n) { return dim3(std::min(P3_BLOCK, (n + 63) / 64 * 64)
 // The vertical transforms by CB columns a block.  The forward transform takes
 // three.  The inverse reads a column twice as often as it multiplies it, from
 // LDS: nine columns share a twiddle (three types of 200 rings, 17 columns:
-// 49 us, three at a time 60) if that leaves four blocks a CU, else three, for
-// more blocks (three types of 61 rings, 9 columns, FP64: 22 us and 10 us).
+// 46 us, three at a time 60) if that leaves four blocks a CU, else three, for
+// more blocks (three types of 61 rings, 9 columns, FP64: 22 us and 9.8 us).
 // With fewer columns in the context, no more of them than it has stand in LDS.
 template <typename R, int CB>
 static hipError_t p3_vertical(const P3SolveArgs<R> &a, bool inverse, hipStream_t s) {
