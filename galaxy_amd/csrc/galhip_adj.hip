@@ -171,46 +171,36 @@ constexpr int ADJ_TILE = 1024;   // LDS window cells (x 2 components x 8 B)
 // spokes: the block accumulates them in LDS (FP64 LDS atomics) and adds
 // each touched cell to the grid with one global atomic; a block whose
 // window exceeds the tile adds every corner globally.
+// Latency bounds it (57 MB, 11 us, at 1e6 particles): every load is issued
+// before the first store, which loads would wait for, and the spokes are
+// counted from the block's middle particle instead of its first on-grid one,
+// which took two barriers to find.  1e6 particles: 30.3 -> 28.4 us (two or
+// four particles per thread 30.2, 35.4).
 template <typename R>
 __global__ __launch_bounds__(GH_BLOCK) void adj_scatter_kernel(AdjArgs<R> a) {
+    typedef typename Vec2<R>::T R2;
     __shared__ double tile[2][ADJ_TILE];
-    __shared__ int s_first, s_sref, s_rmin, s_rmax, s_dmin, s_dmax;
+    __shared__ int s_rmin, s_rmax, s_dmin, s_dmax;
     const int tid = threadIdx.x, lane = tid & 63, na = a.na, half = na >> 1;
-    const long long i = (long long)blockIdx.x * GH_BLOCK + tid;
+    const long long n = a.n, base = (long long)blockIdx.x * GH_BLOCK;
+    const int nblk = (int)min((long long)GH_BLOCK, n - base);
+    const long long i = base + min(tid, nblk - 1);
+    const int z = a.zone[i];
+    const R2 cu = a.ut[i];
+    const double lx = a.lam[i], ly = a.lam[n + i];
+    const double lax = a.lam[2 * n + i] + lx, lay = a.lam[3 * n + i] + ly;
+    const int sref = min(max((int)a.ut[base + (nblk >> 1)].y, 0), na - 1);
     if (tid == 0) {
-        s_first = INT_MAX;
         s_rmin = INT_MAX;
         s_rmax = -1;
         s_dmin = INT_MAX;
         s_dmax = INT_MIN;
     }
-    const bool in = i < a.n;
-    const long long n = a.n, p = i;
-    double lax = 0.0, lay = 0.0;
-    if (in) {
-        lax = a.lam[2 * n + p] + a.lam[p];
-        lay = a.lam[3 * n + p] + a.lam[n + p];
-        a.lam[2 * n + p] = lax;
-        a.lam[3 * n + p] = lay;
-    }
-    const bool on = in && a.zone[i] == 1;
-    double w[4] = {0.0, 0.0, 0.0, 0.0}, wu[4], wt[4];
-    int ring = 0, spoke = 0;
-    if (on) {
-        const typename Vec2<R>::T cu = a.ut[i];
-        cic_grad((double)cu.x, (double)cu.y, a.nr, na, ring, spoke, w, wu, wt);
-    }
     __syncthreads();
-    // reference spoke: the first on-grid particle's (one atomic per wave)
-    {
-        const unsigned long long bm = __ballot(on);
-        if (bm && lane == __ffsll((long long)bm) - 1) atomicMin(&s_first, tid);
-    }
-    __syncthreads();
-    if (tid == s_first) s_sref = spoke;
-    __syncthreads();
-    if (s_first == INT_MAX) return;   // no on-grid particle: nothing to add
-    const int sref = s_sref;
+    const bool on = tid < nblk && z == 1;
+    double w[4], wu[4], wt[4];
+    int ring, spoke;
+    cic_grad((double)cu.x, (double)cu.y, a.nr, na, ring, spoke, w, wu, wt);
     int d = spoke - sref;
     if (d < -half) d += na;
     else if (d >= half) d -= na;
@@ -226,7 +216,8 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_scatter_kernel(AdjArgs<R> a) {
     }
     __syncthreads();
     const int r0 = s_rmin, d0 = s_dmin;
-    const int tw = s_dmax - d0 + 2, th = s_rmax - r0 + 2;
+    const bool some = s_rmax >= 0;   // an on-grid particle: something to add
+    const int tw = some ? s_dmax - d0 + 2 : 0, th = some ? s_rmax - r0 + 2 : 0;
     const bool use_tile = th * tw <= ADJ_TILE;
     const int tlen = use_tile ? th * tw : 0;
     for (int j = tid; j < tlen; j += GH_BLOCK) {
@@ -234,6 +225,10 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_scatter_kernel(AdjArgs<R> a) {
         tile[1][j] = 0.0;
     }
     __syncthreads();
+    if (tid < nblk) {
+        a.lam[2 * n + i] = lax;
+        a.lam[3 * n + i] = lay;
+    }
     if (on) {
         if (use_tile) {
             const int b = (ring - r0) * tw + (d - d0);
@@ -340,8 +335,12 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_gather_kernel(AdjArgs<R> a) {
 // block per field ring: polcat transposed, then the transpose of p2fsyn's
 // synthesis for F_R and F_phi -> wbar (zero outside the field range)
 constexpr int ADJ_MAX_NA = 2048;
+// A harmonic is a wavefront's chain of dependent loads: 16 wavefronts a block
+// take them side by side (4: 6.2 and 10.7 us at 128 x 256, 9 harmonics; 16:
+// 4.8 and 7.9).
+constexpr int ADJ_SOLVE_BLOCK = 1024;
 
-__global__ __launch_bounds__(GH_BLOCK) void adj_wbar_kernel(AdjSolveArgs a) {
+__global__ __launch_bounds__(ADJ_SOLVE_BLOCK) void adj_wbar_kernel(AdjSolveArgs a) {
     __shared__ double gt[2][ADJ_MAX_NA];
     const int ir = blockIdx.x + 1, tid = threadIdx.x, na = a.na, nr = a.nr;
     const int lane = tid & 63, wave = tid >> 6;
@@ -349,9 +348,9 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_wbar_kernel(AdjSolveArgs a) {
     const bool live = jrs >= 1 && ir >= jrf && ir <= krf;
     const size_t row = (size_t)(ir - 1) * na;
     if (!live)
-        for (int j = tid; j < na; j += GH_BLOCK) a.gx[row + j] = a.gy[row + j] = 0.0;
+        for (int j = tid; j < na; j += ADJ_SOLVE_BLOCK) a.gx[row + j] = a.gy[row + j] = 0.0;
     else
-        for (int j = tid; j < na; j += GH_BLOCK) {
+        for (int j = tid; j < na; j += ADJ_SOLVE_BLOCK) {
             const double c = a.twd[2 * j], s = a.twd[2 * j + 1];
             const double gx = a.gx[row + j], gy = a.gy[row + j];
             // the sums of the next step start at zero
@@ -362,7 +361,7 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_wbar_kernel(AdjSolveArgs a) {
         }
     __syncthreads();
     const int maz = min(a.mmax - 2, a.ng - 1);
-    for (int m = wave; m < a.ng; m += GH_BLOCK / 64) {
+    for (int m = wave; m < a.ng; m += ADJ_SOLVE_BLOCK / 64) {
         const bool keep = live && !a.lg[m];
         double sc[2] = {0.0, 0.0}, ss[2] = {0.0, 0.0};
         if (keep) {
@@ -407,7 +406,7 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_wbar_kernel(AdjSolveArgs a) {
 // block per source ring: the transposed Green's contraction (p2conv) and
 // the transposed forward transform (p2manl) -> rbar (zero outside the
 // source range)
-__global__ __launch_bounds__(GH_BLOCK) void adj_rbar_kernel(AdjSolveArgs a) {
+__global__ __launch_bounds__(ADJ_SOLVE_BLOCK) void adj_rbar_kernel(AdjSolveArgs a) {
     __shared__ double mc[64], ms[64];
     const int is = blockIdx.x + 1, tid = threadIdx.x, na = a.na, nr = a.nr, ng = a.ng;
     const int lane = tid & 63, wave = tid >> 6;
@@ -415,7 +414,7 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_rbar_kernel(AdjSolveArgs a) {
     const bool live = jrs >= 1 && is >= jrs && is <= krs;
     const size_t row = (size_t)(is - 1) * na;
     const int maz = min(a.mmax - 2, ng - 1);
-    for (int m = wave; m < ng; m += GH_BLOCK / 64) {
+    for (int m = wave; m < ng; m += ADJ_SOLVE_BLOCK / 64) {
         double c = 0.0, s = 0.0;
         if (live && !a.lg[m]) {
             const bool azim = m >= 1 && m <= maz;
@@ -425,6 +424,7 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_rbar_kernel(AdjSolveArgs a) {
             const double *ws0 = a.wbar + (((size_t)0 * 2 + 1) * ng + m) * nr;
             const double *wc1 = a.wbar + (((size_t)1 * 2 + 0) * ng + m) * nr;
             const double *ws1 = a.wbar + (((size_t)1 * 2 + 1) * ng + m) * nr;
+#pragma unroll 2
             for (int ir = jrf + lane; ir <= krf; ir += 64) {
                 const double G0 = g0[(size_t)(ir - 1) * nr + is - 1];
                 c += G0 * wc0[ir - 1];
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(GH_BLOCK) void adj_rbar_kernel(AdjSolveArgs a) {
         }
     }
     __syncthreads();
-    for (int j = tid; j < na; j += GH_BLOCK) {
+    for (int j = tid; j < na; j += ADJ_SOLVE_BLOCK) {
         double v = 0.0;
         if (live) {
             v = mc[0];
@@ -1104,9 +1104,9 @@ static AdjSolveArgs adj_solve_args(galhip_ctx *c) {
 static int adj_solve(galhip_ctx *c) {
     if (c->na > ADJ_MAX_NA || c->ng > 64) return gh_fail(GALHIP_EINVAL, "grid too large for the adjoint");
     AdjSolveArgs a = adj_solve_args(c);
-    hipLaunchKernelGGL(adj_wbar_kernel, dim3(c->nr), dim3(GH_BLOCK), 0, c->s, a);
+    hipLaunchKernelGGL(adj_wbar_kernel, dim3(c->nr), dim3(ADJ_SOLVE_BLOCK), 0, c->s, a);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(adj_rbar_kernel, dim3(c->nr), dim3(GH_BLOCK), 0, c->s, a);
+    hipLaunchKernelGGL(adj_rbar_kernel, dim3(c->nr), dim3(ADJ_SOLVE_BLOCK), 0, c->s, a);
     HIPCHK(hipGetLastError());
     return 0;
 }

@@ -6,12 +6,14 @@
 //   harmonics m < ng, as a direct real DFT against a twiddle table held in
 //   L2: for the harmonic counts used here (ng <= 33 of na/2+1) this costs
 //   about as much as a radix FFT and keeps exact FFTPACK conventions
-//   (half-complex a_m = sum x cos, b_m = -sum x sin).  Optionally performs
-//   the masscl of the next push (masscl.f:67-146) on its ring.
+//   (half-complex a_m = sum x cos, b_m = -sum x sin).
 // synth_kernel (one block per field ring): p2conv's radial contraction with
 //   the per-harmonic Green's matrices (p2conv.f:95-186), p2fsyn's inverse
 //   transform and 1/na (p2fsyn.f:40-52) and polcat (polcat.f:26-40), writing
-//   interleaved (F_x, F_y) and the potential.
+//   interleaved (F_x, F_y) and the potential; also the masscl of the next push
+//   (masscl.f:67-146) on its ring.
+// analyse_rows_kernel, synth_rows_kernel: the same for several rings at once,
+//   for ensembles.
 // green_kernel: p2grnm's table construction in FP64 (p2grnm.f:98-203):
 //   kernel samples (radfor/azifor/grnfun), DCT-I / DST-I over the half
 //   circle, harmonic filter, p2gwrt's [m][field ring][source ring] layout.
