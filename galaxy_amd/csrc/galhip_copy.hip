@@ -3,16 +3,19 @@
 //
 // A large hipMemcpy to pageable memory runs at 10 GB/s into pages not yet
 // touched (17 GB/s into touched ones): one thread zeroes the pages and copies.
-// Here the device copies into pinned chunks (55 GB/s) while several threads
-// move the chunks that have arrived, so that first touches and copies go on
-// together; loads the other way round.  200 MB in five arrays: unload 20.8 ->
-// 5.6 ms, load 10.4 -> 5.9 ms (with the zone check on the device).  Chunks of
-// 1 MiB: unload 7.9 ms, of 8 MiB 5.2; 4 threads 6.4, 12 threads 5.5.
+// An unload of many bytes goes through pinned chunks (55 GB/s) while several
+// threads move the chunks that have arrived, so that first touches and copies
+// go on together: 200 MB in five arrays 20.8 -> 5.6 ms.  Chunks of 1 MiB: 7.9
+// ms, of 8 MiB 5.2; 4 threads 6.4, 12 threads 5.5.
+// Loads stay plain copies: their pages are there, staging took 1e7 particles
+// from 7.9 to 5.9 ms only, and 24 MB loaded beside a busy host thread took 14
+// ms staged and 1.5 plain.  (Their gain, 10.4 -> 7.9 ms, is the zone check on
+// the device.)
 #include "galhip_ctx.h"
 
 #include <algorithm>
-#include <atomic>
 #include <climits>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -68,10 +71,12 @@ struct Piece {
     size_t bytes;
 };
 
-// The pieces through the pinned chunks of buf; false if it could not be set up
-// (nothing has been copied then) or, with err set, if a copy failed.
-bool staged(const std::vector<Piece> &pieces, bool to_host, char *buf, hipStream_t s,
-            hipError_t *err) {
+// The pieces to the host through the pinned chunks of buf; false if it could
+// not be set up (nothing has been copied then) or, with err set, if a copy
+// failed.  Whoever waits sleeps: threads that yield instead keep the CPU, by
+// slices of 4 ms, from a thread with work on it once the process is busy
+// otherwise.
+bool staged(const std::vector<Piece> &pieces, char *buf, hipStream_t s, hipError_t *err) {
     const int n = (int)pieces.size();
     const int nthr = (int)std::min<unsigned>(MAX_THREADS,
                                              std::max(1u, std::thread::hardware_concurrency()));
@@ -79,25 +84,25 @@ bool staged(const std::vector<Piece> &pieces, bool to_host, char *buf, hipStream
     int nev = 0;
     while (nev < NBUF && hipEventCreateWithFlags(&ev[nev], hipEventDisableTiming) == hipSuccess)
         nev++;
-    // ready: pieces the threads may move; done[i]: threads through with piece i
-    std::atomic<int> ready{0};
-    std::atomic<bool> stop{false};
-    std::vector<std::atomic<int>> done(n);
-    for (auto &d : done) d.store(0);
+    std::mutex mu;
+    std::condition_variable go, moved;
+    int ready = 0;                       // pieces the threads may move
+    bool stop = false;
+    std::vector<int> left(n, nthr);      // threads that have not moved their share
     auto move = [&](int w) {
         for (int i = 0; i < n; i++) {
-            while (ready.load(std::memory_order_acquire) <= i) {
-                if (stop.load()) return;
-                std::this_thread::yield();
+            {
+                std::unique_lock<std::mutex> lock(mu);
+                go.wait(lock, [&] { return stop || ready > i; });
+                if (ready <= i) return;
             }
             // page-aligned shares, so that two threads do not touch one page
             const size_t share = ((pieces[i].bytes + nthr - 1) / nthr + 4095) / 4096 * 4096;
             const size_t lo = std::min(pieces[i].bytes, w * share);
             const size_t hi = std::min(pieces[i].bytes, lo + share);
-            char *pin = buf + (size_t)(i % NBUF) * CHUNK;
-            if (to_host) memcpy(pieces[i].host + lo, pin + lo, hi - lo);
-            else memcpy(pin + lo, pieces[i].host + lo, hi - lo);
-            done[i].fetch_add(1, std::memory_order_release);
+            memcpy(pieces[i].host + lo, buf + (size_t)(i % NBUF) * CHUNK + lo, hi - lo);
+            std::lock_guard<std::mutex> lock(mu);
+            if (--left[i] == 0) moved.notify_one();
         }
     };
     std::vector<std::thread> team;
@@ -110,39 +115,38 @@ bool staged(const std::vector<Piece> &pieces, bool to_host, char *buf, hipStream
             ok = false;
         }
     }
-    auto wait_done = [&](int i) {
-        while (done[i].load(std::memory_order_acquire) < nthr) std::this_thread::yield();
+    auto release = [&](int k) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            ready = k;
+        }
+        go.notify_all();
     };
     hipError_t e = hipSuccess;
-    if (ok && to_host) {
+    if (ok) {
         for (int i = 0; i < n && e == hipSuccess; i++) {
-            if (i >= NBUF) wait_done(i - NBUF);
+            if (i >= NBUF) {
+                std::unique_lock<std::mutex> lock(mu);
+                moved.wait(lock, [&] { return left[i - NBUF] == 0; });
+            }
             e = hipMemcpyAsync(buf + (size_t)(i % NBUF) * CHUNK, pieces[i].dev, pieces[i].bytes,
                                hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipEventRecord(ev[i % NBUF], s);
             if (i > 0 && e == hipSuccess) {
                 e = hipEventSynchronize(ev[(i - 1) % NBUF]);
-                if (e == hipSuccess) ready.store(i, std::memory_order_release);
+                if (e == hipSuccess) release(i);
             }
         }
         if (e == hipSuccess) e = hipEventSynchronize(ev[(n - 1) % NBUF]);
-        if (e == hipSuccess) ready.store(n, std::memory_order_release);
-    } else if (ok) {
-        ready.store(std::min(n, NBUF), std::memory_order_release);
-        for (int i = 0; i < n && e == hipSuccess; i++) {
-            wait_done(i);
-            e = hipMemcpyAsync(pieces[i].dev, buf + (size_t)(i % NBUF) * CHUNK, pieces[i].bytes,
-                               hipMemcpyHostToDevice, s);
-            if (e == hipSuccess) e = hipEventRecord(ev[i % NBUF], s);
-            // the chunk before this one is free for its next piece once copied
-            if (i > 0 && i - 1 + NBUF < n && e == hipSuccess) {
-                e = hipEventSynchronize(ev[(i - 1) % NBUF]);
-                if (e == hipSuccess) ready.store(i + NBUF, std::memory_order_release);
-            }
-        }
-        if (e == hipSuccess) e = hipEventSynchronize(ev[(n - 1) % NBUF]);
+        if (e == hipSuccess) release(n);
     }
-    if (!ok || e != hipSuccess) stop.store(true);
+    if (!ok || e != hipSuccess) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            stop = true;
+        }
+        go.notify_all();
+    }
     for (auto &t : team) t.join();
     for (int k = 0; k < nev; k++) (void)hipEventDestroy(ev[k]);
     if (e != hipSuccess) {
@@ -223,16 +227,16 @@ CopyUser::~CopyUser() {
 }
 
 // Copies the segments (host, device, bytes) on the context's stream and waits
-// for them.  Staged from STAGED_MIN bytes in all, plain copies below it: starting
-// the threads costs 0.2 ms, 8 MB in five arrays 0.79 ms staged and 0.37 plain
-// to the device, 20 MB 0.89 staged and 1.13 plain.
+// for them.  To the host staged from STAGED_MIN bytes in all, plain copies below
+// it: starting the threads costs 0.1 ms, 4 MB in five arrays take 0.34 ms
+// staged and 0.24 plain, 8 MB 0.42 and 0.50, 20 MB 0.7 and 1.2.
 int copy_segments(const galhip_ctx *c, const CopySegment *seg, int nseg, bool to_host) {
     // (a plain copy that finds the stream busy takes 30 us longer)
     HIPCHK(hipStreamSynchronize(c->s));
     size_t total = 0;
     for (int k = 0; k < nseg; k++)
         if (seg[k].host) total += seg[k].bytes;
-    if (total >= STAGED_MIN) {
+    if (to_host && total >= STAGED_MIN) {
         void *buf = take_buffer();
         if (buf) {
             bool ok = false;
@@ -243,7 +247,7 @@ int copy_segments(const galhip_ctx *c, const CopySegment *seg, int nseg, bool to
                     for (size_t o = 0; seg[k].host && o < seg[k].bytes; o += CHUNK)
                         pieces.push_back({(char *)seg[k].host + o, (char *)seg[k].dev + o,
                                           std::min(CHUNK, seg[k].bytes - o)});
-                ok = staged(pieces, to_host, (char *)buf, c->s, &e);
+                ok = staged(pieces, (char *)buf, c->s, &e);
             } catch (...) {
                 ok = false;
             }
