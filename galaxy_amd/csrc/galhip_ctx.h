@@ -63,8 +63,10 @@ struct galhip_ctx {
     void *sort_tmp;
     size_t sort_tmp_bytes;
     long long *mfx[GH_MAXZ], *moz[GH_MAXZ];
-    int *jrad, *krad, *ranges, *lg_d;   // ring ranges in stripes (widen_range)
+    int *jrad, *krad;      // ring ranges in stripes (widen_range), krad behind jrad
+    int *range_d;          // one grid's combined ranges [2][GH_MAXZ], behind krad
     int rstride;
+    int *ranges, *lg_d;
     long long *counters;              // [0] off-grid count (per grid)
     long long *load_chk;              // zone_load_kernel: [0] first bad index, 4 m + 4 noff
     long long *push_cnt;              // pushes, striped (count_pushes)
@@ -156,6 +158,9 @@ struct galhip_ctx {
 // Row length of the striped ring ranges and their size in ints.
 static int range_stride(int nmem) { return (nmem * GH_MAXZ + 31) / 32 * 32; }
 static size_t range_ints(const galhip_ctx *c) { return (size_t)GH_RANGE_STRIPES * c->rstride; }
+
+// jrad, krad and the combined ranges in one allocation, every range empty.
+int ranges_create(galhip_ctx *c, int nmem);
 
 static size_t esize(const galhip_ctx *c) { return c->prec == GALHIP_FP64 ? 8 : 4; }
 

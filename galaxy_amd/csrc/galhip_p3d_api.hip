@@ -137,9 +137,7 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
         rc |= dalloc(&c->mfx[z], sizeof(long long) * c->mesh);
         rc |= dalloc(&c->moz[z], sizeof(long long) * c->mesh);
     }
-    c->rstride = range_stride(1);
-    rc |= dalloc(&c->jrad, sizeof(int) * range_ints(c));
-    rc |= dalloc(&c->krad, sizeof(int) * range_ints(c));
+    rc |= ranges_create(c, 1);
     rc |= dalloc(&c->ranges, sizeof(int) * 4);
     rc |= dalloc(&c->lg_d, sizeof(int) * c->mmax);
     rc |= dalloc(&c->slot_m_d, sizeof(int) * (nm > 0 ? nm : 1));
@@ -190,9 +188,6 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
         HIPCHK(hipMemcpy(c->slot_p_d, slot_p.data(), sizeof(int) * nm, hipMemcpyHostToDevice));
     }
     HIPCHK(hipMemcpy(c->slot_of_d, slot_of.data(), sizeof(int) * c->mmax, hipMemcpyHostToDevice));
-    std::vector<int> jr(range_ints(c), c->nr), kr(range_ints(c), 0);
-    HIPCHK(hipMemcpy(c->jrad, jr.data(), sizeof(int) * jr.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->krad, kr.data(), sizeof(int) * kr.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->counters, 0, sizeof(long long) * 4));
     HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     HIPCHK(hipMemset(c->fld4, 0, 4 * es * c->mesh));

@@ -388,6 +388,12 @@ __global__ void masscl_kernel(ZonePtrs zp, int mz, long long ncell, int *jrad,
     }
 }
 
+// one grid's combined ranges: out[0..nz), out[GH_MAXZ..)
+__global__ void combine_ranges_kernel(const int *jrad, const int *krad, int rstride, int nz,
+                                      int *out) {
+    combine_ranges(jrad, krad, rstride, nz, out, out + GH_MAXZ);
+}
+
 // ---- many rings at once (ensembles) -------------------------------------------
 //
 // A block of 16 wavefronts per ring suits one grid, whose few rings leave most
@@ -905,6 +911,12 @@ hipError_t launch_fill_i32(int *p, int v, long long n, hipStream_t s) {
     hipLaunchKernelGGL(fill_kernel<int>,
                        dim3((unsigned)((n + GH_BLOCK - 1) / GH_BLOCK)),
                        dim3(GH_BLOCK), 0, s, p, v, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_combine_ranges(const int *jrad, const int *krad, int rstride, int nz, int *out,
+                                 hipStream_t s) {
+    hipLaunchKernelGGL(combine_ranges_kernel, dim3(1), dim3(64), 0, s, jrad, krad, rstride, nz, out);
     return hipGetLastError();
 }
 
