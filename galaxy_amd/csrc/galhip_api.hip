@@ -565,7 +565,7 @@ extern "C" int galhip_restrt(galhip_ctx *c, int64_t n, const void *x,
     size_t es = esize(c);
     rc = load_zones(c, n, iz);
     if (rc) return rc;
-    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
+    HIPCHK(reset_pushes(c));
     c->qbits = qbits_for(n);
     c->order_ver++;
     if (n == 0) return 0;
@@ -1673,7 +1673,7 @@ extern "C" int galhip_ens_restrt(galhip_ctx *c, const int64_t *count, const void
     size_t es = esize(c);
     rc = load_zones(c, n, iz);
     if (rc) return rc;
-    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
+    HIPCHK(reset_pushes(c));
     drop_graphs(c);
     if (n == 0) return 0;
     rc = load_xv(c, n, x, y, vx, vy);

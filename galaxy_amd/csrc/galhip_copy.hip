@@ -270,7 +270,7 @@ int copy_segments(const galhip_ctx *c, const CopySegment *seg, int nseg, bool to
 // The zones of a load: the context's zones and off-grid counts stay as they
 // were if one is outside 1..nz+1.  Checked on the device from ZONES_DEVICE
 // particles on, where the host's loop begins to cost more than the round trip
-// of the check (2e5: 0.37 ms a load both ways; 2.5e4: 0.19 ms on the host, 0.21
+// of the check (1.4e5: 0.30 ms a load both ways; 1e3: 0.12 ms on the host, 0.145
 // on the device; 1e7: 14 ms less on the device).
 int load_zones(galhip_ctx *c, long long n, const int32_t *iz) {
     if (n < ZONES_DEVICE) {

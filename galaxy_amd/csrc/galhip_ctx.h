@@ -215,6 +215,11 @@ hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, in
                          hipStream_t);
 }  // namespace gh
 
+// a load starts the push count again
+static inline hipError_t reset_pushes(galhip_ctx *c) {
+    return gh::launch_fill_i64(c->push_cnt, 0, 8 * GH_PUSH_STRIPES, c->s);
+}
+
 // adjoint storage (galhip_adj.hip)
 void adj_free(galhip_ctx *c);
 

@@ -298,7 +298,7 @@ extern "C" int galhip_restrt3(galhip_ctx *c, int64_t n, const void *x, const voi
     const size_t es = esize(c);
     rc = load_zones(c, n, iz);
     if (rc) return rc;
-    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
+    HIPCHK(reset_pushes(c));
     if (n > 0) {
         // the planar arrays through the second record buffer (free outside a
         // sort, 8 n values), interleaved on the device
