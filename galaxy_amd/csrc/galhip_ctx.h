@@ -206,7 +206,6 @@ int copy_segments(const galhip_ctx *c, const CopySegment *seg, int nseg, bool to
 int load_zones(galhip_ctx *c, long long n, const int32_t *iz);
 
 namespace gh {
-hipError_t launch_inverse_order(const unsigned *, unsigned *, long long, hipStream_t);
 hipError_t launch_planar_lo(const float2 *, const unsigned *, float *, long long, hipStream_t);
 hipError_t launch_d2f(const double *, float *, long long, hipStream_t);
 hipError_t launch_fill_i64(long long *, long long, long long, hipStream_t);

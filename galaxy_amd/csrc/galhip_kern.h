@@ -538,6 +538,10 @@ __device__ __forceinline__ void count_pushes(long long *stripes, unsigned b, int
                      (unsigned long long)n);
 }
 
+// Unloads gather their particles from UNLOAD_GATHER particles on (see
+// deinterleave_kernel).
+constexpr long long UNLOAD_GATHER = 50000;
+
 // ---- kernel argument blocks -------------------------------------------------
 
 struct ZonePtrs {

@@ -79,8 +79,9 @@ hipError_t launch_p3_interleave(const R *s4, const R *s2, typename Vec4<R>::T *r
                                 unsigned *id, long long n, hipStream_t);
 template <typename R>
 hipError_t launch_p3_deinterleave(const typename Vec4<R>::T *rec, const uint8_t *zone,
-                                  const unsigned *id, R *d4, R *d2, int *iz, long long n,
-                                  hipStream_t);
+                                  const unsigned *id, unsigned *inv, R *d4, R *d2, int *iz,
+                                  long long n, hipStream_t);
+hipError_t launch_inverse_order(const unsigned *, unsigned *, long long, hipStream_t);
 template <typename R> hipError_t launch_p3_massgn(const P3Args<R> &, hipStream_t);
 template <typename R> hipError_t launch_p3_push(const P3Args<R> &, hipStream_t);
 template <typename R> hipError_t launch_p3_tmcent(const P3Args<R> &, hipStream_t);

@@ -952,16 +952,17 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_interleave_kernel(const R *__res
 }
 
 // Unload: interleaved storage -> planar arrays in load order, zones widened,
-// from the records' places (inv) as on the p2d grid: 2e7 particles 3930 us when
-// each wrote its seven values where they belong, 790 (and 280 for inv) so.
-template <typename R>
+// from the records' places as on the p2d grid: 2e7 particles 3930 us when
+// each wrote its seven values where they belong, 790 (and 280 for the places) so;
+// 2e4 5.0 us and 2.6 + 2.5.
+template <typename R, bool GATHER>
 __global__ __launch_bounds__(P3_PBLOCK) void p3_deinterleave_kernel(
     const typename Vec4<R>::T *__restrict__ rec, const uint8_t *__restrict__ zone,
-    const unsigned *__restrict__ inv, R *__restrict__ d4, R *__restrict__ d2,
+    const unsigned *__restrict__ ord, R *__restrict__ d4, R *__restrict__ d2,
     int *__restrict__ iz, long long n) {
-    const long long p = (long long)blockIdx.x * P3_PBLOCK + threadIdx.x;
-    if (p >= n) return;
-    const long long i = inv[p];
+    const long long t = (long long)blockIdx.x * P3_PBLOCK + threadIdx.x;
+    if (t >= n) return;
+    const long long o = ord[t], i = GATHER ? o : t, p = GATHER ? t : o;
     const typename Vec4<R>::T a = rec[2 * i];
     const typename Vec4<R>::T b = rec[2 * i + 1];
     const int z = zone[i];
@@ -1569,11 +1570,19 @@ hipError_t launch_p3_interleave(const R *s4, const R *s2, typename Vec4<R>::T *r
 
 template <typename R>
 hipError_t launch_p3_deinterleave(const typename Vec4<R>::T *rec, const uint8_t *zone,
-                                  const unsigned *inv, R *d4, R *d2, int *iz, long long n,
-                                  hipStream_t s) {
+                                  const unsigned *id, unsigned *inv, R *d4, R *d2, int *iz,
+                                  long long n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(p3_deinterleave_kernel<R>, dim3(p3_blocks(n)), dim3(P3_PBLOCK), 0, s,
-                       rec, zone, inv, d4, d2, iz, n);
+    const dim3 grid(p3_blocks(n)), block(P3_PBLOCK);
+    if (n < UNLOAD_GATHER) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_deinterleave_kernel<R, false>), grid, block, 0, s,
+                           rec, zone, id, d4, d2, iz, n);
+        return hipGetLastError();
+    }
+    hipError_t e = launch_inverse_order(id, inv, n, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_deinterleave_kernel<R, true>), grid, block, 0, s, rec,
+                       zone, (const unsigned *)inv, d4, d2, iz, n);
     return hipGetLastError();
 }
 
@@ -1689,8 +1698,8 @@ hipError_t launch_p3_green(double *G, const double *twd, const double *twzd, con
     template hipError_t launch_p3_interleave<R>(const R *, const R *, typename Vec4<R>::T *,  \
                                                 unsigned *, long long, hipStream_t);          \
     template hipError_t launch_p3_deinterleave<R>(const typename Vec4<R>::T *, const uint8_t *, \
-                                                  const unsigned *, R *, R *, int *, long long, \
-                                                  hipStream_t);
+                                                  const unsigned *, unsigned *, R *, R *, int *, \
+                                                  long long, hipStream_t);
 P3_INST(float)
 P3_INST(double)
 

@@ -337,12 +337,11 @@ extern "C" int galhip_unload3(galhip_ctx *c, void *x, void *y, void *z, void *vx
     const size_t es = esize(c);
     unsigned char *t4 = (unsigned char *)c->xv2, *t2 = t4 + 4 * es * n;
     int *zs = (int *)c->key;
-    HIPCHK(launch_inverse_order(c->id, c->perm, n, c->s));
     if (c->prec == GALHIP_FP32)
-        HIPCHK(launch_p3_deinterleave<float>((const float4 *)c->xv, c->zone,
-                                             c->perm, (float *)t4, (float *)t2, zs, n, c->s));
+        HIPCHK(launch_p3_deinterleave<float>((const float4 *)c->xv, c->zone, c->id, c->perm,
+                                             (float *)t4, (float *)t2, zs, n, c->s));
     else
-        HIPCHK(launch_p3_deinterleave<double>((const double4 *)c->xv, c->zone, c->perm,
+        HIPCHK(launch_p3_deinterleave<double>((const double4 *)c->xv, c->zone, c->id, c->perm,
                                               (double *)t4, (double *)t2, zs, n, c->s));
     void *dst[6] = {x, y, z, vx, vy, vz};
     CopySegment seg[7];

@@ -996,7 +996,11 @@ __global__ __launch_bounds__(GH_BLOCK) void interleave_kernel(const R *__restric
 // Unload: interleaved storage -> planar arrays in load order, zones widened to
 // int32.  Written where each particle belongs, its five values touch five lines
 // each used for four bytes (1e7: 630 us); so only its place is written (inv),
-// and the records, a line each, are read in load order: 137 + 362 us.
+// and the records, a line each, are read in load order: 137 + 362 us.  A small
+// set stays in the L2, and the second launch costs more than it saves: below
+// UNLOAD_GATHER particles each value is written where it belongs (2e4: 3.7 us
+// against 2.0 + 2.3 and the gap between the launches; 1e5: 7.0 against 2.7 + 2.9
+// and the gap).
 __global__ __launch_bounds__(GH_BLOCK) void inverse_order_kernel(const unsigned *__restrict__ id,
                                                                  unsigned *__restrict__ inv,
                                                                  long long n) {
@@ -1004,15 +1008,16 @@ __global__ __launch_bounds__(GH_BLOCK) void inverse_order_kernel(const unsigned 
     if (i < n) inv[id[i]] = (unsigned)i;
 }
 
-template <typename R>
+// ord: GATHER the places inv, else the load-order ids
+template <typename R, bool GATHER>
 __global__ __launch_bounds__(GH_BLOCK) void deinterleave_kernel(const typename Vec4<R>::T *__restrict__ xv,
                                                                 const uint8_t *__restrict__ zone,
-                                                                const unsigned *__restrict__ inv,
+                                                                const unsigned *__restrict__ ord,
                                                                 R *__restrict__ d,
                                                                 int *__restrict__ iz, long long n) {
-    const long long p = (long long)blockIdx.x * GH_BLOCK + threadIdx.x;
-    if (p >= n) return;
-    const long long i = inv[p];
+    const long long t = (long long)blockIdx.x * GH_BLOCK + threadIdx.x;
+    if (t >= n) return;
+    const long long o = ord[t], i = GATHER ? o : t, p = GATHER ? t : o;
     const typename Vec4<R>::T v = xv[i];
     const int z = zone[i];
     d[p] = v.x;
@@ -1167,13 +1172,22 @@ hipError_t launch_inverse_order(const unsigned *id, unsigned *inv, long long n, 
     return hipGetLastError();
 }
 
+// inv: scratch of n words
 template <typename R>
 hipError_t launch_deinterleave(const typename Vec4<R>::T *xv, const uint8_t *zone,
-                               const unsigned *inv, R *stage, int *iz, long long n,
+                               const unsigned *id, unsigned *inv, R *stage, int *iz, long long n,
                                hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(deinterleave_kernel<R>, dim3(nblocks(n, GH_BLOCK)), dim3(GH_BLOCK), 0, s,
-                       xv, zone, inv, stage, iz, n);
+    const dim3 grid(nblocks(n, GH_BLOCK)), block(GH_BLOCK);
+    if (n < UNLOAD_GATHER) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(deinterleave_kernel<R, false>), grid, block, 0, s, xv,
+                           zone, id, stage, iz, n);
+        return hipGetLastError();
+    }
+    hipError_t e = launch_inverse_order(id, inv, n, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(deinterleave_kernel<R, true>), grid, block, 0, s, xv, zone,
+                       (const unsigned *)inv, stage, iz, n);
     return hipGetLastError();
 }
 
@@ -1211,8 +1225,8 @@ hipError_t launch_permute_all(const PermArgs<R> &p, hipStream_t s) {
     template hipError_t launch_interleave<R>(const R *, typename Vec4<R>::T *, unsigned *, \
                                              long long, hipStream_t);                      \
     template hipError_t launch_deinterleave<R>(const typename Vec4<R>::T *, const uint8_t *, \
-                                               const unsigned *, R *, int *, long long,      \
-                                               hipStream_t);
+                                               const unsigned *, unsigned *, R *, int *,     \
+                                               long long, hipStream_t);
 GH_INST(float)
 GH_INST(double)
 
