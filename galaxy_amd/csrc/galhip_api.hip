@@ -123,6 +123,16 @@ int ranges_create(galhip_ctx *c, int nmem) {
     return 0;
 }
 
+int counters_create(galhip_ctx *c, int nmem) {
+    const size_t np = 8 * GH_PUSH_STRIPES, nc = 4 * (size_t)nmem, words = np + nc + nc + 4;
+    int rc = dalloc(&c->push_cnt, sizeof(long long) * words);
+    if (rc) return rc;
+    c->counters = c->push_cnt + np;
+    c->load_chk = c->counters + nc;
+    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * words));
+    return 0;
+}
+
 // p2dset for one grid (nmem = 1, pmass from the parameters) or an ensemble
 // of nmem grids with per-member particle masses.
 static int p2d_create(const galhip_p2d_params *p, int nmem, const double *pmass,
@@ -217,9 +227,7 @@ static int p2d_create(const galhip_p2d_params *p, int nmem, const double *pmass,
     rc |= ranges_create(c, nmem);
     rc |= dalloc(&c->ranges, sizeof(int) * 4 * nm);
     rc |= dalloc(&c->lg_d, sizeof(int) * c->mmax);
-    rc |= dalloc(&c->counters, sizeof(long long) * 4 * nm);
-    rc |= dalloc(&c->load_chk, sizeof(long long) * 4 * (nm + 1));
-    rc |= dalloc(&c->push_cnt, sizeof(long long) * 8 * GH_PUSH_STRIPES);
+    rc |= counters_create(c, nmem);
     rc |= dalloc(&c->rho, es * cells);
     rc |= dalloc(&c->coef, es * c->ncoef * c->nr * nm);
     rc |= dalloc(&c->fld2, 2 * es * cells);
@@ -249,8 +257,6 @@ static int p2d_create(const galhip_p2d_params *p, int nmem, const double *pmass,
         HIPCHK(hipMemcpy(c->tw, twd.data(), sizeof(double) * 2 * na, hipMemcpyHostToDevice));
     }
     HIPCHK(hipMemcpy(c->lg_d, c->lg.data(), sizeof(int) * c->mmax, hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(c->counters, 0, sizeof(long long) * 4 * nm));
-    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     HIPCHK(hipMemset(c->fld2, 0, 2 * es * cells));
     HIPCHK(hipMemset(c->pot, 0, es * cells));
     HIPCHK(hipMemset(c->rho, 0, es * cells));
@@ -295,8 +301,7 @@ extern "C" int galhip_free(galhip_ctx *c) {
     if (c->p3d) p3_free(c);
     free_particles(c);
     for (int z = 0; z < GH_MAXZ; z++) { dfree(c->mfx[z]); dfree(c->moz[z]); }
-    dfree(c->jrad); dfree(c->ranges); dfree(c->lg_d); dfree(c->counters); dfree(c->load_chk);
-    dfree(c->push_cnt);
+    dfree(c->jrad); dfree(c->ranges); dfree(c->lg_d); dfree(c->push_cnt);
     dfree(c->fp_c);
     dfree(c->rho); dfree(c->coef); dfree(c->fld2); dfree(c->pot); dfree(c->tw); dfree(c->twd);
     if (c->G != (void *)c->Gd) dfree(c->G);

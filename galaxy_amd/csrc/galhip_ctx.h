@@ -67,9 +67,9 @@ struct galhip_ctx {
     int *range_d;          // one grid's combined ranges [2][GH_MAXZ], behind krad
     int rstride;
     int *ranges, *lg_d;
-    long long *counters;              // [0] off-grid count (per grid)
-    long long *load_chk;              // zone_load_kernel: [0] first bad index, 4 m + 4 noff
     long long *push_cnt;              // pushes, striped (count_pushes)
+    long long *counters;              // [0] off-grid count (per grid), behind push_cnt
+    long long *load_chk;              // zone_load_kernel: [0] first bad index, 4 m + 4 noff
     void *rho, *coef, *fld2, *pot, *G, *tw;
     double *Gd, *twd;
     // fixed radial tables as cubic coefficients per interval (radtab_coeffs):
@@ -161,6 +161,8 @@ static size_t range_ints(const galhip_ctx *c) { return (size_t)GH_RANGE_STRIPES 
 
 // jrad, krad and the combined ranges in one allocation, every range empty.
 int ranges_create(galhip_ctx *c, int nmem);
+// push_cnt, counters and load_chk in one allocation, zero.
+int counters_create(galhip_ctx *c, int nmem);
 
 static size_t esize(const galhip_ctx *c) { return c->prec == GALHIP_FP64 ? 8 : 4; }
 

@@ -143,9 +143,7 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
     rc |= dalloc(&c->slot_m_d, sizeof(int) * (nm > 0 ? nm : 1));
     rc |= dalloc(&c->slot_p_d, sizeof(int) * (nm > 0 ? nm : 1));
     rc |= dalloc(&c->slot_of_d, sizeof(int) * c->mmax);
-    rc |= dalloc(&c->counters, sizeof(long long) * 4);
-    rc |= dalloc(&c->load_chk, sizeof(long long) * 8);
-    rc |= dalloc(&c->push_cnt, sizeof(long long) * 8 * GH_PUSH_STRIPES);
+    rc |= counters_create(c, 1);
     rc |= dalloc(&c->rho, es * c->mesh);
     rc |= dalloc(&c->A3, es * c->nr * nm * c->ngz);
     rc |= dalloc(&c->M3, es * c->nr * nm * P);
@@ -188,8 +186,6 @@ extern "C" int galhip_p3dset(const galhip_p3d_params *p, galhip_ctx **out) {
         HIPCHK(hipMemcpy(c->slot_p_d, slot_p.data(), sizeof(int) * nm, hipMemcpyHostToDevice));
     }
     HIPCHK(hipMemcpy(c->slot_of_d, slot_of.data(), sizeof(int) * c->mmax, hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(c->counters, 0, sizeof(long long) * 4));
-    HIPCHK(hipMemset(c->push_cnt, 0, sizeof(long long) * 8 * GH_PUSH_STRIPES));
     HIPCHK(hipMemset(c->fld4, 0, 4 * es * c->mesh));
     HIPCHK(hipMemset(c->rho, 0, es * c->mesh));
     // entries of W no contraction writes (e.g. F_z at k_z = 0) stay zero
