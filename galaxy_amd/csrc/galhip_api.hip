@@ -1043,13 +1043,13 @@ extern "C" int galhip_tmcent(galhip_ctx *c, int32_t start) {
     return c->prec == GALHIP_FP32 ? tmcent_impl<float>(c, start) : tmcent_impl<double>(c, start);
 }
 
-// Partial-sum rows of the p2d integrals kernels: 9 per block of the
-// largest grid, then the 9 totals of every grid.
+// Partial-sum rows of the p2d integrals kernels: 9 sums per block of the
+// largest grid (int_split), then the 9 totals of every grid.
 static long long integrals_nb(const galhip_ctx *c) {
     long long nbmax = 1;
     for (int m = 0; m < c->nmem; m++) {
         const long long nm = c->ens ? c->m_off[m + 1] - c->m_off[m] : c->n;
-        nbmax = std::max(nbmax, (nm + GH_BLOCK - 1) / GH_BLOCK);
+        nbmax = std::max(nbmax, int_split(nm, GH_BLOCK).nb);
     }
     return nbmax;
 }

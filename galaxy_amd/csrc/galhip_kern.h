@@ -538,6 +538,28 @@ __device__ __forceinline__ void count_pushes(long long *stripes, unsigned b, int
                      (unsigned long long)n);
 }
 
+// Particles per thread and blocks of the integrals' kernels for n particles:
+// the one place that the launch and the sizes of the partial sums come from.
+// Several particles share a block's reductions, but a thread takes them one
+// after the other: one while that leaves fewer than 2 INT_BLOCKS blocks, then 2, 4
+// and 8, as many as leave INT_BLOCKS.  us of a whole call, FP32, by particles per
+// thread (1, 2, 4, 8):
+//   p2d 1e5  31 32 36 42   8e5  41 38 40 44   4e6  95 82 79 85   1e7 224 153 142 139
+//   p3d 1e5  34 36 41 51   8e5  47 47 49 60   4e6 108 97 93 98   1e7 238 218 217 227
+constexpr int INT_PT = 8;
+constexpr long long INT_BLOCKS = 2048;
+constexpr int P3_INT_BLOCK = 512;   // threads per block on the p3d grid (p2d: GH_BLOCK)
+struct IntSplit {
+    int per;
+    long long nb;
+};
+inline IntSplit int_split(long long n, int block) {
+    IntSplit s = {INT_PT, 0};
+    while (s.per > 1 && n < INT_BLOCKS * block * s.per) s.per >>= 1;
+    s.nb = (n + (long long)block * s.per - 1) / ((long long)block * s.per);
+    return s;
+}
+
 // Unloads gather their particles from UNLOAD_GATHER particles on (see
 // deinterleave_kernel).
 constexpr long long UNLOAD_GATHER = 50000;

@@ -796,28 +796,27 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_gather_kernel(P3GatherArgs<R> b)
 }
 
 // icheck's global integrals for the 3-D grid (SRC/lib15/icheck.f:24-70):
-// per-block FP64 sums of 11 quantities in a fixed order (P3_INT_PT particles
-// per thread, as on the p2d grid), then a block per quantity adds the block
+// per-block FP64 sums of 11 quantities in a fixed order (int_split's
+// particles per thread, as on the p2d grid), then a block per quantity adds the block
 // sums in a fixed order.  [0] count, [1..3] position, [4..6] velocity per
 // zone-1 step ((v + a/2)/tfac when centred), [7] v^2, [8] Lz, [9] the grid
 // potential interpolated with the particle's own weights (grid particles),
 // [10] the fixed potential of the spherical radius.
 constexpr int NINT3 = 11;
-constexpr int P3_INT_PT = 8;
 
 template <typename R, int J>
-__global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_kernel(P3Args<R> a, int with_pot,
+__global__ __launch_bounds__(P3_INT_BLOCK) void p3_integrals_kernel(P3Args<R> a, int per, int with_pot,
                                                                  const double4 *fp_c, int nfp,
                                                                  double fp_dr, int centred,
                                                                  double *part) {
     typedef typename Vec4<R>::T R4;
-    __shared__ double red[P3_PBLOCK / 64][NINT3];
+    __shared__ double red[P3_INT_BLOCK / 64][NINT3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     double v[NINT3];
 #pragma unroll
     for (int q = 0; q < NINT3; q++) v[q] = 0.0;
-    for (int k = 0; k < P3_INT_PT; k++) {
-        const long long i = ((long long)blockIdx.x * P3_INT_PT + k) * P3_PBLOCK + tid;
+    for (int k = 0; k < per; k++) {
+        const long long i = ((long long)blockIdx.x * per + k) * P3_INT_BLOCK + tid;
         if (i >= a.n) break;
         const int z = a.zone[i];
         if (z >= 1) {
@@ -870,23 +869,23 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_kernel(P3Args<R> a, in
     __syncthreads();
     if (tid < NINT3) {
         double t = 0.0;
-        for (int w = 0; w < P3_PBLOCK / 64; w++) t += red[w][tid];
+        for (int w = 0; w < P3_INT_BLOCK / 64; w++) t += red[w][tid];
         part[(long long)tid * gridDim.x + blockIdx.x] = t;
     }
 }
 
-__global__ __launch_bounds__(P3_PBLOCK) void p3_integrals_sum_kernel(const double *part, int nb,
+__global__ __launch_bounds__(P3_INT_BLOCK) void p3_integrals_sum_kernel(const double *part, int nb,
                                                                      double *out) {
-    __shared__ double red[P3_PBLOCK / 64];
+    __shared__ double red[P3_INT_BLOCK / 64];
     const int tid = threadIdx.x, q = blockIdx.x;
     double t = 0.0;
-    for (int b = tid; b < nb; b += P3_PBLOCK) t += part[(long long)q * nb + b];
+    for (int b = tid; b < nb; b += P3_INT_BLOCK) t += part[(long long)q * nb + b];
     t = wave_sum_dpp(t);
     if ((tid & 63) == 0) red[tid >> 6] = t;
     __syncthreads();
     if (tid == 0) {
         double s = 0.0;
-        for (int w = 0; w < P3_PBLOCK / 64; w++) s += red[w];
+        for (int w = 0; w < P3_INT_BLOCK / 64; w++) s += red[w];
         out[q] = s;
     }
 }
@@ -1596,16 +1595,17 @@ template <typename R>
 hipError_t launch_p3_integrals(const P3Args<R> &a, int with_pot, const double4 *fp_c,
                                int nfp, double fp_dr, int centred,
                                double *part, double *out, hipStream_t s) {
-    const unsigned nb = a.n > 0 ? p3_blocks((a.n + P3_INT_PT - 1) / P3_INT_PT) : 0;
+    const IntSplit sp = int_split(a.n, P3_INT_BLOCK);
+    const unsigned nb = (unsigned)sp.nb;
     if (nb && a.jmass == 3)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_integrals_kernel<R, 3>), dim3(nb), dim3(P3_PBLOCK), 0, s, a,
-                           with_pot, fp_c, nfp, fp_dr, centred, part);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_integrals_kernel<R, 3>), dim3(nb),
+                           dim3(P3_INT_BLOCK), 0, s, a, sp.per, with_pot, fp_c, nfp, fp_dr, centred, part);
     else if (nb)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_integrals_kernel<R, 2>), dim3(nb), dim3(P3_PBLOCK), 0, s, a,
-                           with_pot, fp_c, nfp, fp_dr, centred, part);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_integrals_kernel<R, 2>), dim3(nb),
+                           dim3(P3_INT_BLOCK), 0, s, a, sp.per, with_pot, fp_c, nfp, fp_dr, centred, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(p3_integrals_sum_kernel, dim3(NINT3), dim3(P3_PBLOCK), 0, s, part, (int)nb,
+    hipLaunchKernelGGL(p3_integrals_sum_kernel, dim3(NINT3), dim3(P3_INT_BLOCK), 0, s, part, (int)nb,
                        out);
     return hipGetLastError();
 }

@@ -524,7 +524,7 @@ int p3_tmcent(galhip_ctx *c, int start) {
 // (partials, then the P3_NINT totals), or null to allocate them here.
 template <typename R>
 static int p3_integrals_impl(galhip_ctx *c, int centred, double *out, double *buf) {
-    const long long nb = c->n > 0 ? (c->n + 511) / 512 : 0;
+    const long long nb = int_split(c->n, P3_INT_BLOCK).nb;
     double *part = buf, *dout = buf ? buf + P3_NINT * (nb > 0 ? nb : 1) : nullptr;
     int rc = 0;
     if (!buf)
@@ -549,7 +549,7 @@ static int p3_integrals_impl(galhip_ctx *c, int centred, double *out, double *bu
 }
 
 long long p3_integrals_doubles(const galhip_ctx *c) {
-    const long long nb = c->n > 0 ? (c->n + 511) / 512 : 0;
+    const long long nb = int_split(c->n, P3_INT_BLOCK).nb;
     return P3_NINT * ((nb > 0 ? nb : 1) + 1);
 }
 

@@ -804,17 +804,16 @@ __global__ __launch_bounds__(GH_BLOCK) void stpgrp_group_kernel(PushArgs<R> a,
 // step factor of their zone (the off-grid list that of the top zone).
 // centred: the velocities time-centred as icheck takes them, v + a/2 in
 // the working precision (anlgrp's (v + a/2)/tfac) before the division.  A
-// thread adds INT_PT particles before its block reduces: the wavefront
+// thread adds several particles (int_split) before its block reduces: the wavefront
 // reductions of the nine FP64 sums cost as much as a particle's terms.  Each
 // block writes its sums; a second pass, a block per sum, adds them in a
 // fixed order, so the result does not depend on scheduling.  1e7 particles:
 // kernel 207 -> 131 us, sum of the blocks 190 -> 7 us.
 constexpr int NINT = 9;
-constexpr int INT_PT = 8;       // particles per thread
 constexpr int INT_SUM_BLOCK = 512;
 
 template <typename R>
-__global__ __launch_bounds__(GH_BLOCK) void integrals_kernel(PushArgs<R> a, const R *pot,
+__global__ __launch_bounds__(GH_BLOCK) void integrals_kernel(PushArgs<R> a, int per, const R *pot,
                                                              const double4 *fp_c, int nfp,
                                                              double fp_dr, int centred,
                                                              double *part) {
@@ -823,8 +822,8 @@ __global__ __launch_bounds__(GH_BLOCK) void integrals_kernel(PushArgs<R> a, cons
     double v[NINT];
 #pragma unroll
     for (int q = 0; q < NINT; q++) v[q] = 0.0;
-    for (int k = 0; k < INT_PT; k++) {
-        const long long i = ((long long)blockIdx.x * INT_PT + k) * GH_BLOCK + tid;
+    for (int k = 0; k < per; k++) {
+        const long long i = ((long long)blockIdx.x * per + k) * GH_BLOCK + tid;
         if (i >= a.n) break;
         const int z = a.zone[i];
         if (z >= 1) {
@@ -1119,9 +1118,10 @@ template <typename R>
 hipError_t launch_integrals(const PushArgs<R> &a, const R *pot, const double4 *fp_c,
                             int nfp, double fp_dr, int centred,
                             double *part, double *out, hipStream_t s) {
-    const unsigned nb = a.n > 0 ? nblocks(a.n, GH_BLOCK * INT_PT) : 0;
+    const IntSplit sp = int_split(a.n, GH_BLOCK);
+    const unsigned nb = (unsigned)sp.nb;
     if (nb)
-        hipLaunchKernelGGL(integrals_kernel<R>, dim3(nb), dim3(GH_BLOCK), 0, s, a, pot,
+        hipLaunchKernelGGL(integrals_kernel<R>, dim3(nb), dim3(GH_BLOCK), 0, s, a, sp.per, pot,
                            fp_c, nfp, fp_dr, centred, part);
     hipLaunchKernelGGL(integrals_sum_kernel, dim3(NINT), dim3(INT_SUM_BLOCK), 0, s,
                        (const double *)part, (int)nb, out);

@@ -223,9 +223,9 @@ int galhip_integrals(galhip_ctx *ctx, int32_t centred, double *out);
  * reference (its icheck sums on the host); it is for callers that cannot
  * allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Limit: at most 3 x 2^19 partial sums, i.e.
- * 9 x (ceil(n / 256) + 1) on a p2d grid (n up to about 44.7M particles) and
- * 11 x (ceil(n / 512) + 1) on a p3d grid (about 73.2M); larger contexts get
- * GALHIP_ERANGE.  Every call on one GPU uses that GPU's one array: calls
+ * for large n 9 x (ceil(n / 2048) + 1) on a p2d grid (n up to about 357.9M
+ * particles) and 11 x (ceil(n / 4096) + 1) on a p3d grid (about 585.6M); larger
+ * contexts get GALHIP_ERANGE.  Every call on one GPU uses that GPU's one array: calls
  * that overlap on a GPU (other host threads, other contexts) race. */
 int galhip_integrals_noalloc(galhip_ctx *ctx, int32_t centred, double *out);
 
