@@ -30,28 +30,35 @@ namespace gh {
 
 constexpr int LG_MAXQ = 512;     // np * nm coefficients at most
 constexpr int LG_MAXW = 8;       // wavefronts per block at most
+constexpr int LG_HARM = 16;      // harmonics per wavefront at most without pitches
 constexpr int LG_SUM_BLOCK = 256;
 
 // How the coefficients are dealt out: a unit is harmonic im with len pitch
-// offsets (unit u: im = u / nch + 1, offsets (u % nch) len + 1 ..); a block
-// has one wavefront per unit of its group.
+// offsets (unit u: im = u / nch + 1, offsets (u % nch) len + 1 ..); without
+// pitches (np <= 2) a unit is len harmonics from u len + 1 on.  A block has one
+// wavefront per unit of its group.
 struct LgPlan {
     int kmax;      // largest pitch offset
-    int nch, len;  // runs per harmonic and their length
-    int units;     // nm * nch
+    int nch, len;  // runs per harmonic (of the harmonics) and their length
+    int units;
     int groups;    // gridDim.y
     int waves;     // wavefronts per block
     int nb;        // gridDim.x
 };
 
 // Runs of at most 12 offsets: 48 FP64 sums (96 VGPRs) per lane, three
-// wavefronts per SIMD.
+// wavefronts per SIMD.  Without pitches a harmonic of its own per wavefront spends
+// its time on forming z^im and, beyond eight harmonics, the tile again for every
+// group: runs of LG_HARM harmonics, each the product of the last one and z (4e6
+// particles, 512 harmonics: 27.0 ms one by one, 2.14 so; 64: 2.35 and 0.25;
+// before the wavefronts had units 11.1 and 2.08).
 static LgPlan lg_plan(long long n, int np, int nm) {
     LgPlan p;
     p.kmax = np - (np / 2 + 1);
-    p.nch = p.kmax > 12 ? (p.kmax + 11) / 12 : 1;
-    p.len = (p.kmax + p.nch - 1) / p.nch;
-    p.units = nm * p.nch;
+    const int all = p.kmax ? p.kmax : nm, most_len = p.kmax ? 12 : LG_HARM;
+    p.nch = (all + most_len - 1) / most_len;
+    p.len = (all + p.nch - 1) / p.nch;
+    p.units = p.kmax ? nm * p.nch : (nm + p.len - 1) / p.len;
     p.groups = (p.units + LG_MAXW - 1) / LG_MAXW;
     p.waves = (p.units + p.groups - 1) / p.groups;
     // twelve wavefronts per CU (three per SIMD) over 256 CUs
@@ -83,6 +90,104 @@ __device__ __forceinline__ void cpow(double zr, double zi, int e, double &pr, do
     }
 }
 
+// A particle's e^{i nsect theta} and, if PITCH, e^{i a}; false if it is not among
+// those summed (its factors are left as they were).
+template <typename R, bool PITCH>
+__device__ __forceinline__ bool lg_factors(const typename Vec4<R>::T *__restrict__ xv, int ps,
+                                           const uint8_t *__restrict__ zone, long long i, int nz,
+                                           int offanal, int nsect, double inv_lscale, double &c1,
+                                           double &s1, double &ca, double &sa) {
+    const int z = zone[i];
+    const bool inc = z >= 1 && (z <= nz || (offanal && z == nz + 1));
+    // x, y lead the particle's data
+    const typename Vec2<R>::T p = *reinterpret_cast<const typename Vec2<R>::T *>(xv + i * ps);
+    const double x = (double)p.x, y = (double)p.y;
+    const double rc = sqrt(x * x + y * y);
+    if (!(inc && rc > 0.0)) return false;
+    const double cx = x / rc, sy = y / rc;
+    c1 = cx;
+    s1 = sy;
+    for (int m = 2; m <= nsect; m++) {
+        const double t = c1 * cx - s1 * sy;
+        s1 = s1 * cx + c1 * sy;
+        c1 = t;
+    }
+    if (PITCH) sincos(0.25 * (double)nsect * log(rc * inv_lscale), &sa, &ca);
+    return true;
+}
+
+// The block's particle count, by the blocks of the first group.
+__device__ __forceinline__ void lg_count(double cnt, double *s_cnt, double *out) {
+    const int tid = threadIdx.x;
+    cnt = wave_sum_dpp(cnt);
+    if ((tid & 63) == 0) s_cnt[tid >> 6] = cnt;
+    __syncthreads();
+    if (tid == 0) {
+        double v = 0.0;
+        for (int k = 0; k < (int)blockDim.x / 64; k++) v += s_cnt[k];
+        *out = v;
+    }
+}
+
+// No pitches (np 1 or 2): a wavefront's harmonics in turn.
+template <typename R>
+__global__ __launch_bounds__(64 * LG_MAXW, 3) void lgsp_harm_kernel(
+    const typename Vec4<R>::T *__restrict__ xv, int ps, const uint8_t *__restrict__ zone,
+    long long n, int nz, int offanal, int nsect, int np, int nm, LgPlan pl,
+    double *__restrict__ part) {
+    __shared__ double2 s_z[64 * LG_MAXW];
+    __shared__ double s_cnt[LG_MAXW];
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, T = blockDim.x;
+    const int unit = blockIdx.y * pl.waves + w;
+    const bool work = unit < pl.units;         // uniform over the wavefront
+    const int im0 = work ? unit * pl.len + 1 : 1;
+    double sr[LG_HARM], si[LG_HARM], cnt = 0.0;
+#pragma unroll
+    for (int h = 0; h < LG_HARM; h++) sr[h] = si[h] = 0.0;
+    const long long stride = (long long)gridDim.x * T;
+    for (long long base = (long long)blockIdx.x * T; base < n; base += stride) {
+        const long long i = base + tid;
+        double c1 = 0.0, s1 = 0.0, ca, sa;
+        if (i < n && lg_factors<R, false>(xv, ps, zone, i, nz, offanal, nsect, 1.0, c1, s1, ca, sa))
+            cnt += 1.0;
+        __syncthreads();   // the last tile has been read
+        s_z[tid] = make_double2(c1, s1);
+        __syncthreads();
+        if (work)
+            for (int e = lane; e < T; e += 64) {
+                const double2 z = s_z[e];
+                double zr, zi;
+                cpow(z.x, z.y, im0, zr, zi);
+#pragma unroll
+                for (int h = 0; h < LG_HARM; h++) {
+                    if (h >= pl.len) break;    // uniform
+                    sr[h] += zr;
+                    si[h] += zi;
+                    const double t = fma(zr, z.x, -(zi * z.y));
+                    zi = fma(zi, z.x, zr * z.y);
+                    zr = t;
+                }
+            }
+    }
+    const size_t nb = gridDim.x, b = blockIdx.x;
+    const int nq = np * nm;
+#pragma unroll
+    for (int h = 0; h < LG_HARM; h++) {
+        if (!work || h >= pl.len || im0 + h > nm) break;
+        const double vr = wave_sum_dpp(sr[h]), vi = wave_sum_dpp(si[h]);
+        if (lane) continue;
+        // the last pitch index; the first of two holds none
+        const int q = (np - 1) * nm + im0 + h - 1;
+        part[(size_t)q * nb + b] = vr;
+        part[(size_t)(nq + q) * nb + b] = vi;
+        if (np == 2) {
+            part[(size_t)(q - nm) * nb + b] = 0.0;
+            part[(size_t)(nq + q - nm) * nb + b] = 0.0;
+        }
+    }
+    if (blockIdx.y == 0) lg_count(cnt, s_cnt, part + 2 * (size_t)nq * nb + b);
+}
+
 // part[q][block]: q = [cos parts][sin parts][count].  KC: pitch offsets of
 // a run at most.
 template <typename R, int KC>
@@ -106,27 +211,8 @@ __global__ __launch_bounds__(64 * LG_MAXW, 3) void lgsp_part_kernel(
     for (long long base = (long long)blockIdx.x * T; base < n; base += stride) {
         const long long i = base + tid;
         double c1 = 0.0, s1 = 0.0, ca = 1.0, sa = 0.0;
-        if (i < n) {
-            const int z = zone[i];
-            const bool inc = z >= 1 && (z <= nz || (offanal && z == nz + 1));
-            // x, y lead the particle's data
-            const typename Vec2<R>::T p =
-                *reinterpret_cast<const typename Vec2<R>::T *>(xv + i * ps);
-            const double x = (double)p.x, y = (double)p.y;
-            const double rc = sqrt(x * x + y * y);
-            if (inc && rc > 0.0) {
-                const double cx = x / rc, sy = y / rc;
-                c1 = cx;
-                s1 = sy;
-                for (int m = 2; m <= nsect; m++) {
-                    const double t = c1 * cx - s1 * sy;
-                    s1 = s1 * cx + c1 * sy;
-                    c1 = t;
-                }
-                sincos(0.25 * (double)nsect * log(rc * inv_lscale), &sa, &ca);
-                cnt += 1.0;
-            }
-        }
+        if (i < n && lg_factors<R, true>(xv, ps, zone, i, nz, offanal, nsect, inv_lscale, c1, s1, ca, sa))
+            cnt += 1.0;
         __syncthreads();   // the last tile has been read
         s_z[tid] = make_double2(c1, s1);
         s_w[tid] = make_double2(ca, sa);
@@ -181,16 +267,7 @@ __global__ __launch_bounds__(64 * LG_MAXW, 3) void lgsp_part_kernel(
             }
         }
     }
-    if (blockIdx.y == 0) {
-        cnt = wave_sum_dpp(cnt);
-        if (lane == 0) s_cnt[w] = cnt;
-        __syncthreads();
-        if (tid == 0) {
-            double v = 0.0;
-            for (int k = 0; k < T / 64; k++) v += s_cnt[k];
-            part[2 * (size_t)nq * nb + b] = v;
-        }
-    }
+    if (blockIdx.y == 0) lg_count(cnt, s_cnt, part + 2 * (size_t)nq * nb + b);
 }
 
 // Fixed-order sum of row[0 .. nb) over the block.
@@ -233,7 +310,11 @@ hipError_t launch_lgspia(const void *xv, int ps, const uint8_t *zone, long long 
                          double *out, hipStream_t s) {
     if (np * nm > LG_MAXQ) return hipErrorInvalidValue;
     const LgPlan pl = lg_plan(n, np, nm);
-    if (pl.len <= 4)
+    if (pl.kmax == 0)
+        hipLaunchKernelGGL(lgsp_harm_kernel<R>, dim3(pl.nb, pl.groups), dim3(64 * pl.waves), 0, s,
+                           (const typename Vec4<R>::T *)xv, ps, zone, n, nz, offanal, nsect, np, nm,
+                           pl, part);
+    else if (pl.len <= 4)
         launch_lgsp_part<R, 4>(xv, ps, zone, n, nz, offanal, nsect, np, nm, lscale, pl, part, s);
     else if (pl.len <= 8)
         launch_lgsp_part<R, 8>(xv, ps, zone, n, nz, offanal, nsect, np, nm, lscale, pl, part, s);
