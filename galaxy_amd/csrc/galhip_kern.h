@@ -560,6 +560,14 @@ inline IntSplit int_split(long long n, int block) {
     return s;
 }
 
+// Harmonics per pass of the analyses that take several rings or planes at once:
+// as few passes as nine allow (registers), then the least of 3, 5, 7 and 9 that
+// takes them, since a pass forms its sums whether they are wanted or not.
+inline int harm_per_pass(int nharm) {
+    const int passes = (nharm + 8) / 9, need = passes > 0 ? (nharm + passes - 1) / passes : 0;
+    return need <= 3 ? 3 : need <= 5 ? 5 : need <= 7 ? 7 : 9;
+}
+
 // Unloads gather their particles from UNLOAD_GATHER particles on (see
 // deinterleave_kernel).
 constexpr long long UNLOAD_GATHER = 50000;

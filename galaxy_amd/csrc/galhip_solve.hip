@@ -405,14 +405,13 @@ __global__ void combine_ranges_kernel(const int *jrad, const int *krad, int rstr
 // harmonics: analysis 46.7 -> 15.7 us (four rings a wavefront 19.8, one 16.0),
 // synthesis 40.9 -> 15.6 (two rings a block 17.0, eight 20.0).
 constexpr int ROWS_BLOCK = 256;
-constexpr int ROWS_HARM = 9;     // harmonics per pass of the analysis
 template <typename R> constexpr int ana_rows() { return sizeof(R) == 4 ? 2 : 1; }
 constexpr int SYN_ROWS = 4;
 
-// grid (rings / (4 wavefronts x ana_rows), nmem)
-template <typename R>
+// grid (rings / (4 wavefronts x ana_rows), nmem); HB: harmonics per pass
+template <typename R, int HB>
 __global__ __launch_bounds__(ROWS_BLOCK) void analyse_rows_kernel(AnaArgs<R> a) {
-    constexpr int RW = ana_rows<R>(), HB = ROWS_HARM;
+    constexpr int RW = ana_rows<R>();
     typedef typename Vec2<R>::T R2;
     extern __shared__ unsigned char rows_lds[];
     R2 *tws = (R2 *)rows_lds;                 // [na]
@@ -606,9 +605,12 @@ __global__ __launch_bounds__(ROWS_BLOCK) void synth_rows_kernel(SynArgs<R> a) {
 // The rows kernels' time hardly depends on the number of rings until they fill
 // the chip; a block per ring costs the same for every 512 rings.  The lines lie
 // where the two were equal (rings x members):
-//   analysis  1200 at 256 spokes x 9 harmonics (10.7 us against 9.6 at 1536),
-//             1900 at 512 x 9, 3200 at 512 x 17 (14 discs of 256 rings 31.6 and
-//             28.3), 4400 at 1024 x 17: the passes over a ring grow with both;
+//   analysis  by spokes (128, 256, 512, 1024) and the harmonics that its passes
+//             form: 3: 900 1050 1400 2600; 9: 1200 1500 1800 3000; 18: 1900 1950
+//             3200 4400; 27: 2400 2700 4400 5300; 36: 3100 3200 5700 5500 (FP64
+//             up to a third lower).  With the wanted harmonics in the place of
+//             those formed the line was too low below nine and beyond: 10 discs
+//             of 100 x 512, 3 harmonics, 17.8 us a solve by rings, 23.0 by rows;
 //   synthesis after a contraction 1000 to 1450 (1536 rings of 256 spokes 10.1
 //             and 7.9 us, 1024 8.0 and 7.5, 512 4.6 and 7.1).
 // The synthesis with its own contraction keeps its blocks, of 256 threads
@@ -616,17 +618,29 @@ __global__ __launch_bounds__(ROWS_BLOCK) void synth_rows_kernel(SynArgs<R> a) {
 // keep others off the CU: 64 discs of 128 x 256 99 -> 52 us, FP64 195 -> 80;
 // 768 rings of 512 21.2 and 23.7, FP64 37.9 and 31.3.
 template <typename R> static bool ana_by_rows(const AnaArgs<R> &a) {
-    return 10LL * a.nr * a.nmem >= 5000 + 3LL * a.na * a.ng;
+    const long long h = harm_per_pass(a.ng), formed = (a.ng + h - 1) / h * h;
+    return 100LL * a.nr * a.nmem >= 60000 + 120LL * a.na + formed * (5000 + 13LL * a.na);
 }
 constexpr int SYN_ROWS_MIN = 1400;
+
+template <typename R, int HB>
+static void launch_analyse_rows(const AnaArgs<R> &a, hipStream_t s) {
+    const unsigned per = ROWS_BLOCK / 64 * ana_rows<R>();
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(analyse_rows_kernel<R, HB>),
+                       dim3((a.nr + per - 1) / per, a.nmem), dim3(ROWS_BLOCK),
+                       2 * a.na * sizeof(R), s, a);
+}
 
 template <typename R>
 hipError_t launch_analyse(const AnaArgs<R> &a, hipStream_t s) {
     if (a.na > MAX_NA) return hipErrorInvalidValue;
     if (ana_by_rows(a)) {
-        const unsigned per = ROWS_BLOCK / 64 * ana_rows<R>();
-        hipLaunchKernelGGL(analyse_rows_kernel<R>, dim3((a.nr + per - 1) / per, a.nmem),
-                           dim3(ROWS_BLOCK), 2 * a.na * sizeof(R), s, a);
+        switch (harm_per_pass(a.ng)) {
+        case 3: launch_analyse_rows<R, 3>(a, s); break;
+        case 5: launch_analyse_rows<R, 5>(a, s); break;
+        case 7: launch_analyse_rows<R, 7>(a, s); break;
+        default: launch_analyse_rows<R, 9>(a, s);
+        }
         return hipGetLastError();
     }
     hipLaunchKernelGGL(analyse_kernel<R>, dim3(a.nr, ANA_SPLIT, a.nmem), dim3(SOLVE_BLOCK), 0,
