@@ -56,7 +56,7 @@ template <typename R> struct P3SolveArgs {
     const int *lg, *slot_m, *slot_p, *slot_of;
     typename Vec4<R>::T *fld;
     double q, pmass;
-    int nr, na, ngz, ng, mmax, nm, nz, mzone, lpot, jzone, kzone, explicit_zones, ntypes;
+    int nr, na, ngz, ng, mmax, nm, nharm, nz, mzone, lpot, jzone, kzone, explicit_zones, ntypes;
 };
 
 template <typename R> struct P3PermArgs {

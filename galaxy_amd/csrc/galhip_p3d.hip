@@ -991,7 +991,6 @@ __global__ __launch_bounds__(P3_PBLOCK) void p3_deinterleave_kernel(
 template <typename R> struct P3Solve {
     static constexpr int planes = sizeof(R) == 4 ? 2 : 1;
     static constexpr int splanes = sizeof(R) == 4 ? 4 : 2;
-    static constexpr int harm = 9;
 };
 
 // combined, scaled mass of a cell (zoncmb + scaled)
@@ -1005,11 +1004,11 @@ __device__ __forceinline__ R p3_cell_mass(const P3SolveArgs<R> &a, size_t idx) {
     return (R)(acc * a.pmass);
 }
 
-// grid (planes / (4 wavefronts x P3Solve::planes), nr): a wavefront takes some
-// planes of a ring
-template <typename R>
+// grid (planes / (4 wavefronts x PL), nr, 1): a wavefront takes PL planes of a
+// ring and, HB at a time, all harmonics; with gridDim.z passes of HB harmonics
+// each takes one of them
+template <typename R, int PL, int HB>
 __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) {
-    constexpr int PL = P3Solve<R>::planes, HB = P3Solve<R>::harm;
     typedef typename Vec2<R>::T R2;
     extern __shared__ unsigned char p3_lds[];
     R2 *tws = (R2 *)p3_lds;                   // [na]
@@ -1024,7 +1023,7 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
                                      a.explicit_zones, a.jzone, a.kzone, kr, rg);
         s_ok = ok;
         for (int q = 0; q < 4; q++) s_rng[q] = rg[q];
-        if (blockIdx.x == 0 && ir == 1) {
+        if (blockIdx.x == 0 && ir == 1 && blockIdx.z == 0) {
             for (int q = 0; q < 4; q++) a.ranges[q] = ok ? rg[q] : -1;
             if (ok)
                 for (int z = 1; z < a.nz; z++) a.krad[z] = kr[z];
@@ -1038,20 +1037,22 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
 #pragma unroll
     for (int p = 0; p < PL; p++)
         row[p] = ((size_t)(ir - 1) * a.ngz + min(plane0 + p, a.ngz - 1)) * na;
-    int s = 0;
+    // the slot of the i-th harmonic: two slots each, one for m = 0 (and the last
+    // one for m = na / 2)
+    const int zero = nm > 0 && a.slot_m[0] == 0;
+    auto slot = [&](int i) { return zero && i ? 2 * i - 1 : 2 * i; };
+    int i0 = (int)blockIdx.z * HB;
     bool first = true;
     do {
-        // the next HB harmonics of the slot list
-        int k[HB], step[HB], sn = s;
+        // the harmonics i0 .. i0 + HB - 1
+        int k[HB], step[HB];
 #pragma unroll
         for (int h = 0; h < HB; h++) {
-            int m = 0;
-            if (sn < nm) {
-                m = a.slot_m[sn];
-                sn += sn + 1 < nm && a.slot_p[sn + 1] ? 2 : 1;
-            }
-            k[h] = (int)(((long long)m * lane) % na);
-            step[h] = (int)(((long long)m * 64) % na);
+            const int s = slot(i0 + h), m = s < nm ? a.slot_m[s] : 0;
+            // (m < P3_MAX_NA: 32 bits hold the products, and their remainders are
+            // a third of a small grid's time with 64)
+            k[h] = (m * lane) % na;
+            step[h] = (m * 64) % na;
         }
         R sa[HB][PL], sb[HB][PL];
 #pragma unroll
@@ -1062,7 +1063,7 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
             R rv[PL];
 #pragma unroll
             for (int p = 0; p < PL; p++) rv[p] = first ? p3_cell_mass(a, row[p] + j) : a.rho[row[p] + j];
-            if (first)
+            if (first && blockIdx.z == 0)
 #pragma unroll
                 for (int p = 0; p < PL; p++)
                     if (plane0 + p < a.ngz) a.rho[row[p] + j] = rv[p];
@@ -1082,6 +1083,7 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
         if (!active) return;
 #pragma unroll
         for (int h = 0; h < HB; h++) {
+            const int s = slot(i0 + h);
             const bool pair = s + 1 < nm && a.slot_p[s + 1];
             R va = 0, vb = 0;
 #pragma unroll
@@ -1097,10 +1099,10 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
                 out[0] = va;
                 if (pair) out[a.ngz] = vb;
             }
-            s += pair ? 2 : 1;
         }
         first = false;
-    } while (s < nm);
+        i0 += HB;
+    } while (gridDim.z == 1 && slot(i0) < nm);
 }
 
 // The vertical twiddles (cos, sin of 2 pi k / P) in LDS with one pad entry
@@ -1294,11 +1296,11 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_zinv_kernel(P3SolveArgs<R> a) {
 // grid (planes / P3Solve::planes, nr): inverse azimuthal transform of the
 // active components of some planes of a ring, scale, polcat; interleaved
 // field store
-template <typename R, bool LPOT>
+template <typename R, bool LPOT, int PL>
 __global__ __launch_bounds__(P3_BLOCK) void p3_synth_kernel(P3SolveArgs<R> a) {
     typedef typename Vec4<R>::T R4;
     typedef typename Vec2<R>::T R2;
-    constexpr int PL = P3Solve<R>::splanes, NT = LPOT ? 4 : 3;
+    constexpr int NT = LPOT ? 4 : 3;
     extern __shared__ unsigned char p3_lds[];
     R4 *zc = (R4 *)p3_lds;                    // [nm][PL]
     R2 *tws = (R2 *)(zc + a.nm * PL);         // [na]
@@ -1623,7 +1625,10 @@ template <typename R> bool p3_solve_fits(const P3SolveArgs<R> &a) {
 static dim3 p3_lanes(int n) { return dim3(std::min(P3_BLOCK, (n + 63) / 64 * 64)); }
 
 // The vertical transforms by CB columns a block.  The forward transform takes
-// three.  The inverse reads a column twice as often as it multiplies it, from
+// three, the inverse nine or three.  Below 1500 columns of all rings (2000, of all
+// types, in the inverse) one: more blocks for a chip that is not full (61 rings, 45 planes, 5
+// columns: forward 6.5 us by threes, 4.6 by one, inverse 7.7 and 6.6; 140 rings, 17
+// columns: forward 10.0 and 11.8).  The inverse reads a column twice as often as it multiplies it, from
 // LDS: nine columns share a twiddle (three types of 200 rings, 17 columns:
 // 46 us, three at a time 60) if that leaves four blocks a CU, else three, for
 // more blocks (three types of 61 rings, 9 columns, FP64: 22 us and 9.8 us).
@@ -1643,16 +1648,54 @@ static hipError_t p3_vertical(const P3SolveArgs<R> &a, bool inverse, hipStream_t
 template <typename R>
 static hipError_t p3_vertical(const P3SolveArgs<R> &a, bool inverse, hipStream_t s) {
     if (a.nm == 0) return hipSuccess;
+    if (a.nm < 3 || a.nr * a.nm * (inverse ? a.ntypes : 1) < (inverse ? 2000 : 1500))
+        return p3_vertical<R, 1>(a, inverse, s);
     if (inverse && a.nm >= 9 && (long long)a.nr * a.ntypes * ((a.nm + 8) / 9) >= 1024)
         return p3_vertical<R, 9>(a, inverse, s);
-    return a.nm >= 3 ? p3_vertical<R, 3>(a, inverse, s) : p3_vertical<R, 1>(a, inverse, s);
+    return p3_vertical<R, 3>(a, inverse, s);
 }
+
+template <typename R, int PL, int HB>
+static void p3_analysis(const P3SolveArgs<R> &a, hipStream_t s, int passes = 1) {
+    constexpr unsigned per = P3_BLOCK / 64 * PL;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_analyse_kernel<R, PL, HB>),
+                       dim3((a.ngz + per - 1) / per, a.nr, passes), dim3(P3_BLOCK), 2 * a.na * sizeof(R),
+                       s, a);
+}
+template <typename R, int PL> static void p3_analysis(const P3SolveArgs<R> &a, hipStream_t s) {
+    switch (harm_per_pass(a.nharm)) {
+    case 3: return p3_analysis<R, PL, 3>(a, s);
+    case 5: return p3_analysis<R, PL, 5>(a, s);
+    case 7: return p3_analysis<R, PL, 7>(a, s);
+    default: return p3_analysis<R, PL, 9>(a, s);
+    }
+}
+
+template <typename R, bool LPOT, int PL>
+static void p3_synthesis(const P3SolveArgs<R> &a, hipStream_t s) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_synth_kernel<R, LPOT, PL>),
+                       dim3((a.ngz + PL - 1) / PL, a.nr), p3_lanes(a.na),
+                       (4 * (size_t)a.nm * PL + 2 * a.na) * sizeof(R), s, a);
+}
+template <typename R, int PL> static void p3_synthesis(const P3SolveArgs<R> &a, hipStream_t s) {
+    if (a.lpot) p3_synthesis<R, true, PL>(a, s);
+    else p3_synthesis<R, false, PL>(a, s);
+}
+
+// A wavefront per plane of a ring leaves a small grid's chip idle and takes its
+// harmonics one pass after the other: below P3_SPLIT planes of all rings each pass
+// of three harmonics gets wavefronts of its own, and the synthesis one plane a
+// block (24 rings x 16 planes, 9 harmonics: analysis 10.0 -> 4.9 us, synthesis 7.6
+// -> 5.6; 61 x 45: 9.8 and 10.1, 8.2 and 9.0); below P3_PAIR a wavefront takes one
+// plane (61 x 45 10.5 -> 9.8; 100 x 61 12.5 and 15.0).
+constexpr int P3_SPLIT = 2000, P3_PAIR = 3000;
 
 template <typename R> hipError_t launch_p3_solve(const P3SolveArgs<R> &a, hipStream_t s) {
     if (!p3_solve_fits(a)) return hipErrorInvalidValue;
-    constexpr unsigned PL = P3Solve<R>::planes, per = P3_BLOCK / 64 * PL;
-    hipLaunchKernelGGL(p3_analyse_kernel<R>, dim3((a.ngz + per - 1) / per, a.nr), dim3(P3_BLOCK),
-                       2 * a.na * sizeof(R), s, a);
+    const int cells = a.nr * a.ngz;   // rings of all planes
+    if (cells < P3_SPLIT) p3_analysis<R, 1, 3>(a, s, std::max(1, (a.nharm + 2) / 3));
+    else if (cells < P3_PAIR) p3_analysis<R, 1>(a, s);
+    else p3_analysis<R, P3Solve<R>::planes>(a, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if ((e = p3_vertical(a, false, s)) != hipSuccess) return e;
@@ -1660,13 +1703,8 @@ template <typename R> hipError_t launch_p3_solve(const P3SolveArgs<R> &a, hipStr
                        0, s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = p3_vertical(a, true, s)) != hipSuccess) return e;
-    constexpr int SL = P3Solve<R>::splanes;
-    const dim3 grid((a.ngz + SL - 1) / SL, a.nr);
-    const size_t lds = (4 * (size_t)a.nm * SL + 2 * a.na) * sizeof(R);
-    if (a.lpot)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_synth_kernel<R, true>), grid, p3_lanes(a.na), lds, s, a);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_synth_kernel<R, false>), grid, p3_lanes(a.na), lds, s, a);
+    if (cells < P3_SPLIT) p3_synthesis<R, 1>(a, s);
+    else p3_synthesis<R, P3Solve<R>::splanes>(a, s);
     return hipGetLastError();
 }
 

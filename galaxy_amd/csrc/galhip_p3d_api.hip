@@ -9,6 +9,7 @@
 
 #include <rocprim/device/device_radix_sort.hpp>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -441,6 +442,7 @@ static P3SolveArgs<R> p3_solve_args(galhip_ctx *c, int lpot, int explicit_zones,
     a.q = ldexp(1.0, -c->qbits);
     a.pmass = c->pmass;
     a.nr = c->nr; a.na = c->na; a.ngz = c->ngz; a.ng = c->ng; a.mmax = c->mmax; a.nm = c->nm3;
+    a.nharm = (int)std::count(c->lg.begin(), c->lg.begin() + c->ng, 0);
     a.nz = c->nz; a.mzone = c->mzone; a.lpot = lpot; a.jzone = jzone; a.kzone = kzone;
     a.explicit_zones = explicit_zones;
     a.ntypes = lpot ? 4 : 3;
