@@ -37,7 +37,7 @@
 namespace gh {
 
 constexpr int P3_BLOCK = 256;    // solve kernels
-constexpr int P3_PBLOCK = 512;   // particle kernels: a larger block shares one deposit window
+constexpr int P3_PBLOCK = 512;   // particle kernels without a deposit (those: P3Shape)
 
 // (u, t) of particle i: the second half of its record's second R4
 template <typename R>
@@ -288,21 +288,30 @@ __device__ __forceinline__ void getacc3(const P3Args<R> &a, R ox, R oy, R oz, R 
     }
 }
 
-// Launch shape of the push and the mass assignment.  Linear FP32: two
-// particles per thread share the window's reductions, clearing and flush, and
-// 20 KB of LDS leave seven wavefronts per SIMD (2e7 particles on 200 x 256 x
-// 125, push averaged over an eight-step sort cycle, us: one particle per
-// thread in blocks of 512 with 4096 cells 686; two in blocks of 256 with 4096,
-// 3072, 2560, 2048 cells 708, 640, 633, 736; four 697; two in blocks of 512
-// 689-706; 749 before, at one per thread).  The 27 weights of the quadratic
-// scheme and FP64 keep one.
-template <typename R, int J> struct P3Shape {
-    static constexpr bool two = J == 2 && sizeof(R) == 4;
-    static constexpr int ppt = two ? 2 : 1;
-    static constexpr int block = two ? 256 : 512;
-    static constexpr int tile = two ? 2560 : 4096;
-    static constexpr int waves = two ? 7 : 4;
+// Launch shapes of the push and the mass assignment by particles per thread;
+// push averaged over an eight-step sort cycle, us.
+// Linear FP32, two particles per thread: they share the window's reductions,
+// clearing and flush, and 20 KB of LDS leave seven wavefronts per SIMD (2e7
+// particles on 200 x 256 x 125: one particle per thread in blocks of 512 with 4096
+// cells 681; two in blocks of 256 with 4096, 3072, 2560, 2048 cells 708, 640, 623,
+// 736; four 697; two in blocks of 512 689-706).  Fewer particles wait for a
+// block's own latency, which grows with the particles per thread, and a sparse
+// grid's blocks for the passes that a smaller window takes: two and one per thread
+//   n                1e5        1e6        3e6        8e6
+//   61 x  90 x  45   38   26    49   40    77   79    159  184
+//  140 x 200 x  81   49   40    73   68   125  121    238  256
+//  200 x 256 x 125   53   45   129  116   212  197    344  351
+// Quadratic: 256 threads with 4096 cells (140 x 200 x 81, 2e6, FP64: 512 threads
+// 306, 256 with 2560, 3328 cells 293, 287, with 4096 275; FP32 224 and 194).  Its
+// FP64 push spills 14 registers (36 bytes) in the gather of the 27 corners at four
+// wavefronts per SIMD; three without spills are slower (512 threads, same case:
+// 408 us against 318).
+template <typename R, int J, int PPT> struct P3Shape {
+    static constexpr int block = PPT == 2 || J == 3 ? 256 : 512;
+    static constexpr int tile = PPT == 2 ? 2560 : 4096;
+    static constexpr int waves = PPT == 2 ? 7 : 4;
 };
+constexpr long long P3_TWO = 5000000;   // linear FP32: two per thread above
 constexpr int P3_PASSES = 8;   // window passes before the direct fallback
 
 // LDS of a block's deposit.
@@ -372,12 +381,25 @@ __device__ __forceinline__ void deposit3_block(const P3Args<R> &a, Deposit3Lds<T
     auto in_zone = [&](int k, int z) {
         return (pend >> k & 1u) && (int)(dzone >> (4 * k) & 15u) == z;
     };
+    // the quadratic scheme's 27 fixed-point weights are formed once: again in
+    // every pass, as the linear one's eight, they cost 3 to 9 % (140 x 200 x 81, 3e5,
+    // FP64: 104 us, so 96)
+    constexpr bool KEEP = J == 3 && PPT == 1;
+    long long v0[NW];
+    if constexpr (KEEP) {
+        int ring, plane, spoke;
+        loc3<R, J>(pos[0], a, ring, plane, spoke);
+        R w[NW];
+        weights3(pos[0], ring, plane, w);
+        quant_n<R, NW>(w, a.qbits, dzone != 0, v0);
+    }
 #pragma unroll 1
     for (int pass = 0;; pass++) {
         int *const sb = s.box + 6 * (pass & 1);
         // cells and weights are formed again from the grid coordinates
+        if (!KEEP)
 #pragma unroll
-        for (int k = 0; k < PPT; k++) opaque3(pos[k]);
+            for (int k = 0; k < PPT; k++) opaque3(pos[k]);
         {
             int r0 = INT_MAX, r1 = -1, p0 = INT_MAX, p1 = -1, q0 = INT_MAX, q1 = -1;
 #pragma unroll
@@ -449,10 +471,15 @@ __device__ __forceinline__ void deposit3_block(const P3Args<R> &a, Deposit3Lds<T
                                 plane - LO >= p0 && plane - p0 + 1 < NP && spoke - LO >= q0 &&
                                 spoke - q0 + 1 < NQ;
             if (inside) {
-                R w[NW];
-                weights3(pos[k], ring, plane, w);
                 long long v[NW];
-                quant_n<R, NW>(w, a.qbits, true, v);
+                if constexpr (KEEP) {
+#pragma unroll
+                    for (int q = 0; q < NW; q++) v[q] = v0[q];
+                } else {
+                    R w[NW];
+                    weights3(pos[k], ring, plane, w);
+                    quant_n<R, NW>(w, a.qbits, true, v);
+                }
                 const int b = ((ring - r0) * NP + (plane - p0)) * NQ + (spoke - q0);
 #pragma unroll
                 for (int q = 0; q < NW; q++) {
@@ -560,9 +587,9 @@ __device__ __forceinline__ void deposit3_ranges(const Deposit3Lds<TILE> &s, int 
     }
 }
 
-template <typename R, int J>
-__global__ __launch_bounds__((P3Shape<R, J>::block), (P3Shape<R, J>::waves)) void p3_massgn_kernel(P3Args<R> a) {
-    constexpr int TB = P3Shape<R, J>::block, PPT = P3Shape<R, J>::ppt, TILE = P3Shape<R, J>::tile;
+template <typename R, int J, int PPT>
+__global__ __launch_bounds__((P3Shape<R, J, PPT>::block), (P3Shape<R, J, PPT>::waves)) void p3_massgn_kernel(P3Args<R> a) {
+    constexpr int TB = P3Shape<R, J, PPT>::block, TILE = P3Shape<R, J, PPT>::tile;
     __shared__ Deposit3Lds<TILE> s_dep;
     __shared__ P3Ref s_ref0;
     const int tid = threadIdx.x;
@@ -598,10 +625,10 @@ __global__ __launch_bounds__((P3Shape<R, J>::block), (P3Shape<R, J>::waves)) voi
     deposit3_ranges(s_dep, a.nz, a.nr, J == 3 ? 1 : 0, a.jrad, a.krad, a.rstride);
 }
 
-template <typename R, int J>
-__global__ __launch_bounds__((P3Shape<R, J>::block), (P3Shape<R, J>::waves)) void p3_push_kernel(P3Args<R> a) {
+template <typename R, int J, int PPT>
+__global__ __launch_bounds__((P3Shape<R, J, PPT>::block), (P3Shape<R, J, PPT>::waves)) void p3_push_kernel(P3Args<R> a) {
     typedef typename Vec4<R>::T R4;
-    constexpr int TB = P3Shape<R, J>::block, PPT = P3Shape<R, J>::ppt, TILE = P3Shape<R, J>::tile;
+    constexpr int TB = P3Shape<R, J, PPT>::block, TILE = P3Shape<R, J, PPT>::tile;
     __shared__ Deposit3Lds<TILE> s_dep;
     __shared__ int s_dn, s_np;
     __shared__ double s_tab[UtTab<R>::n];
@@ -1343,7 +1370,7 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_synth_kernel(P3SolveArgs<R> a) {
                 F[p][0] += z.x * b;
                 F[p][1] += z.y * b;
                 F[p][2] += z.z * b;
-                if (LPOT) F[p][3] += z.w * b;
+                if (LPOT) F[p][NT - 1] += z.w * b;
             }
         }
         const R cp = tws[j].x, sn = tws[j].y;
@@ -1496,30 +1523,30 @@ __global__ __launch_bounds__(GREEN3_BLOCK) void p3_green_kernel(
 // ---- launchers ------------------------------------------------------------------------
 
 static unsigned p3_blocks(long long n) { return (unsigned)((n + P3_PBLOCK - 1) / P3_PBLOCK); }
-template <typename R, int J> static dim3 p3_grid(long long n) {
-    const int per = P3Shape<R, J>::block * P3Shape<R, J>::ppt;
-    return dim3((unsigned)((n + per - 1) / per));
+template <typename R, int J, int PPT> static void p3_massgn(const P3Args<R> &a, hipStream_t s) {
+    constexpr int TB = P3Shape<R, J, PPT>::block, per = TB * PPT;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, J, PPT>),
+                       dim3((unsigned)((a.n + per - 1) / per)), dim3(TB), 0, s, a);
+}
+template <typename R, int J, int PPT> static void p3_push(const P3Args<R> &a, hipStream_t s) {
+    constexpr int TB = P3Shape<R, J, PPT>::block, per = TB * PPT;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, J, PPT>),
+                       dim3((unsigned)((a.n + per - 1) / per)), dim3(TB), 0, s, a);
 }
 
 template <typename R> hipError_t launch_p3_massgn(const P3Args<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
-    if (a.jmass == 3)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, 3>), (p3_grid<R, 3>(a.n)),
-                           dim3(P3Shape<R, 3>::block), 0, s, a);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_massgn_kernel<R, 2>), (p3_grid<R, 2>(a.n)),
-                           dim3(P3Shape<R, 2>::block), 0, s, a);
+    if (a.jmass == 3) p3_massgn<R, 3, 1>(a, s);
+    else if (sizeof(R) == 8 || a.n <= P3_TWO) p3_massgn<R, 2, 1>(a, s);
+    else if constexpr (sizeof(R) == 4) p3_massgn<R, 2, 2>(a, s);
     return hipGetLastError();
 }
 
 template <typename R> hipError_t launch_p3_push(const P3Args<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
-    if (a.jmass == 3)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, 3>), (p3_grid<R, 3>(a.n)),
-                           dim3(P3Shape<R, 3>::block), 0, s, a);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(p3_push_kernel<R, 2>), (p3_grid<R, 2>(a.n)),
-                           dim3(P3Shape<R, 2>::block), 0, s, a);
+    if (a.jmass == 3) p3_push<R, 3, 1>(a, s);
+    else if (sizeof(R) == 8 || a.n <= P3_TWO) p3_push<R, 2, 1>(a, s);
+    else if constexpr (sizeof(R) == 4) p3_push<R, 2, 2>(a, s);
     return hipGetLastError();
 }
 
