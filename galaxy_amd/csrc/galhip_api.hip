@@ -711,9 +711,12 @@ static UtConst ut_const(const galhip_ctx *c) {
 }
 
 // Particles per thread of the push and the mass assignment (the table at
-// PushShape): FP64 one; FP32 one up to 1.5e6 particles, four above.
-static int push_ppt(int prec, long long n) {
-    return prec == GALHIP_FP64 || n <= 1500000 ? 1 : 4;
+// PushShape): one up to 1.5e6 particles, four above in FP32; in FP64 one, but two
+// above on a grid whose particles are never sorted again (an ensemble's blocks are
+// laid out before its sort interval is known).
+static int push_ppt(int prec, long long n, bool unsorted = false) {
+    if (n <= 1500000) return 1;
+    return prec == GALHIP_FP32 ? 4 : unsorted ? 2 : 1;
 }
 
 template <typename R> static PushArgs<R> push_args(galhip_ctx *c) {
@@ -747,7 +750,7 @@ template <typename R> static PushArgs<R> push_args(galhip_ctx *c) {
         a.qbits_m = c->m_qbits_d;
         a.nblocks = c->nblk;
     }
-    a.ppt = push_ppt(c->prec, c->n);
+    a.ppt = push_ppt(c->prec, c->n, !c->ens && c->sort_interval == 0);
     a.xlo = (typename Vec2<R>::T *)c->xlo;
     return a;
 }

@@ -40,7 +40,9 @@ constexpr int PB = GH_PUSH_BLOCK;      // threads per block
 //   8e5             24.3 | 27.9      24.3 | 31.9  26.3 | 42.7
 //   2e6             45.6 | 47.9      43.7 | 44.7  44.3 | 45.7
 //   1e7, 3 zones    124              104          102
-// FP64, 3e6 in 3 zones: 55.8, 56.2, 60.6; 1e7: 169, -, 170.  A block's own latency is what a
+// FP64, 3e6 in 3 zones: 55.8, 56.2, 60.6; 1e7: 169, -, 170; never sorted again, a
+// block's particles lie all over the disc, and more of them share the flush of a
+// window (93 x 128, step us): 3e6 91.7, 81.0, 79.1; 1e7 281, 248, 241.  A block's own latency is what a
 // small count waits for, and it grows with the particles per thread; a large
 // one pays for the window work of every block.  The tile: 3072 cells in one
 // copy against 1024 in two copies (lanes of one cell spread over them) takes
@@ -49,9 +51,7 @@ constexpr int PB = GH_PUSH_BLOCK;      // threads per block
 // many as the registers allow without spills.
 template <typename R, bool COMP, int PPT> struct PushShape {
     static constexpr int tile = PPT == 1 ? 2048 : 3072;
-    static constexpr int waves = sizeof(R) == 8 ? 8
-                                 : PPT == 1     ? 8
-                                                : (COMP ? 5 : 6);
+    static constexpr int waves = PPT == 1 ? 8 : (COMP ? 5 : 6);
 };
 constexpr int PUSH_PASSES = 8;         // deposit window passes before global atomics
 constexpr int CLIP_RINGS = 16;          // rings of a window that had to be clipped
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(PB, (PushShape<R, COMP, PPT>::waves)) void push_ker
 
 // masset / massgn for every on-grid particle without a push: also fills the
 // particles' (u, t) so the next push finds them.  ENS: the members' blocks
-// of a.blk.  The push's deposit, one particle per thread (with a reduction
+// of a.blk.  The push's deposit and its particles per thread (with a reduction
 // over the wavefront per cell and global atomics it took 530 us for 1e7
 // particles, 108 us now).
 template <typename R, bool ENS, int PPT>
@@ -1056,8 +1056,11 @@ hipError_t launch_push(const PushArgs<R> &a, hipStream_t s) {
         }
     } else {
         if (a.xlo) return hipErrorInvalidValue;   // compensated positions are FP32 only
-        if (a.ppt != 1) return hipErrorInvalidValue;
-        launch_push_c<R, false, 1>(a, s);
+        if (a.ppt == 1) launch_push_c<R, false, 1>(a, s);
+        else if (a.ppt == 2 && !a.blk)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(push_kernel<R, false, false, 2>),
+                               dim3(nblocks(a.n, PB * 2)), dim3(PB), 0, s, a);
+        else return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
@@ -1077,6 +1080,9 @@ hipError_t launch_massgn(const PushArgs<R> &a, hipStream_t s) {
     if (a.n <= 0) return hipSuccess;
     if (a.ppt == 1) launch_massgn_p<R, 1>(a, s);
     else if constexpr (sizeof(R) == 4) launch_massgn_p<R, 4>(a, s);
+    else if (a.ppt == 2 && !a.blk)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(massgn_kernel<R, false, 2>), dim3(nblocks(a.n, PB * 2)),
+                           dim3(PB), 0, s, a);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
