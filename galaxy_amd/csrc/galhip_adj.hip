@@ -854,7 +854,15 @@ static int adj_check(galhip_ctx *c) {
     if (c->nz != 1 || c->nsect != 1)
         return gh_fail(GALHIP_EINVAL, "the adjoint needs one zone and one sector");
     if (c->comp) return gh_fail(GALHIP_EINVAL, "the adjoint differentiates the plain position update");
+    // (before anything is changed; no context is made that large)
+    if (c->na > ADJ_MAX_NA || c->ng > 64) return gh_fail(GALHIP_EINVAL, "grid too large for the adjoint");
     return 0;
+}
+
+// The grid sums of a scatter start at zero: every solve leaves them so, and a
+// sweep clears them once more, should a step before it have failed in between.
+static hipError_t adj_clear_g(galhip_ctx *c) {
+    return launch_fill_i64((long long *)c->adj_g, 0, 2 * (long long)c->mesh, c->s);
 }
 
 // per-particle adjoints and grid work arrays, sized for the loaded particles
@@ -876,8 +884,7 @@ static int adj_ensure(galhip_ctx *c) {
     }
     if (rc) return rc;
     c->adj_n = c->n;
-    // (each solve leaves it zero)
-    HIPCHK(hipMemset(c->adj_g, 0, sizeof(double) * 2 * (size_t)c->mesh));
+    HIPCHK(adj_clear_g(c));
     HIPCHK(hipMemset(c->adj_lam, 0, sizeof(double) * 4 * (size_t)(c->n > 0 ? c->n : 1)));
     HIPCHK(hipMemset(adj_tail(c), 0, sizeof(double) * 4));
     return 0;
@@ -977,6 +984,7 @@ extern "C" int galhip_adj_set(galhip_ctx *c, const double *lam) {
         HIPCHK(hipMemcpyAsync(c->adj_id, c->id, sizeof(unsigned) * n, hipMemcpyDeviceToDevice, c->s));
     }
     HIPCHK(hipMemsetAsync(adj_tail(c), 0, sizeof(double) * 4, c->s));
+    HIPCHK(adj_clear_g(c));
     HIPCHK(hipStreamSynchronize(c->s));
     c->adj_ver = c->order_ver;
     return 0;
@@ -1002,6 +1010,7 @@ template <typename R> static int adj_seed_a2_impl(galhip_ctx *c, double lscale, 
         HIPCHK(hipMemcpyAsync(c->adj_id, c->id, sizeof(unsigned) * n, hipMemcpyDeviceToDevice, c->s));
     }
     HIPCHK(hipMemsetAsync(tail, 0, sizeof(double) * 4, c->s));
+    HIPCHK(adj_clear_g(c));
     double h[4];
     HIPCHK(hipMemcpyAsync(h, tail + 4, sizeof h, hipMemcpyDeviceToHost, c->s));
     HIPCHK(hipStreamSynchronize(c->s));
@@ -1102,7 +1111,6 @@ static AdjSolveArgs adj_solve_args(galhip_ctx *c) {
 
 // rbar = K^T (gx, gy), with the ranges of the last solve
 static int adj_solve(galhip_ctx *c) {
-    if (c->na > ADJ_MAX_NA || c->ng > 64) return gh_fail(GALHIP_EINVAL, "grid too large for the adjoint");
     AdjSolveArgs a = adj_solve_args(c);
     hipLaunchKernelGGL(adj_wbar_kernel, dim3(c->nr), dim3(ADJ_SOLVE_BLOCK), 0, c->s, a);
     HIPCHK(hipGetLastError());
