@@ -70,7 +70,6 @@ hipError_t launch_split_bf16(const double *, unsigned short *, int, int, int,
 hipError_t launch_ens_gemm(const EnsGemmArgs &, int, hipStream_t);
 hipError_t launch_d2f(const double *, float *, long long, hipStream_t);
 hipError_t launch_fill_i64(long long *, long long, long long, hipStream_t);
-hipError_t launch_fill_i32(int *, int, long long, hipStream_t);
 hipError_t launch_combine_ranges(const int *, const int *, int, int, int *, hipStream_t);
 hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, int, int,
                          hipStream_t);

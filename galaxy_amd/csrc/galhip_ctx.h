@@ -211,7 +211,6 @@ namespace gh {
 hipError_t launch_planar_lo(const float2 *, const unsigned *, float *, long long, hipStream_t);
 hipError_t launch_d2f(const double *, float *, long long, hipStream_t);
 hipError_t launch_fill_i64(long long *, long long, long long, hipStream_t);
-hipError_t launch_fill_i32(int *, int, long long, hipStream_t);
 hipError_t launch_masscl(const ZonePtrs &, int, long long, int *, int *, int, int, int,
                          hipStream_t);
 }  // namespace gh

@@ -65,14 +65,6 @@ __device__ __forceinline__ int wave_max_i32(int v) {
     return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
                max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
-__device__ __forceinline__ int wave_sum_i32(int v) {
-    v = v + GH_DPP(v, GH_DPP_QUAD_1032);
-    v = v + GH_DPP(v, GH_DPP_QUAD_2301);
-    v = v + GH_DPP(v, GH_DPP_ROW_HALF_MIRROR);
-    v = v + GH_DPP(v, GH_DPP_ROW_MIRROR);
-    return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) +
-           (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
-}
 
 // n / d for 0 <= n < 2^16 and 1 <= d < 2^16 without the integer division
 // sequence: n times the single-precision reciprocal of d is within 2^-6 of

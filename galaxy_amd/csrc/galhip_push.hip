@@ -105,14 +105,8 @@ __device__ __forceinline__ R comp_add(R x, R v, R lo, R &lo_out) {
     return s;
 }
 
-__device__ __forceinline__ long long wave_sum64(long long v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 __device__ __forceinline__ int wave_min(int v) { return wave_min_i32(v); }
 __device__ __forceinline__ int wave_max(int v) { return wave_max_i32(v); }
-
 
 // Hides a value's origin from the optimiser (no instruction is issued).
 __device__ __forceinline__ void opaque(float2 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }

@@ -920,14 +920,6 @@ hipError_t launch_fill_i64(long long *p, long long v, long long n, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_fill_i32(int *p, int v, long long n, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(fill_kernel<int>,
-                       dim3((unsigned)((n + GH_BLOCK - 1) / GH_BLOCK)),
-                       dim3(GH_BLOCK), 0, s, p, v, n);
-    return hipGetLastError();
-}
-
 hipError_t launch_combine_ranges(const int *jrad, const int *krad, int rstride, int nz, int *out,
                                  hipStream_t s) {
     hipLaunchKernelGGL(combine_ranges_kernel, dim3(1), dim3(64), 0, s, jrad, krad, rstride, nz, out);
