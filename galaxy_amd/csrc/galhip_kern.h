@@ -157,7 +157,9 @@ __device__ __forceinline__ void ut_of(double x, double y, double rr,
 __device__ __forceinline__ bool any_lane(bool c) { return __ballot(c) != 0; }
 
 // sqrt(x), correctly rounded: the hardware estimate is within one unit, and
-// the two neighbours' residuals decide (no scaling for x >= 2^-96).
+// the two neighbours' residuals decide (no scaling for x >= 2^-96): Markstein's
+// test, Computation of elementary functions on the IBM RISC System/6000
+// processor, IBM J. Res. Dev. 34 (1990).
 __device__ __forceinline__ double sqrt_rn(double x) { return sqrt(x); }
 __device__ __forceinline__ float sqrt_rn(float x) {
     float s = __builtin_amdgcn_sqrtf(x);
@@ -174,8 +176,8 @@ __device__ __forceinline__ float sqrt_rn(float x) {
     return s;
 }
 
-// a / b, correctly rounded: reciprocal with one Newton step, the quotient
-// corrected twice by its residual (|a| and b within 2^-60 .. 2^60, where no
+// a / b, correctly rounded (Markstein, as above): reciprocal with one Newton
+// step, the quotient corrected twice by its residual (|a| and b within 2^-60 .. 2^60, where no
 // step can underflow or overflow).
 __device__ __forceinline__ double div_rn(double a, double b) { return a / b; }
 __device__ __forceinline__ float div_rn(float a, float b) {
