@@ -13,7 +13,9 @@
 // index np/2 is left at 0, as in the reference).
 //
 // The sums take 8 FP64 operations per coefficient pair and particle and read
-// 9 bytes (FP32) per particle: FP64 issue bounds them.  A wavefront owns one
+// 9 bytes (FP32) per particle.  The latency of dependent FP64 products bounds
+// them: VALU issue is busy half of the time, with six wavefronts on a CU (1150
+// instructions per particle at 25 pitches x 6 harmonics).  A wavefront owns one
 // harmonic and a run of pitches for the whole pass, so its sums stay in
 // registers (four products per pitch and its mirror) and are reduced over
 // the lanes once at the end; the particles' e^{i nsect theta} and e^{i a}
@@ -47,7 +49,9 @@ struct LgPlan {
 };
 
 // Runs of at most 12 offsets: 48 FP64 sums (96 VGPRs) per lane, three
-// wavefronts per SIMD.  Without pitches a harmonic of its own per wavefront spends
+// wavefronts per SIMD; 8 of the 168 registers go to scratch (36 bytes) all the same.
+// Runs of 8 and 4 offsets do not spill, but form the tile again for more groups: 1e7
+// particles, 25 pitches x 6 harmonics 0.64 ms, 1.17 and 1.35.  Without pitches a harmonic of its own per wavefront spends
 // its time on forming z^im and, beyond eight harmonics, the tile again for every
 // group: runs of LG_HARM harmonics, each the product of the last one and z (4e6
 // particles, 512 harmonics: 27.0 ms one by one, 2.14 so; 64: 2.35 and 0.25;

@@ -1076,8 +1076,7 @@ __global__ __launch_bounds__(P3_BLOCK) void p3_analyse_kernel(P3SolveArgs<R> a) 
 #pragma unroll
         for (int h = 0; h < HB; h++) {
             const int s = slot(i0 + h), m = s < nm ? a.slot_m[s] : 0;
-            // (m < P3_MAX_NA: 32 bits hold the products, and their remainders are
-            // a third of a small grid's time with 64)
+            // (m < P3_MAX_NA: 32 bits hold the products)
             k[h] = (m * lane) % na;
             step[h] = (m * 64) % na;
         }
